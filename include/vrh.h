@@ -114,8 +114,8 @@ int vrh_set_radial_mesh(vrh_t *h, const double *rm, const double *rc, const doub
  * z cosine transform by the generalised eigenvectors of its z operator
  * (dense nz x nz transforms, GEMMs on the device), which on the uniform
  * mesh are the same cosines.  No reference counterpart.  Particles need the
- * uniform axial mesh; a handle with an axial mesh steps without a HIP graph
- * and cannot join an ensemble. */
+ * uniform axial mesh; a mixed-precision handle with an axial mesh steps
+ * without a HIP graph, and no handle with one can join an ensemble. */
 int vrh_set_axial_mesh(vrh_t *h, const double *zm, const double *zc, const double *dmz, const double *dcz);
 
 /* One RK substep irk=1..3 (loop.F90:71-127) of the step that has reached
@@ -146,8 +146,8 @@ int vrh_snapshot_begin(vrh_t *h);
 int vrh_snapshot_wait(vrh_t *h, double *q1, double *q2, double *q3, double *pres, double *ntime);
 /* vrh_step replays one RK3 step captured as a HIP graph (captured on first
  * use, recaptured after vrh_autotune, vrh_set_tuning, vrh_set_radial_mesh or a
- * particle change; not used while the kernel timer is on or with an axial
- * mesh).  on = 0 launches the kernels one by one instead.  No
+ * particle change; not used while the kernel timer is on, with a per-mode
+ * solver, or in mixed precision with an axial mesh).  on = 0 launches the kernels one by one instead.  No
  * reference counterpart. */
 int vrh_set_graph(vrh_t *h, int on);
 /* One phase of substep irk (parity tests and profiling). */

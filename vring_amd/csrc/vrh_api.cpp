@@ -404,6 +404,9 @@ int vrh_create(const vrh_grid *grid, const vrh_params *p, int precision, vrh_t *
   for (size_t q = 0; q < mint.size() && q < 243; q++) h->h_mint[q] = mint[q];
   if ((rc = dalloc(h, &h->d_sc, 16))) return rc;
   HIPCHK(h, hipHostMalloc((void **)&h->h_pin, 16 * sizeof(double), hipHostMallocDefault));
+  if (dense_lds_need(h->nt, h->nz) > (size_t)h->lds_block)
+    return fail(h, "vrh_create: the transforms' line tiles need more LDS than the device grants", -3);
+  if ((rc = dense_create(h))) return rc;
   if ((rc = refresh_mesh(h))) return rc;
   HIPCHK(h, hipStreamSynchronize(h->stream));
   return 0;
@@ -417,7 +420,7 @@ int vrh_destroy(vrh_t *h) {
                   f.q3, f.dq1, f.dq2, f.dq3, f.pres, f.dph, f.ru1, f.ru2, f.ru3, f.r1, f.r2, f.r3, f.prg1, f.prg2,
                   f.prg3, f.S, f.ib, f.S64, f.ib64, f.csort, f.dq3no, f.corr3n, f.flag};
   for (void *p : ptrs) if (p) hipFree(p);
-  void *zp[] = {h->d_zmet, h->d_zv, h->d_zvf, h->S2, h->S2_64};
+  void *zp[] = {h->d_zmet, h->d_zv, h->d_zvf, h->d_zeig, h->S2, h->S2_64, h->d_zcos, h->d_tdft};
   for (void *p : zp) if (p) hipFree(p);
   if (h->blas) rocblas_destroy_handle((rocblas_handle)h->blas);
   for (auto &e : h->kt_pool) hipEventDestroy(e);
@@ -576,22 +579,25 @@ int vrh_set_axial_mesh(vrh_t *h, const double *zm, const double *zc, const doubl
   std::vector<double> vi, vf, lam;
   std::string emsg;
   if (host_axial_transforms(m3, c3, nz, vi, vf, lam, emsg)) return fail(h, ("axial mesh: " + emsg).c_str());
+  if (h->prec == VRH_FP64 && (size_t)nz * 16 * sizeof(double) > (size_t)h->lds_block)
+    return fail(h, "axial mesh: the z transform's line tile needs more LDS than the device grants", -3);
   const size_t nn = (size_t)nz * nz;
   int rc;
   if (!h->d_zmet && (rc = dalloc(h, &h->d_zmet, mb.size()))) return rc;
-  if (!h->d_zv && (rc = dalloc(h, &h->d_zv, 2 * nn))) return rc;
   if (h->prec == VRH_MIXED) {
+    if (!h->d_zv && (rc = dalloc(h, &h->d_zv, 2 * nn))) return rc;
     if (!h->d_zvf && (rc = dalloc(h, &h->d_zvf, 2 * nn))) return rc;
     if (!h->S2_64 && (rc = dalloc(h, &h->S2_64, (size_t)5 * h->nr * nz))) return rc;
+    if (!h->S2 && (rc = dalloc_bytes(h, &h->S2, compact(h) * wsize(h)))) return rc;
   }
-  if (!h->S2 && (rc = dalloc_bytes(h, &h->S2, compact(h) * wsize(h)))) return rc;
-  if (!h->blas) {
+  if (h->prec == VRH_MIXED && !h->blas) {
     rocblas_handle b = nullptr;
     if (rocblas_create_handle(&b) != rocblas_status_success) return fail(h, "axial mesh: rocblas_create_handle failed", -3);
     h->blas = b;
     if (rocblas_set_stream(b, h->stream) != rocblas_status_success)
       return fail(h, "axial mesh: rocblas_set_stream failed", -3);
   }
+  if (h->prec == VRH_FP64 && (rc = dense_axial(h, vi, vf))) return rc;
   h->hz = nullptr;  // a per-mode solve set for another mesh: switched off
   for (int q = 0; q < 4; q++) h->zmesh[q] = zmn[q];
   h->zlam = lam;
@@ -600,13 +606,11 @@ int vrh_set_axial_mesh(vrh_t *h, const double *zm, const double *zc, const doubl
   h->zmet.fm = h->d_zmet + 4 * L; h->zmet.fp = h->d_zmet + 5 * L; h->zmet.zpos = h->d_zmet + 6 * L;
   h->zmet.ws = 2.0 / (h1 * (h1 + h2));
   h->zmet.w2 = 2.0 / (h2 * (h1 + h2));
-  std::vector<double> zv(2 * nn);
-  std::memcpy(zv.data(), vi.data(), nn * sizeof(double));
-  std::memcpy(zv.data() + nn, vf.data(), nn * sizeof(double));
-  if ((rc = h2d(h, h->d_zv, zv.data(), zv.size() * sizeof(double)))) return rc;
   if (h->prec == VRH_MIXED) {
     std::vector<float> zf(2 * nn);
-    for (size_t i = 0; i < 2 * nn; i++) zf[i] = (float)zv[i];
+    for (size_t i = 0; i < nn; i++) { zf[i] = (float)vi[i]; zf[nn + i] = (float)vf[i]; }
+    if ((rc = h2d(h, h->d_zv, vi.data(), nn * sizeof(double)))) return rc;
+    if ((rc = h2d(h, h->d_zv + nn, vf.data(), nn * sizeof(double)))) return rc;
     if ((rc = h2d(h, h->d_zvf, zf.data(), zf.size() * sizeof(float)))) return rc;
   }
   if ((rc = refresh_mesh(h))) return rc;
@@ -694,8 +698,9 @@ int step_enqueue(vrh_t *h, int nsteps) {
     HIPCHK(h, hipMemcpyAsync(h->d_sc, h->h_pin, sizeof(double), hipMemcpyHostToDevice, h->stream));
     h->time_dirty = false;
   }
-  // an axial mesh's z transforms are library GEMMs: launched eagerly
-  const bool graph = h->use_graph && !h->kt_on && h->zmesh[0].empty();
+  // eager: the FP32 z transforms of an axial mesh are library GEMMs, and a
+  // per-mode solve waits for its iterations
+  const bool graph = h->use_graph && !h->kt_on && !h->hz && (h->zmesh[0].empty() || h->prec == VRH_FP64);
   if (graph && !h->graph_ok) { int rc = build_graph(h); if (rc) return rc; }
   for (int s = 0; s < nsteps; s++) {
     h->ntime = h->dt + h->ntime;  // loop.F90:53 (k_scalars does the same on the device)

@@ -66,6 +66,20 @@ struct LineCoef {
   int n, P;
 };
 
+// divq's right-hand side at a cell (divergence.F90:31-41) from the three
+// one-sided differences: wr = 1/rm, ct, cr, cz the difference factors.  The
+// fused operations are written out, so that every kernel rounds alike.
+__device__ __forceinline__ double divq_rhs(double d1, double ct, double d2, double cr, double wr, double d3, double cz,
+                                           double inv_adt) {
+#pragma clang fp contract(off)
+  const double t12 = __builtin_fma(d1, ct, d2 * cr);
+  return -__builtin_fma(d3, cz, t12 * wr) * inv_adt;
+}
+
+// A matrix packed for the FP64 matrix cores (vrh_dense.hip): mt tiles of 16
+// rows, ks steps of 4 columns.
+struct DenseMat { const double *a; int mt, ks; };
+
 enum SweepMode { SW_R1 = 0, SW_R3 = 1, SW_R2 = 2, SW_Z1 = 3, SW_Z3 = 4, SW_Z2 = 5 };
 
 // Work type TW (double in FP64 mode, float in mixed mode); state type TS is
@@ -161,10 +175,10 @@ struct vrh_s {
   std::vector<double> mesh[4];
   // axial mesh set by vrh_set_axial_mesh (zm, zc, dmz, dcz over k = 0..nz+2);
   // empty: the uniform mesh.  zlam: eigenvalues of the pressure solve's z
-  // operator (ascending, zlam[0] = 0); d_zmet: the ZMet arrays; d_zv: the z
-  // transforms V^-1 then V (nz x nz each, double), d_zvf: their float copies
-  // (mixed precision); S2: the spectral work array's twin (out-of-place
-  // transforms), S2_64: the same for the FP64 low modes
+  // operator (ascending, zlam[0] = 0); d_zmet: the ZMet arrays.  The z
+  // transforms V^-1 then V: FP64 path packed (d_zeig, zeig); mixed path row
+  // major nz x nz, double (d_zv) and float (d_zvf), for library GEMMs out of
+  // place into the twins S2 and S2_64 of the spectral arrays
   std::vector<double> zmesh[4];
   std::vector<double> zlam;
   ZMet zmet{};
@@ -172,7 +186,14 @@ struct vrh_s {
   float *d_zvf = nullptr;
   void *S2 = nullptr;
   double *S2_64 = nullptr;
-  void *blas = nullptr;  // rocBLAS handle of the z transforms (on `stream`)
+  void *blas = nullptr;  // rocBLAS handle of the mixed path's z transforms (on `stream`)
+  double *d_zeig = nullptr;
+  DenseMat zeig[2] = {};  // [0] forward, [1] inverse
+  // lengths that are no power of two: the z cosine matrices, the forward
+  // theta matrix and the inverse theta transform's table
+  double *d_zcos = nullptr, *d_tdft = nullptr;
+  DenseMat zdct[2] = {}, tdft = {};
+  const double *idft_tab = nullptr;
   // per-mode iterative pressure solve (vrh_set_mode_solver): theta
   // positions pos >= hz_pos0 (modes m >= mmin) are solved by the Helmholtz
   // handle hz instead of the direct z transform + radial solve; hz_f is the
@@ -289,6 +310,14 @@ void lds_optin(vrh_t *h);
 template <typename TW> void launch_sweeps(vrh_t *h, int irk, double c3s, const double *c3s_dev, bool hdnbc = false,
                                           double cor = 0.0, const double *cor_dev = nullptr);
 template <typename TW> void launch_poisson(vrh_t *h, int irk, const double *ext_rhs, double *phi_out);
+// dense transforms (vrh_dense.hip)
+int dense_create(vrh_t *h);
+int dense_axial(vrh_t *h, const std::vector<double> &vi, const std::vector<double> &vf);
+size_t dense_lds_need(int nt, int nz);
+bool dense_lds_optin(int bytes);
+template <typename TW> void launch_zdense(vrh_t *h, hipStream_t st, TW *S, long nl, int dir);
+template <typename TW> void launch_divdft(vrh_t *h, double inv_adt, const double *ext, TW *S, double *S64);
+template <typename TW> void launch_idft(vrh_t *h, const TW *S, const double *S64, double *phi_out, double *dph);
 template <typename TW> void launch_project(vrh_t *h, int irk);
 // the particle stage of substep irk on stream st (nothing launched where
 // the scheme has no stage at irk); returns whether anything was launched

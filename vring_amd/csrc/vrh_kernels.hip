@@ -1198,8 +1198,8 @@ __device__ __forceinline__ void lds_fft(T *re, T *im, int nfft, int logn, int ss
 __host__ __device__ constexpr size_t al16(size_t b) { return (b + 15) & ~(size_t)15; }
 
 // divq (divergence.F90:31-41) + fft_ptf_multi packing
-// (fastfouriertransform.F90:39-43) for LB theta lines per block.  Power-of-two
-// ntheta: two real lines per complex FFT in LDS.  Other ntheta: direct DFT.
+// (fastfouriertransform.F90:39-43) for LB theta lines per block, ntheta a
+// power of two: two real lines per complex FFT in LDS (other ntheta: k_divdft).
 // In mixed mode the packed positions 0..4 (m = 0,1,2) are also produced in
 // double from the double divergence into S64 (layout (5, nr, nz)).
 template <typename TW>
@@ -1212,17 +1212,12 @@ __global__ __launch_bounds__(256) void k_divfft(VGrid g, VCoef c, ZMet zm, doubl
   const int N = g.nt, tid = threadIdx.x, nth = blockDim.x;
   const long nlines = (long)g.nr * g.nz;
   const long l0 = (long)blockIdx.x * LB;
-  // LDS: [dv (LB*N double)] | re, im ((LB/2)*N TW each) | [tw (2N double), part (10 LB double)] |
-  // twl (N TW) | jk (2 LB int) | 1/rm, dx2/dmr (LB double each).  The double
-  // copy dv feeds only the direct DFT (ntheta not a power of two); the FP64
+  // LDS: re, im ((LB/2)*N TW each) | [tw (2N double), part (10 LB double)] |
+  // twl (N TW) | jk (2 LB int) | 1/rm, dx2/dmr (LB double each).  The FP64
   // low modes of the mixed path are summed in registers.
-  const bool pow2 = N >= 2 && (N & (N - 1)) == 0;
-  const bool keep_dv = !pow2;
-  size_t off = keep_dv ? al16(sizeof(double) * LB * N) : 0;
-  double *dv = reinterpret_cast<double *>(smem_raw);
-  TW *re = reinterpret_cast<TW *>(smem_raw + off);
+  TW *re = reinterpret_cast<TW *>(smem_raw);
   TW *im = re + (size_t)(LB / 2) * N;
-  off = al16(off + sizeof(TW) * LB * N);
+  size_t off = al16(sizeof(TW) * LB * N);
   double *tw = reinterpret_cast<double *>(smem_raw + off);     // cos (N) then sin (N), S64 only
   double *part = tw + 2 * (size_t)N;                           // (line, coefficient, 2 waves), S64 only
   if (S64) off = al16(off + sizeof(double) * (2 * (size_t)N + 10 * (size_t)LB));
@@ -1241,8 +1236,7 @@ __global__ __launch_bounds__(256) void k_divfft(VGrid g, VCoef c, ZMet zm, doubl
     lirm[tid] = 1.0 / c.rm[j];
     lcx2[tid] = g.dx2 / c.dmr[j];
   }
-  if (pow2)
-    for (int q = tid; q < N / 2; q += nth) { twl[q] = (TW)twr[q]; twl[N / 2 + q] = (TW)twi[q]; }
+  for (int q = tid; q < N / 2; q += nth) { twl[q] = (TW)twr[q]; twl[N / 2 + q] = (TW)twi[q]; }
   if (S64)
     for (int q = tid; q < N; q += nth) { tw[q] = twr[q]; tw[N + q] = twi[q]; }
   __syncthreads();
@@ -1254,11 +1248,8 @@ __global__ __launch_bounds__(256) void k_divfft(VGrid g, VCoef c, ZMet zm, doubl
   const bool lvalid = l0 + lpt < nlines;
   double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0;
   auto put = [&](int ii, double val) {
-    if (keep_dv) dv[lpt * N + ii] = val;
-    if (pow2) {
-      const int pos = (lpt >> 1) * N + ii;
-      if (lpt & 1) im[pos] = (TW)val; else re[pos] = (TW)val;
-    }
+    const int pos = (lpt >> 1) * N + ii;
+    if (lpt & 1) im[pos] = (TW)val; else re[pos] = (TW)val;
     if (S64) {  // cos and sin sums of wavenumbers 0, 1, 2
       int q2 = 2 * ii;
       if (q2 >= N) q2 -= N;
@@ -1300,9 +1291,8 @@ __global__ __launch_bounds__(256) void k_divfft(VGrid g, VCoef c, ZMet zm, doubl
       for (int u = 0; u < U; ++u) {
         const int ii = tl + TPL * (ub + u);
         if (ii < N) {
-          const double t12 = ((b1[u] - a1[u]) * (g.dx1 * g.axsym) + (b2[u] - a2[u]) * rdv) * rmv;
-          const double t3 = (b3[u] - a3[u]) * zkv;
-          put(ii, lvalid ? -(t12 + t3) * inv_adt : 0.0);
+          const double rhs = divq_rhs(b1[u] - a1[u], g.dx1 * g.axsym, b2[u] - a2[u], rdv, rmv, b3[u] - a3[u], zkv, inv_adt);
+          put(ii, lvalid ? rhs : 0.0);
         }
       }
     }
@@ -1324,35 +1314,22 @@ __global__ __launch_bounds__(256) void k_divfft(VGrid g, VCoef c, ZMet zm, doubl
     }
   }
   __syncthreads();
-  if (pow2) lds_fft(re, im, LB / 2, logn, N, twl, twl + N / 2, (TW)-1, tid, nth);
+  lds_fft(re, im, LB / 2, logn, N, twl, twl + N / 2, (TW)-1, tid, nth);
   // a power-of-two N scales exactly, so x * (1/N) is x / N bit for bit
   // without a double division per element
   const double inv_n = 1.0 / N;
   for (int e = tid; e < LB * N; e += nth) {
-    const int lp = pow2 ? e >> logn : e / N, pos = e - lp * N;
+    const int lp = e >> logn, pos = e - lp * N;
     const long l = l0 + lp;
     if (l >= nlines) continue;
     const int k = (pos + 1) >> 1;  // wavenumber of this packed position
     double Fr, Fi;
-    if (pow2) {
-      const int q = lp >> 1, kr = (N - k) & (N - 1);
-      const double zr = re[q * N + k], zi = im[q * N + k], wr = re[q * N + kr], wi = im[q * N + kr];
-      if ((lp & 1) == 0) { Fr = 0.5 * (zr + wr); Fi = 0.5 * (zi - wi); }
-      else { Fr = 0.5 * (zi + wi); Fi = -0.5 * (zr - wr); }
-    } else {
-      Fr = 0.0; Fi = 0.0;
-      int ph = 0;
-      for (int jj = 0; jj < N; ++jj) {
-        const double x = dv[lp * N + jj];
-        Fr += x * twr[ph];
-        Fi -= x * twi[ph];
-        ph += k;
-        if (ph >= N) ph -= N;
-      }
-    }
+    const int q = lp >> 1, kr = (N - k) & (N - 1);
+    const double zr = re[q * N + k], zi = im[q * N + k], wr = re[q * N + kr], wi = im[q * N + kr];
+    if ((lp & 1) == 0) { Fr = 0.5 * (zr + wr); Fi = 0.5 * (zi - wi); }
+    else { Fr = 0.5 * (zi + wi); Fi = -0.5 * (zr - wr); }
     const double num = (pos == 0) ? Fr : (pos & 1) ? 2.0 * Fr : -2.0 * Fi;
-    const double outv = pow2 ? num * inv_n : num / N;
-    S[(size_t)pos + (size_t)N * l] = (TW)outv;
+    S[(size_t)pos + (size_t)N * l] = (TW)(num * inv_n);
   }
   if (S64) {
     // FP64 modes m = 0, 1, 2 (t(1), t(2k), t(2k+1) packing) from the wave
@@ -1370,7 +1347,7 @@ __global__ __launch_bounds__(256) void k_divfft(VGrid g, VCoef c, ZMet zm, doubl
 }
 
 // z DCT-II (REDFT10, then /(2nz): fastfouriertransform.F90:299-332) of TL
-// lines per block; lines are contiguous in memory (line stride 1, position
+// lines per block, nz a power of two (other nz: k_zdense); lines are contiguous in memory (line stride 1, position
 // stride nl).  Makhoul's reordering turns each pair of real lines into one
 // complex FFT of length nz.  dir=+1 forward, -1 inverse (REDFT01).
 template <typename TW>
@@ -1394,111 +1371,86 @@ __global__ __launch_bounds__(1024) void k_dctz(TW *__restrict__ S, long nl, int 
   auto esin = [&](int k) { return lds_tw ? etw[n + k] : (TW)ei[k]; };
   const int tid = threadIdx.x, nth = blockDim.x;
   const long l0 = xcd_tile(blockIdx.x, gridDim.x) * TL;
-  const bool pow2 = n >= 2 && (n & (n - 1)) == 0;
-  if (pow2) {
-    for (int q = tid; q < n / 2; q += nth) { twl[q] = (TW)twr[q]; twl[n / 2 + q] = (TW)twi[q]; }
-    if (lds_tw)
-      for (int q = tid; q < n; q += nth) { etw[q] = (TW)er[q]; etw[n + q] = (TW)ei[q]; }
-    // Element u of a thread is line lp = tid mod TL (consecutive lanes,
-    // consecutive lines) at position kz0 + u dk, dk = nth / TL (a multiple
-    // of 8, so every position of a thread has the parity of kz0).  The
-    // launch keeps TL n <= 16 nth; lanes with kz0 >= n (TL n < nth) only
-    // help with the LDS phases.  Lines past nl load the last line and are
-    // zeroed (forward) or not stored.
-    constexpr int PF = 16;
-    const int tot = TL * n, lp = tid & (TL - 1), kz0 = tid >> logtl, dk = nth >> logtl;
-    const int nu = min(PF, (tot + nth - 1) / nth);
-    const bool lin = l0 + lp < nl;
-    TW v[PF];
-    {
-      const int kc = min(kz0, n - 1);
-      const TW *src = S + min(l0 + lp, nl - 1) + nl * kc;
-      const long step = nl * dk, last = (long)((n - 1 - kc) / dk) * step;
-#pragma unroll
-      for (int u = 0; u < PF; ++u)
-        if (u < nu) v[u] = src[min(u * step, last)];
-    }
-    __syncthreads();  // twiddle tables
-    // Makhoul order of position kz: kz/2 for even kz, n-1-kz/2 for odd kz,
-    // for the thread's positions pm0 + u dpm.  Forward: the lines go into
-    // the pair's complex sequence in Makhoul order (and come out in natural
-    // order); inverse: in natural order (and out in Makhoul order).
-    TW *const dpair = ((lp & 1) ? im : re) + (lp >> 1) * sn;
-    const int pm0 = (kz0 & 1) ? n - 1 - (kz0 >> 1) : (kz0 >> 1);
-    const int dpm = (kz0 & 1) ? -(dk >> 1) : (dk >> 1);
-    const int pi0 = dir > 0 ? pm0 : kz0, dpi = dir > 0 ? dpm : dk;
+  for (int q = tid; q < n / 2; q += nth) { twl[q] = (TW)twr[q]; twl[n / 2 + q] = (TW)twi[q]; }
+  if (lds_tw)
+    for (int q = tid; q < n; q += nth) { etw[q] = (TW)er[q]; etw[n + q] = (TW)ei[q]; }
+  // Element u of a thread is line lp = tid mod TL (consecutive lanes,
+  // consecutive lines) at position kz0 + u dk, dk = nth / TL (a multiple
+  // of 8, so every position of a thread has the parity of kz0).  The
+  // launch keeps TL n <= 16 nth; lanes with kz0 >= n (TL n < nth) only
+  // help with the LDS phases.  Lines past nl load the last line and are
+  // zeroed (forward) or not stored.
+  constexpr int PF = 16;
+  const int tot = TL * n, lp = tid & (TL - 1), kz0 = tid >> logtl, dk = nth >> logtl;
+  const int nu = min(PF, (tot + nth - 1) / nth);
+  const bool lin = l0 + lp < nl;
+  TW v[PF];
+  {
+    const int kc = min(kz0, n - 1);
+    const TW *src = S + min(l0 + lp, nl - 1) + nl * kc;
+    const long step = nl * dk, last = (long)((n - 1 - kc) / dk) * step;
 #pragma unroll
     for (int u = 0; u < PF; ++u)
-      if (u < nu && kz0 + u * dk < n) dpair[pi0 + u * dpi] = lin ? v[u] : (TW)0;
-    __syncthreads();
-    if (dir < 0) {
-      // in place, one (k, n-k) pair per task (k = 0..n/2, Y[n] = 0):
-      // W[k] = e^{i pi k/2n} ((Ya[k] + Yb[n-k]) + i (Yb[k] - Ya[n-k]))
-      const int ltq = logtl - 1, TQ = TL >> 1, nh = n >> 1, tq = TQ * (nh + 1);
-      for (int e = tid; e < tq; e += nth) {
-        const int q = e & (TQ - 1), k = e >> ltq, kn = (n - k) & (n - 1);
-        TW *rq = re + q * sn, *iq = im + q * sn;
-        const TW a0 = rq[k], b0 = iq[k];
-        const TW an = k > 0 ? rq[kn] : (TW)0, bn = k > 0 ? iq[kn] : (TW)0;
-        {
-          const TW uu = a0 + bn, w = b0 - an, c = ecos(k), sv = esin(k);
-          rq[k] = uu * c - w * sv;
-          iq[k] = uu * sv + w * c;
-        }
-        if (k > 0 && k < nh) {
-          const TW uu = an + b0, w = bn - a0, c = ecos(kn), sv = esin(kn);
-          rq[kn] = uu * c - w * sv;
-          iq[kn] = uu * sv + w * c;
-        }
-      }
-      __syncthreads();
-    }
-    lds_fft(re, im, TL / 2, logn, sn, twl, twl + n / 2, (TW)(dir > 0 ? -1 : 1), tid, nth);
-    const TW inv_n = (TW)1 / (TW)n;  // exact: n is a power of two
-    if (kz0 < n && lin) {
-      TW *dst = S + (l0 + lp) + nl * kz0;
-      const long step = nl * dk;
-      const TW *zq = re + (lp >> 1) * sn, *zi = im + (lp >> 1) * sn;
+      if (u < nu) v[u] = src[min(u * step, last)];
+  }
+  __syncthreads();  // twiddle tables
+  // Makhoul order of position kz: kz/2 for even kz, n-1-kz/2 for odd kz,
+  // for the thread's positions pm0 + u dpm.  Forward: the lines go into
+  // the pair's complex sequence in Makhoul order (and come out in natural
+  // order); inverse: in natural order (and out in Makhoul order).
+  TW *const dpair = ((lp & 1) ? im : re) + (lp >> 1) * sn;
+  const int pm0 = (kz0 & 1) ? n - 1 - (kz0 >> 1) : (kz0 >> 1);
+  const int dpm = (kz0 & 1) ? -(dk >> 1) : (dk >> 1);
+  const int pi0 = dir > 0 ? pm0 : kz0, dpi = dir > 0 ? dpm : dk;
 #pragma unroll
-      for (int u = 0; u < PF; ++u) {
-        const int kz = kz0 + u * dk;
-        if (u < nu && kz < n) {
-          TW outv;
-          if (dir > 0) {
-            const int kr = (n - kz) & (n - 1);
-            const TW zr = zq[kz], zim = zi[kz], wr = zq[kr], wi = zi[kr];
-            TW vr, vi;
-            if ((lp & 1) == 0) { vr = (TW)0.5 * (zr + wr); vi = (TW)0.5 * (zim - wi); }
-            else { vr = (TW)0.5 * (zim + wi); vi = (TW)(-0.5) * (zr - wr); }
-            outv = (vr * ecos(kz) + vi * esin(kz)) * inv_n;  // Re(e^{-i pi k/2n} V)/n
-          } else {
-            outv = dpair[pm0 + u * dpm];
-          }
-          dst[u * step] = outv;
-        }
+  for (int u = 0; u < PF; ++u)
+    if (u < nu && kz0 + u * dk < n) dpair[pi0 + u * dpi] = lin ? v[u] : (TW)0;
+  __syncthreads();
+  if (dir < 0) {
+    // in place, one (k, n-k) pair per task (k = 0..n/2, Y[n] = 0):
+    // W[k] = e^{i pi k/2n} ((Ya[k] + Yb[n-k]) + i (Yb[k] - Ya[n-k]))
+    const int ltq = logtl - 1, TQ = TL >> 1, nh = n >> 1, tq = TQ * (nh + 1);
+    for (int e = tid; e < tq; e += nth) {
+      const int q = e & (TQ - 1), k = e >> ltq, kn = (n - k) & (n - 1);
+      TW *rq = re + q * sn, *iq = im + q * sn;
+      const TW a0 = rq[k], b0 = iq[k];
+      const TW an = k > 0 ? rq[kn] : (TW)0, bn = k > 0 ? iq[kn] : (TW)0;
+      {
+        const TW uu = a0 + bn, w = b0 - an, c = ecos(k), sv = esin(k);
+        rq[k] = uu * c - w * sv;
+        iq[k] = uu * sv + w * c;
       }
-    }
-  } else {
-    // direct transform for non-power-of-two nz (small test grids)
-    TW *buf = re;  // TL * n
-    for (int e = tid; e < TL * n; e += nth) {
-      const int lp = e % TL, kz = e / TL;
-      const long l = l0 + lp;
-      buf[lp * n + kz] = (l < nl) ? S[l + nl * kz] : (TW)0;
+      if (k > 0 && k < nh) {
+        const TW uu = an + b0, w = bn - a0, c = ecos(kn), sv = esin(kn);
+        rq[kn] = uu * c - w * sv;
+        iq[kn] = uu * sv + w * c;
+      }
     }
     __syncthreads();
-    for (int e = tid; e < TL * n; e += nth) {
-      const int lp = e % TL, kz = e / TL;
-      const long l = l0 + lp;
-      double sacc = 0.0;
-      if (dir > 0) {
-        for (int jj = 0; jj < n; ++jj) sacc += (double)buf[lp * n + jj] * cos(M_PI * (jj + 0.5) * kz / n);
-        sacc = 2.0 * sacc / (2.0 * n);
-      } else {
-        sacc = buf[lp * n];
-        for (int kk = 1; kk < n; ++kk) sacc += 2.0 * (double)buf[lp * n + kk] * cos(M_PI * kk * (kz + 0.5) / n);
+  }
+  lds_fft(re, im, TL / 2, logn, sn, twl, twl + n / 2, (TW)(dir > 0 ? -1 : 1), tid, nth);
+  const TW inv_n = (TW)1 / (TW)n;  // exact: n is a power of two
+  if (kz0 < n && lin) {
+    TW *dst = S + (l0 + lp) + nl * kz0;
+    const long step = nl * dk;
+    const TW *zq = re + (lp >> 1) * sn, *zi = im + (lp >> 1) * sn;
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+      const int kz = kz0 + u * dk;
+      if (u < nu && kz < n) {
+        TW outv;
+        if (dir > 0) {
+          const int kr = (n - kz) & (n - 1);
+          const TW zr = zq[kz], zim = zi[kz], wr = zq[kr], wi = zi[kr];
+          TW vr, vi;
+          if ((lp & 1) == 0) { vr = (TW)0.5 * (zr + wr); vi = (TW)0.5 * (zim - wi); }
+          else { vr = (TW)0.5 * (zim + wi); vi = (TW)(-0.5) * (zr - wr); }
+          outv = (vr * ecos(kz) + vi * esin(kz)) * inv_n;  // Re(e^{-i pi k/2n} V)/n
+        } else {
+          outv = dpair[pm0 + u * dpm];
+        }
+        dst[u * step] = outv;
       }
-      if (l < nl) S[l + nl * kz] = (TW)sacc;
     }
   }
 }
@@ -1606,14 +1558,12 @@ __global__ __launch_bounds__(256) void k_ifft(VGrid g, const TW *__restrict__ S,
   // table (N each) staged in LDS for the merge
   double *s64l = reinterpret_cast<double *>(smem_raw + al16(ojk + sizeof(int) * 2 * LB));
   double *tw64 = s64l + 5 * (size_t)LB;
-  const bool pow2 = N >= 2 && (N & (N - 1)) == 0;
   if (tid < LB) {
     const long l = l0 + tid;
     jk[2 * tid] = (int)(l % g.nr) + 1;
     jk[2 * tid + 1] = (int)(l / g.nr) + 1;
   }
-  if (pow2)
-    for (int q = tid; q < N / 2; q += nth) { twl[q] = (TW)twr[q]; twl[N / 2 + q] = (TW)twi[q]; }
+  for (int q = tid; q < N / 2; q += nth) { twl[q] = (TW)twr[q]; twl[N / 2 + q] = (TW)twi[q]; }
   if (S64) {
     for (int q = tid; q < N; q += nth) { tw64[q] = twr[q]; tw64[N + q] = twi[q]; }
     for (int e = tid; e < 5 * LB; e += nth) s64l[e] = S64[5 * min(l0 + e / 5, nlines - 1) + e % 5];
@@ -1628,7 +1578,7 @@ __global__ __launch_bounds__(256) void k_ifft(VGrid g, const TW *__restrict__ S,
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int e = min(eb + u * nth, tot - 1);
-        const int lp = pow2 ? e >> logn : e / N, pos = e - lp * N;
+        const int lp = e >> logn, pos = e - lp * N;
         v[u] = S[(size_t)pos + (size_t)N * min(l0 + lp, nlines - 1)];
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -1636,14 +1586,14 @@ __global__ __launch_bounds__(256) void k_ifft(VGrid g, const TW *__restrict__ S,
       for (int u = 0; u < U; ++u) {
         const int e = eb + u * nth;
         if (e < tot) {
-          const int lp = pow2 ? e >> logn : e / N, pos = e - lp * N;
+          const int lp = e >> logn, pos = e - lp * N;
           tb[e] = (l0 + lp < nlines && !(S64 && pos < 5)) ? v[u] : (TW)0;
         }
       }
     }
   }
   __syncthreads();
-  if (pow2) {
+  {
     // Z[k] = Fa[k] + i Fb[k], Fa[k] = (t(2k-1) - i t(2k))/2, Hermitian extension
     for (int e = tid; e < (LB / 2) * N; e += nth) {
       const int q = e >> logn, k = e - q * N;
@@ -1666,8 +1616,8 @@ __global__ __launch_bounds__(256) void k_ifft(VGrid g, const TW *__restrict__ S,
     __syncthreads();
     lds_fft(re, im, LB / 2, logn, N, twl, twl + N / 2, (TW)1, tid, nth);
   }
-  if (pow2 && (nth & (N - 1)) == 0) {
-    // N divides the block: every element of a thread has the same theta
+  {
+    // N divides the block (N <= 256 = nth): every element of a thread has the same theta
     // index ii, so the low-mode twiddles of the merge are loaded once
     const int ii = tid & (N - 1), lstep = nth >> logn;
     double cw1 = 0.0, sw1 = 0.0, cw2 = 0.0, sw2 = 0.0;
@@ -1683,7 +1633,6 @@ __global__ __launch_bounds__(256) void k_ifft(VGrid g, const TW *__restrict__ S,
       const int q = lp >> 1;
       double v = (lp & 1) ? (double)im[q * N + ii] : (double)re[q * N + ii];
       if (S64) {
-        // the terms of the generic loop below, in its order
         const double *t = s64l + 5 * lp;
         v += t[0];
         {
@@ -1703,43 +1652,6 @@ __global__ __launch_bounds__(256) void k_ifft(VGrid g, const TW *__restrict__ S,
         dph[hidx(g, ii + 1, j, k)] = v;
         if (k == g.nz) dph[hidx(g, ii + 1, j, g.nzc)] = v;
       }
-    }
-    return;
-  }
-  for (int e = tid; e < LB * N; e += nth) {
-    const int lp = pow2 ? e >> logn : e / N, ii = e - lp * N;
-    const long l = l0 + lp;
-    if (l >= nlines) continue;
-    double v;
-    if (pow2) {
-      const int q = lp >> 1;
-      v = (lp & 1) ? (double)im[q * N + ii] : (double)re[q * N + ii];
-    } else {
-      const TW *t = tb + lp * N;
-      v = t[0];
-      for (int kk = 1; 2 * kk - 1 < N; ++kk) {
-        const int ph = (int)(((long)ii * kk) % N);
-        const double a = t[2 * kk - 1], b = (2 * kk < N) ? t[2 * kk] : 0.0;
-        if (2 * kk == N) v += 0.5 * a * twr[ph];
-        else v += a * twr[ph] + b * twi[ph];
-      }
-    }
-    if (S64) {
-      const double *t = s64l + 5 * lp;
-      v += t[0];
-      for (int kk = 1; kk <= 2 && 2 * kk - 1 < N; ++kk) {
-        int ph = ii * kk;
-        if (ph >= N) ph -= N;
-        const double a = t[2 * kk - 1], b = (2 * kk < N) ? t[2 * kk] : 0.0;
-        if (2 * kk == N) v += 0.5 * a * tw64[ph];
-        else v += a * tw64[ph] + b * tw64[N + ph];
-      }
-    }
-    const int j = jk[2 * lp], k = jk[2 * lp + 1];
-    if (phi_out) phi_out[cidx(g, ii + 1, j, k)] = v;
-    if (dph) {
-      dph[hidx(g, ii + 1, j, k)] = v;
-      if (k == g.nz) dph[hidx(g, ii + 1, j, g.nzc)] = v;
     }
   }
 }
@@ -2177,6 +2089,8 @@ void lds_optin(vrh_t *h) {
       ok = ok && hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lb) == hipSuccess;
   }
   (void)hipGetLastError();
+  if (lb > 65536) ok = ok && dense_lds_optin(lb);
+  (void)hipGetLastError();
   if (ok) { h->lds_block = lb; h->lds_cu = lc; }
 }
 
@@ -2269,9 +2183,10 @@ static void radial_launch(vrh_t *h, T *S, const T *ib, long nm, hipStream_t st) 
     hipLaunchKernelGGL((k_radial<T, 32>), grd, blk, 0, st, S, ib, nm, nlines, g.nr, ra, rc);
 }
 
-// z transform of the pressure solve on an axial mesh: every spectral line
-// (the nl lines of one z position are contiguous, so the array is a
-// column-major nl x nz matrix) times a dense nz x nz matrix, out of place.
+// z transform of the mixed path's pressure solve on an axial mesh (FP64 path:
+// launch_zdense): every spectral line (the nl lines of one z position are
+// contiguous, so the array is a column-major nl x nz matrix) times a dense
+// nz x nz matrix, out of place.
 // Forward: out(:, q) = sum_k in(:, k) Vinv(q, k); inverse: out(:, k) =
 // sum_q in(:, q) V(k, q).  The row-major matrices read column-major are
 // their transposes, the right operand of both products.
@@ -2343,59 +2258,61 @@ __global__ __launch_bounds__(256) void k_hz_scatter(const double *__restrict__ x
   }
 }
 
-template <typename TW> void launch_poisson(vrh_t *h, int irk, const double *ext_rhs, double *phi_out) {
-  const VGrid &g = h->g;
-  const int N = g.nt, logn = ilog2(N);
-  const bool pow2 = N >= 2 && (N & (N - 1)) == 0;
-  int LB = pow2 ? (h->fft_lines > 0 ? h->fft_lines : 1024 / N) : 2;
-  if (LB > 16) LB = 16;
-  if (pow2) {  // butterflies per thread of the LDS FFT: (LB/2) N / rmin <= qt * 256
-    while (LB > 2 && (LB / 2) * N / fft_min_radix(logn) > 256 * fft_qt<TW>()) LB /= 2;
-  }
-  if (LB < 2) LB = 2;
-  const long nlines = (long)g.nr * g.nz;
-  TW *S = (TW *)h->f.S;
-  double *S64 = (h->prec == VRH_MIXED) ? h->f.S64 : nullptr;
-  const double adt = h->rk[irk].a * h->dt;
-  const bool keep_dv = !pow2;   // the kernel's FP64 copy of the lines (direct DFT)
-  size_t sh1 = (keep_dv ? al16(sizeof(double) * LB * N) : 0) + al16(sizeof(TW) * LB * N);
-  if (S64) sh1 = al16(sh1 + sizeof(double) * (2 * (size_t)N + 10 * (size_t)LB));
-  sh1 = al16(al16(sh1 + sizeof(TW) * N) + sizeof(int) * 2 * LB) + sizeof(double) * 2 * LB;
-  { KTimer kt(h, KT_DIVFFT);
-  hipLaunchKernelGGL(k_divfft<TW>, dim3((unsigned)((nlines + LB - 1) / LB)), dim3(256), sh1, h->stream, g, h->coef,
-                     h->zmet, 1.0 / adt, h->f.dq1, h->f.dq2, h->f.dq3, ext_rhs, S, S64, h->d_twt, h->d_twt + N, LB, logn); }
-  // z transforms
-  const int nz = g.nz, lz = ilog2(nz);
+// One z transform of the pressure solve, in place on nl lines: the cosine
+// transform by FFT (nz a power of two) or as a dense product, or on an axial
+// mesh the product with its eigenvectors.
+template <typename T> static void z_transform(vrh_t *h, hipStream_t st, T *S, long nl, int dir, int want) {
+  const int nz = h->g.nz, lz = ilog2(nz);
+  if (h->zmet.m3 || (nz & (nz - 1)) != 0) { launch_zdense<T>(h, st, S, nl, dir); return; }
   // lines per block: a power of two, data + twiddles within 64 KB of LDS
   // (a tuned width may take the device's larger per-block LDS: 32 FP32
   // lines read whole 128-byte rows of the strided layout), one FFT
   // butterfly per thread with up to 1024 threads
-  auto lines = [&](size_t es, int want) {
-    const size_t lim = want > 0 ? (size_t)h->lds_block : 65536;
-    const int tmax = want > 0 ? 32 : 16;
-    int tl = 2;
-    while (tl * 2 <= tmax && (size_t)(tl * 2) * (nz + 1) * es + (size_t)(es == 4 ? 3 : 1) * nz * es <= lim &&
-           (tl * 2 / 2) * nz / fft_min_radix(lz) <= 1024)
-      tl *= 2;
-    if (want > 0) while (tl > 2 && tl > want) tl /= 2;
-    return tl;
-  };
-  auto threads = [&](int tl) {
-    const int b = (tl / 2) * nz / fft_min_radix(lz);
-    return b > 512 ? 1024 : b > 256 ? 512 : 256;
-  };
-  const int TL = lines(sizeof(TW), h->dct_lines), TL64 = lines(sizeof(double), 0);
-  const int ltl = ilog2(TL), ltl64 = ilog2(TL64);
-  const int NTD = threads(TL), NTD64 = threads(TL64);
-  const long nl = (long)N * g.nr;
+  const size_t es = sizeof(T), lim = want > 0 ? (size_t)h->lds_block : 65536;
+  const int tmax = want > 0 ? 32 : 16;
+  int tl = 2;
+  while (tl * 2 <= tmax && (size_t)(tl * 2) * (nz + 1) * es + (size_t)(es == 4 ? 3 : 1) * nz * es <= lim &&
+         (tl * 2 / 2) * nz / fft_min_radix(lz) <= 1024)
+    tl *= 2;
+  if (want > 0) while (tl > 2 && tl > want) tl /= 2;
+  const int b = (tl / 2) * nz / fft_min_radix(lz), nth = b > 512 ? 1024 : b > 256 ? 512 : 256;
   // tile lines, FFT twiddles, and in FP32 the Makhoul twiddles
-  const size_t sh2 = sizeof(TW) * ((size_t)TL * (nz + 1) + (size_t)(sizeof(TW) == 4 ? 3 : 1) * nz),
-               sh64 = sizeof(double) * ((size_t)TL64 * (nz + 1) + nz);
-  // The FP64 low-mode chain (mixed precision) reads only what k_divfft
-  // wrote to S64 and feeds only k_ifft: it runs on a side stream, forked
-  // after k_divfft and joined before k_ifft, beside the FP32 transforms.
-  // With the kernel timer on, or inside an ensemble graph, it stays in
-  // order on the handle's stream.
+  const size_t sh = es * ((size_t)tl * (nz + 1) + (size_t)(es == 4 ? 3 : 1) * nz);
+  hipLaunchKernelGGL(k_dctz<T>, dim3((unsigned)((nl + tl - 1) / tl)), dim3(nth), sh, st, S, nl, nz, lz, tl, ilog2(tl),
+                     dir, h->d_twz, h->d_twz + nz, h->d_ez, h->d_ez + nz);
+}
+
+template <typename TW> void launch_poisson(vrh_t *h, int irk, const double *ext_rhs, double *phi_out) {
+  const VGrid &g = h->g;
+  const int N = g.nt, logn = ilog2(N), nz = g.nz;
+  const bool pow2 = (N & (N - 1)) == 0;
+  const long nlines = (long)g.nr * nz, nl = (long)N * g.nr, nl64 = 5L * g.nr;
+  TW *S = (TW *)h->f.S;
+  double *S64 = (h->prec == VRH_MIXED) ? h->f.S64 : nullptr;
+  const double adt = h->rk[irk].a * h->dt;
+  int LB = h->fft_lines > 0 ? h->fft_lines : 1024 / N;
+  if (LB > 16) LB = 16;
+  // butterflies per thread of the LDS FFT: (LB/2) N / rmin <= qt * 256
+  while (LB > 2 && (LB / 2) * N / fft_min_radix(logn) > 256 * fft_qt<TW>()) LB /= 2;
+  if (LB < 2) LB = 2;
+  const dim3 fgrd((unsigned)((nlines + LB - 1) / LB));
+  {
+    KTimer kt(h, KT_DIVFFT);
+    if (pow2) {
+      size_t sh = al16(sizeof(TW) * LB * N);
+      if (S64) sh = al16(sh + sizeof(double) * (2 * (size_t)N + 10 * (size_t)LB));
+      sh = al16(al16(sh + sizeof(TW) * N) + sizeof(int) * 2 * LB) + sizeof(double) * 2 * LB;
+      hipLaunchKernelGGL(k_divfft<TW>, fgrd, dim3(256), sh, h->stream, g, h->coef, h->zmet, 1.0 / adt, h->f.dq1,
+                         h->f.dq2, h->f.dq3, ext_rhs, S, S64, h->d_twt, h->d_twt + N, LB, logn);
+    } else {
+      launch_divdft<TW>(h, 1.0 / adt, ext_rhs, S, S64);
+    }
+  }
+  // The FP64 low-mode chain (mixed precision) reads only what the forward
+  // theta transform wrote to S64 and feeds only the inverse one: it runs on
+  // a side stream, forked and joined between them, beside the FP32
+  // transforms.  With the kernel timer on, or inside an ensemble graph, it
+  // stays in order on the handle's stream.
   const bool par = S64 && !h->kt_on && !h->serial_sweeps;
   hipStream_t s64 = par ? h->side[0] : h->stream;
   const int ie = (irk >= 1 && irk <= 3) ? irk : 0;
@@ -2404,17 +2321,13 @@ template <typename TW> void launch_poisson(vrh_t *h, int irk, const double *ext_
     (void)hipStreamWaitEvent(s64, h->poi_ev[ie][0], 0);
   }
   if (S64 && h->zmet.m3) {
-    const long nl64 = 5L * g.nr;
     zgemm(h, s64, S64, h->S2_64, nl64, 1);
     radial_launch<double>(h, h->S2_64, h->f.ib64, 5, s64);
     zgemm(h, s64, h->S2_64, S64, nl64, -1);
   } else if (S64) {
-    const long nl64 = 5L * g.nr;
-    hipLaunchKernelGGL(k_dctz<double>, dim3((unsigned)((nl64 + TL64 - 1) / TL64)), dim3(NTD64), sh64, s64, S64,
-                       nl64, nz, lz, TL64, ltl64, 1, h->d_twz, h->d_twz + nz, h->d_ez, h->d_ez + nz);
+    z_transform<double>(h, s64, S64, nl64, 1, 0);
     radial_launch<double>(h, S64, h->f.ib64, 5, s64);
-    hipLaunchKernelGGL(k_dctz<double>, dim3((unsigned)((nl64 + TL64 - 1) / TL64)), dim3(NTD64), sh64, s64, S64,
-                       nl64, nz, lz, TL64, ltl64, -1, h->d_twz, h->d_twz + nz, h->d_ez, h->d_ez + nz);
+    z_transform<double>(h, s64, S64, nl64, -1, 0);
   }
   // per-mode iterative solve of the positions >= hz_pos0: stage their
   // right-hand sides before the direct path overwrites them
@@ -2422,19 +2335,20 @@ template <typename TW> void launch_poisson(vrh_t *h, int irk, const double *ext_
   if (h->hz)
     hipLaunchKernelGGL(k_hz_gather<TW>, hzg, dim3(256), 0, h->stream, S, hz_step_input(h->hz), N, g.nr, nz,
                        h->hz_pos0);
-  if (h->zmet.m3) {
-    TW *S2 = (TW *)h->S2;
-    { KTimer kt(h, KT_DCT_FWD); zgemm(h, h->stream, S, S2, nl, 1); }
-    radial_launch<TW>(h, S2, (const TW *)h->f.ib, N, h->stream);
-    { KTimer kt(h, KT_DCT_INV); zgemm(h, h->stream, S2, S, nl, -1); }
-  } else {
-  { KTimer kt(h, KT_DCT_FWD);
-  hipLaunchKernelGGL(k_dctz<TW>, dim3((unsigned)((nl + TL - 1) / TL)), dim3(NTD), sh2, h->stream, S, nl, nz, lz, TL,
-                     ltl, 1, h->d_twz, h->d_twz + nz, h->d_ez, h->d_ez + nz); }
-  radial_launch<TW>(h, S, (const TW *)h->f.ib, N, h->stream);
-  { KTimer kt(h, KT_DCT_INV);
-  hipLaunchKernelGGL(k_dctz<TW>, dim3((unsigned)((nl + TL - 1) / TL)), dim3(NTD), sh2, h->stream, S, nl, nz, lz, TL,
-                     ltl, -1, h->d_twz, h->d_twz + nz, h->d_ez, h->d_ez + nz); }
+  bool done = false;
+  if constexpr (sizeof(TW) == 4) {
+    if (h->zmet.m3) {  // mixed path on an axial mesh: library GEMMs, out of place
+      TW *S2 = (TW *)h->S2;
+      { KTimer kt(h, KT_DCT_FWD); zgemm(h, h->stream, S, S2, nl, 1); }
+      radial_launch<TW>(h, S2, (const TW *)h->f.ib, N, h->stream);
+      { KTimer kt(h, KT_DCT_INV); zgemm(h, h->stream, S2, S, nl, -1); }
+      done = true;
+    }
+  }
+  if (!done) {
+    { KTimer kt(h, KT_DCT_FWD); z_transform<TW>(h, h->stream, S, nl, 1, h->dct_lines); }
+    radial_launch<TW>(h, S, (const TW *)h->f.ib, N, h->stream);
+    { KTimer kt(h, KT_DCT_INV); z_transform<TW>(h, h->stream, S, nl, -1, h->dct_lines); }
   }
   if (par) {
     (void)hipEventRecord(h->poi_ev[ie][1], s64);
@@ -2449,11 +2363,13 @@ template <typename TW> void launch_poisson(vrh_t *h, int irk, const double *ext_
     hipLaunchKernelGGL(k_hz_scatter<TW>, hzg, dim3(256), 0, h->stream, hz_step_output(h->hz), S, N, g.nr, nz,
                        h->hz_pos0);
   }
+  double *dph = ext_rhs ? nullptr : h->f.dph;
+  KTimer kti(h, KT_IFFT);
+  if (!pow2) { launch_idft<TW>(h, S, S64, phi_out, dph); return; }
   size_t sh3 = al16(sizeof(TW) * ((size_t)2 * LB * N + N)) + sizeof(int) * 2 * LB;
   if (S64) sh3 = al16(sh3) + sizeof(double) * (5 * (size_t)LB + 2 * (size_t)N);
-  KTimer kti(h, KT_IFFT);
-  hipLaunchKernelGGL(k_ifft<TW>, dim3((unsigned)((nlines + LB - 1) / LB)), dim3(256), sh3, h->stream, g, S, S64,
-                     phi_out, ext_rhs ? nullptr : h->f.dph, h->d_twt, h->d_twt + N, LB, logn);
+  hipLaunchKernelGGL(k_ifft<TW>, fgrd, dim3(256), sh3, h->stream, g, S, S64, phi_out, dph, h->d_twt, h->d_twt + N, LB,
+                     logn);
 }
 
 template <typename TW> void launch_project(vrh_t *h, int irk) {
