@@ -1658,7 +1658,7 @@ __global__ __launch_bounds__(256) void k_ifft(VGrid g, const TW *__restrict__ S,
 
 // ---------------------------------------------------------------------------
 // upsol (divergence.F90:69-236) fused with uppres (divergence.F90:239-480).
-// A block owns a 64 (theta) x R (r) column tile and marches up a chunk of z
+// A block owns a W (theta) x R (r) column tile and marches up a chunk of z
 // planes.  The planes k-2..k+1 of dph live in a 4-slot LDS ring (with two
 // theta columns and two r rows of halo on the low side, one on the high
 // side), so each dph value is fetched from HBM about once; the gradient
@@ -1666,15 +1666,15 @@ __global__ __launch_bounds__(256) void k_ifft(VGrid g, const TW *__restrict__ S,
 // them.  Everything that depends on the thread's r row only (metric ratios,
 // reciprocals of rm) is hoisted out of the z loop.
 // ---------------------------------------------------------------------------
-template <typename TW, int R, bool ZS>
-__global__ __launch_bounds__(64 * R) void k_project(VGrid g, VCoef c, ZMet zm, double adt, double be, int kchunk,
+template <int W, int R, bool ZS>
+__global__ __launch_bounds__(W * R) void k_project(VGrid g, VCoef c, ZMet zm, double adt, double be, int kchunk,
                                                     const double *__restrict__ dph, const double *__restrict__ dq1,
                                                     const double *__restrict__ dq2, const double *__restrict__ dq3,
                                                     double *__restrict__ q1, double *__restrict__ q2,
                                                     double *__restrict__ q3, double *__restrict__ prg1,
                                                     double *__restrict__ prg2, double *__restrict__ prg3,
                                                     double *__restrict__ pres, int *__restrict__ flag) {
-  constexpr int W = 64, LC = W + 3, LR = R + 3, NE = LR * LC, NT = 64 * R;
+  constexpr int LC = W + 3, LR = R + 3, NE = LR * LC, NT = W * R;
   constexpr int NL = (NE + NT - 1) / NT;
   __shared__ double ring[4][LR][LC + 1];
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * W + tx;
@@ -2376,11 +2376,19 @@ template <typename TW> void launch_project(vrh_t *h, int irk) {
   const VGrid &g = h->g;
   const double adt = h->rk[irk].a * h->dt;
   const double be = 0.5 * (h->rk[irk].a * h->dt) / h->Re;
-  constexpr int R = 4;
-  const int kchunk = 32;
-  dim3 blk(64, R), grd((g.nt + 63) / 64, (g.nrc + 1 + R - 1) / R, (g.nzc + kchunk - 1) / kchunk);
+  // Planes per block: 8 (a block re-reads three planes of phi, 2 % of its
+  // bytes; its waves' first loads are exposed once per chunk).  us at 4, 8, 16, 32 planes:
+  // 128x256x512 411, 387, 391, 412; 129x128x128 80, 77, 87, 88;
+  // 32x64x128 19, 21, 27, 45.  4 where 8 leaves fewer than 2 blocks per CU.
+  // Up to 32 angles a tile of 32 x 8 idles no lanes (32x64x128: 15.5 us
+  // with 4 planes).
+  const int W = g.nt <= 32 ? 32 : 64, R = 256 / W;
+  const long cols = (long)((g.nt + W - 1) / W) * ((g.nrc + 1 + R - 1) / R);
+  const int kchunk = cols * ((g.nzc + 7) / 8) < 512 ? 4 : 8;
+  dim3 blk(W, R), grd((g.nt + W - 1) / W, (g.nrc + 1 + R - 1) / R, (g.nzc + kchunk - 1) / kchunk);
   KTimer kt(h, KT_PROJECT);
-  auto kern = h->zmet.m3 ? k_project<TW, R, true> : k_project<TW, R, false>;
+  auto kern = W == 64 ? (h->zmet.m3 ? k_project<64, 4, true> : k_project<64, 4, false>)
+                      : (h->zmet.m3 ? k_project<32, 8, true> : k_project<32, 8, false>);
   hipLaunchKernelGGL(kern, grd, blk, 0, h->stream, g, h->coef, h->zmet, adt, be, kchunk, h->f.dph, h->f.dq1,
                      h->f.dq2, h->f.dq3, h->f.q1, h->f.q2, h->f.q3, h->f.prg1, h->f.prg2,
                      h->f.prg3, h->f.pres, h->f.flag);
