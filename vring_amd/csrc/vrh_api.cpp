@@ -223,8 +223,8 @@ void graph_invalidate(vrh_t *h) {
 
 namespace {
 // Everything that depends on the radial mesh, recomputed on the host and
-// uploaded into the handle's buffers: the metric vectors, the theta PCR
-// depths, the line-sweep coefficients, the radial Poisson rows and pivots,
+// uploaded into the handle's buffers: the metric vectors, the explicit
+// kernels' tables, the line-sweep coefficients, the radial Poisson rows and pivots,
 // the inlet area.
 int refresh_mesh(vrh_t *h) {
   host_mesh_vectors(h);
@@ -233,25 +233,10 @@ int refresh_mesh(vrh_t *h) {
   std::vector<double> vb((size_t)kNumVec * nv);
   for (int q = 0; q < kNumVec; q++) std::memcpy(&vb[(size_t)q * nv], h->hv[q].data(), nv * sizeof(double));
   if ((rc = h2d(h, h->d_vec, vb.data(), vb.size() * sizeof(double)))) return rc;
-  // parallel-cyclic-reduction depth of the theta solves: log2(nt) for a
-  // power-of-two nt, otherwise until the off-diagonal ratio is below 1e-18
-  for (int irk = 1; irk <= 3; irk++) {
-    const double betadx = 0.5 * h->rk[irk].a * h->dt / h->Re;
-    int lv = 0;
-    if ((h->nt & (h->nt - 1)) == 0) {
-      while ((1 << lv) < h->nt) lv++;
-    } else {
-      for (int j = 1; j <= h->nr; j++)
-        for (int which = 0; which < 2; which++) {
-          double acc = betadx * h->hv[which ? 14 : 10][j];
-          double a = -acc, b = 1.0 + 2.0 * acc;
-          int l = 0;
-          while (fabs(a) >= 1e-18 * fabs(b) && l < 40) { double al = -a / b; b += 2.0 * al * a; a *= al; l++; }
-          if (l > lv) lv = l;
-        }
-    }
-    h->theta_levels[irk] = lv;
-  }
+  std::vector<double> et;
+  explicit_tables(h, et);
+  if (!h->d_rowc && (rc = dalloc(h, &h->d_rowc, et.size()))) return rc;
+  if ((rc = h2d(h, h->d_rowc, et.data(), et.size() * sizeof(double)))) return rc;
   if ((rc = build_line_coefs(h))) return rc;
   std::vector<double> aab(h->nr + 1, 0.0), ccb(h->nr + 1, 0.0);
   for (int j = 1; j <= h->nr; j++) { double dd; host_radial_row(h, j, aab[j], ccb[j], dd); }
@@ -420,7 +405,7 @@ int vrh_destroy(vrh_t *h) {
                   f.q3, f.dq1, f.dq2, f.dq3, f.pres, f.dph, f.ru1, f.ru2, f.ru3, f.r1, f.r2, f.r3, f.prg1, f.prg2,
                   f.prg3, f.S, f.ib, f.S64, f.ib64, f.csort, f.dq3no, f.corr3n, f.flag};
   for (void *p : ptrs) if (p) hipFree(p);
-  void *zp[] = {h->d_zmet, h->d_zv, h->d_zvf, h->d_zeig, h->S2, h->S2_64, h->d_zcos, h->d_tdft};
+  void *zp[] = {h->d_rowc, h->d_zmet, h->d_zv, h->d_zvf, h->d_zeig, h->S2, h->S2_64, h->d_zcos, h->d_tdft};
   for (void *p : zp) if (p) hipFree(p);
   if (h->blas) rocblas_destroy_handle((rocblas_handle)h->blas);
   for (auto &e : h->kt_pool) hipEventDestroy(e);

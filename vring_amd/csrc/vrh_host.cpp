@@ -67,6 +67,65 @@ void host_mesh_vectors(vrh_t *h) {
     if (rc[j] <= (double)0.4999f) h->jlim = j;
 }
 
+// Tables of the explicit kernels.  The theta systems (-a, 1 + 2a, -a) of a row
+// are solved by cyclic reduction; each level couples twice as far with the
+// ratio a/b squared, so a row stops where its couplings no longer reach a
+// bit of the result: below 1e-18 of the diagonal in FP64 (at the latest after
+// log2 of a power-of-two ntheta, where the last diagonal takes both
+// couplings).  The FP32 form goes on to 1e-30, within the depth of the
+// deepest row to 1e-18, so that values next to exact zeros keep their bits.
+// Most rows of the workloads need 3 or 4 of 7 levels, the ones at the axis all.
+void explicit_tables(vrh_t *h, std::vector<double> &tab) {
+  const int nr = h->nr, nt = h->nt;
+  const std::vector<double> *v = h->hv;
+  tab.assign((size_t)(nr + 1) * (kRowCoefs + 3 * kPcrRow), 0.0);
+  const int src[18] = {2, 3, 4, 5, 6, 8, 7, 9, 10, 11, 12, 13, 14, 15, 17, 16, 18, 19};
+  for (int j = 1; j <= nr; j++) {
+    double *cf = &tab[(size_t)j * kRowCoefs];
+    for (int q = 0; q < 18; q++) cf[q] = v[src[q]][j];
+    cf[18] = 1.0 / v[0][j + 1];
+    cf[19] = 1.0 / v[0][j];
+    cf[20] = 1.0 / v[0][j == 1 ? 1 : j - 1];
+  }
+  const bool pow2 = (nt & (nt - 1)) == 0;
+  int full = 0;
+  while ((1 << full) < nt) full++;
+  for (int irk = 1; irk <= 3; irk++) {
+    const double betadx = 0.5 * h->rk[irk].a * h->dt / h->Re;
+    auto depth = [&](int j, double thr, int cap) {
+      int lv = 0;
+      for (int which = 0; which < 2; which++) {
+        const double acc = betadx * v[which ? 14 : 10][j];
+        double a = -acc, b = 1.0 + 2.0 * acc;
+        int l = 0;
+        while (l < cap && std::fabs(a) >= thr * std::fabs(b)) { const double al = -a / b; b = std::fma(2.0 * al, a, b); a *= al; l++; }
+        lv = std::max(lv, l);
+      }
+      return lv;
+    };
+    int deepest = pow2 ? full : 0;
+    if (!pow2)
+      for (int j = 1; j <= nr; j++) deepest = std::max(deepest, depth(j, 1e-18, kMaxPcrLevels));
+    h->theta_levels[irk] = deepest;
+    for (int j = 1; j <= nr; j++) {
+      double *p = &tab[(size_t)(nr + 1) * (kRowCoefs + (size_t)(irk - 1) * kPcrRow) + (size_t)j * kPcrRow];
+      const int lv = depth(j, h->prec == VRH_MIXED ? 1e-30 : 1e-18, deepest);
+      p[2] = lv;
+      for (int which = 0; which < 2; which++) {
+        const double acc = betadx * v[which ? 14 : 10][j];
+        double a = -acc, b = 1.0 + 2.0 * acc;
+        for (int l = 0; l < lv; l++) {
+          const double al = -a / b;
+          p[kPcrHead + 2 * l + which] = al;
+          b = std::fma(2.0 * al, a, b);
+          a = al * a;
+        }
+        p[which] = 1.0 / (pow2 ? std::fma(2.0, a, b) : b);
+      }
+    }
+  }
+}
+
 // Partitioned-Thomas coefficients from (aa, bb, cc) with aa(1)=0, cc(n)=0
 // forced as solve_lap_par does (tripar.F90:30-35); Thomas pivots as
 // solve_lap_thom (tripar.F90:128-138).

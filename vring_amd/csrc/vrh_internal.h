@@ -66,6 +66,13 @@ struct LineCoef {
   int n, P;
 };
 
+// Tables of the explicit kernels (explicit_tables), one row per r index j =
+// 0..nr: kRowCoefs metric coefficients (cf[...] in the kernels), and per
+// substep kPcrRow numbers of the theta solves: the factors 1/diagonal of the
+// q1/q3 and the q2 systems after the reduction, its depth, a pad, then the two
+// systems' reduction ratios level by level.
+constexpr int kMaxPcrLevels = 40, kRowCoefs = 24, kPcrHead = 4, kPcrRow = kPcrHead + 2 * kMaxPcrLevels;
+
 // divq's right-hand side at a cell (divergence.F90:31-41) from the three
 // one-sided differences: wr = 1/rm, ct, cr, cz the difference factors.  The
 // fused operations are written out, so that every kernel rounds alike.
@@ -217,7 +224,9 @@ struct vrh_s {
   int explicit_variant = -1;  // 0: plane per block, 1: z marching, 2/3: one wave per r row, -1: default
   // LDS a block may take beyond 64 KB (after the kernels' opt-in) and LDS per CU
   int lds_block = 65536, lds_cu = 65536;
-  int theta_levels[4];  // PCR levels of the theta solve per substep
+  int theta_levels[4];  // deepest theta reduction of a row, per substep
+  double *d_rowc = nullptr;  // tables of the explicit kernels: row coefficients, then substeps 1..3
+  double *pcrt(int irk) const { return d_rowc + (size_t)(nr + 1) * (kRowCoefs + (size_t)(irk - 1) * kPcrRow); }
   // transform tables (double): theta twiddles (nt/2 complex), z twiddles
   // (nz/2 complex), z post-twiddles (nz complex)
   double *d_twt, *d_twz, *d_ez;
@@ -272,6 +281,7 @@ void ktimer_harvest(vrh_t *h);
 void host_mesh_vectors(vrh_t *h);
 void host_line_coefs(vrh_t *h, int irk, std::vector<double> out[6][7], const int M[6]);
 int build_line_coefs(vrh_t *h);
+void explicit_tables(vrh_t *h, std::vector<double> &tab);
 void host_radial_row(const vrh_t *h, int j, double &aa, double &cc, double &dd);
 void host_radial_pivots(vrh_t *h, std::vector<double> &ib, std::vector<double> &ib64);
 // Pressure-solve z transforms on an axial mesh with z differences m3 (centres)

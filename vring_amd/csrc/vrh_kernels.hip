@@ -102,12 +102,10 @@ __global__ void k_scalars(double *sc, double dt, double a1, double a2, double a3
 // comes from LDS; the next plane is prefetched into registers while the
 // current one is computed.  The theta systems (constant coefficients
 // (-acc, 1+2acc, -acc) per r row) are solved by parallel cyclic reduction
-// on LDS-resident lines; the reduction ratios of each row are computed once
-// per block.  The inlet planes q1s, q2s, q3s are zero
+// on LDS-resident lines.  Row coefficients, reduction ratios and the depth
+// of each row's reduction come from host tables (explicit_tables).  The inlet planes q1s, q2s, q3s are zero
 // (momentum_terms_swirl.F90:216-223).
 // ---------------------------------------------------------------------------
-constexpr int kMaxPcrLevels = 40;
-constexpr int kRowCoefs = 24;
 
 // z second differences on the axial mesh (ZMet, vrh_set_axial_mesh): at a
 // cell centre (q1, q2, p, the first two pressure-gradient components) with
@@ -122,7 +120,7 @@ template <typename T> __device__ __forceinline__ T zd2f(const ZMet &z, int k, T 
 }
 
 template <typename TW, typename TC, bool ZS>
-__global__ __launch_bounds__(512, sizeof(TC) == 4 ? 4 : 3) void k_explicit_march(VGrid g, VCoef c, VRK rk, ZMet zm, double betadx, int nlev, int kchunk,
+__global__ __launch_bounds__(512, sizeof(TC) == 4 ? 4 : 3) void k_explicit_march(VGrid g, const double *__restrict__ rowc, const double *__restrict__ pcrt, VRK rk, ZMet zm, int kchunk,
                                                   const double *__restrict__ q1, const double *__restrict__ q2,
                                                   const double *__restrict__ q3, const double *__restrict__ prg1,
                                                   const double *__restrict__ prg2, const double *__restrict__ prg3,
@@ -138,37 +136,16 @@ __global__ __launch_bounds__(512, sizeof(TC) == 4 ? 4 : 3) void k_explicit_march
   const int j0 = 1 + bx * RJ;
   const int kb = 1 + by * kchunk, ke = min(kb + kchunk - 1, nz);
   const int LRW = RJ + 2, PL = LRW * NTP;
-  double *pcr = reinterpret_cast<double *>(smem_raw);             // [RJ][kMaxPcrLevels][2] + [RJ][2]
-  double *fin = pcr + RJ * kMaxPcrLevels * 2;
-  TC *cfs = reinterpret_cast<TC *>(fin + RJ * 2);                 // [RJ][kRowCoefs]
+  double *pcr = reinterpret_cast<double *>(smem_raw);             // [RJ][kPcrRow]
+  TC *cfs = reinterpret_cast<TC *>(pcr + RJ * kPcrRow);           // [RJ][kRowCoefs]
   TC *ring = cfs + RJ * kRowCoefs;                                // [3 slots][3 arrays][LRW][NTP]
   TC *fb = ring + 9 * PL;                                         // [2][3][RJ][NTP]
   const int j = j0 + tj;
   const bool cell = (ti < nt) && (j <= nr);
   const int jc = (j <= nr) ? j : nr;
-  // PCR ratios of this row (one lane per row)
-  if (ti == 0) {
-    double a1 = -(betadx * c.s1t11[jc]), b1 = 1.0 + 2.0 * (betadx * c.s1t11[jc]);
-    double a2 = -(betadx * c.s2t11[jc]), b2 = 1.0 + 2.0 * (betadx * c.s2t11[jc]);
-    for (int lvl = 0; lvl < nlev; ++lvl) {
-      const double al1 = -a1 / b1, al2 = -a2 / b2;
-      pcr[(tj * kMaxPcrLevels + lvl) * 2] = al1;
-      pcr[(tj * kMaxPcrLevels + lvl) * 2 + 1] = al2;
-      b1 = b1 + 2.0 * al1 * a1; a1 = al1 * a1;
-      b2 = b2 + 2.0 * al2 * a2; a2 = al2 * a2;
-    }
-    const bool pow2 = nt >= 2 && (nt & (nt - 1)) == 0;
-    fin[tj * 2] = 1.0 / (pow2 ? b1 + 2.0 * a1 : b1);
-    fin[tj * 2 + 1] = 1.0 / (pow2 ? b2 + 2.0 * a2 : b2);
-    const int jm = (jc == 1) ? 1 : jc - 1;
-    TC *cf = cfs + tj * kRowCoefs;
-    cf[0] = (TC)c.h1d11[jc]; cf[1] = (TC)c.h1d22d[jc]; cf[2] = (TC)c.h1d22n[jc]; cf[3] = (TC)c.h1dare[jc];
-    cf[4] = (TC)c.h2d11[jc]; cf[5] = (TC)c.h2d22p[jc]; cf[6] = (TC)c.h2d22m[jc]; cf[7] = (TC)c.h2dare[jc];
-    cf[8] = (TC)c.s1t11[jc]; cf[9] = (TC)c.s1t2n[jc]; cf[10] = (TC)c.s1t2s[jc]; cf[11] = (TC)c.s1t2c[jc];
-    cf[12] = (TC)c.s2t11[jc]; cf[13] = (TC)c.s2t2p[jc]; cf[14] = (TC)c.s2t2c[jc]; cf[15] = (TC)c.s2t2m[jc];
-    cf[16] = (TC)c.s3t2n[jc]; cf[17] = (TC)c.s3t2s[jc];
-    cf[18] = (TC)(1.0 / c.rm[jc + 1]); cf[19] = (TC)(1.0 / c.rm[jc]); cf[20] = (TC)(1.0 / c.rm[jm]);
-  }
+  // this row's coefficients, and its reduction ratios, depth and last factors
+  if (ti < kRowCoefs) cfs[tj * kRowCoefs + ti] = (TC)rowc[(size_t)jc * kRowCoefs + ti];
+  for (int q = ti; q < kPcrRow; q += NTP) pcr[tj * kPcrRow + q] = pcrt[(size_t)jc * kPcrRow + q];
   // plane fetch: element e = tid + l*NTH of the (LRW x NTP) tile, three arrays
   constexpr int NL = 3;
   long goff[NL];
@@ -363,10 +340,14 @@ __global__ __launch_bounds__(512, sizeof(TC) == 4 ? 4 : 3) void k_explicit_march
     f1[ti] = v1; f2[ti] = v2; f3[ti] = v3;
     __syncthreads();
     int sm = 1 % nt;
-    for (int lvl = 0; lvl < nlev; ++lvl) {
-      const TC al1 = (TC)pcr[(tj * kMaxPcrLevels + lvl) * 2], al2 = (TC)pcr[(tj * kMaxPcrLevels + lvl) * 2 + 1];
+    const double *pr = pcr + tj * kPcrRow;
+    const int mylev = (int)pr[2];
+    int blev = 0;  // the block's deepest row (its barriers)
+    for (int r = 0; r < RJ; r++) blev = max(blev, (int)pcr[r * kPcrRow + 2]);
+    for (int lvl = 0; lvl < blev; ++lvl) {
+      const TC al1 = (TC)pr[kPcrHead + 2 * lvl], al2 = (TC)pr[kPcrHead + 2 * lvl + 1];
       TC n1 = v1, n2 = v2, n3 = v3;
-      if (ti < nt) {
+      if (ti < nt && lvl < mylev) {
         int imv = ti - sm; if (imv < 0) imv += nt;
         int ipv = ti + sm; if (ipv >= nt) ipv -= nt;
         n1 = v1 + al1 * (f1[imv] + f1[ipv]);
@@ -381,7 +362,7 @@ __global__ __launch_bounds__(512, sizeof(TC) == 4 ? 4 : 3) void k_explicit_march
       __syncthreads();
     }
     if (cell) {
-      const TC d1 = (TC)fin[tj * 2], d2 = (TC)fin[tj * 2 + 1];
+      const TC d1 = (TC)pr[0], d2 = (TC)pr[1];
       r1[o] = v1 * d1;
       if (j >= 2) r2[o] = v2 * d2;
       if (k >= 2) r3[o] = v3 * d1;
@@ -412,16 +393,13 @@ __global__ __launch_bounds__(512, sizeof(TC) == 4 ? 4 : 3) void k_explicit_march
 #undef irmm
 }
 
-// Variant with one z plane per block (no z marching): every stencil operand
-// is read through L1/L2.  Fewer registers and LDS than the marching form;
-// the autotuner picks whichever is faster for the precision and grid.
 // The explicit kernel with one wavefront per r row (nθ <= 64 CPL): each
 // lane computes the cells θ = lane + 64 c, and the periodic θ solves run by
 // PCR inside the wavefront (LDS exchange ordered by wave-local fences, no
 // block barrier per level), which leaves two block barriers per z plane for
 // the plane ring.  Same arithmetic as k_explicit_march.
 template <typename TW, typename TC, int CPL, int RJT, int WPE, bool ZS>
-__global__ __launch_bounds__(64 * RJT, WPE) void k_explicit_wave(VGrid g, VCoef c, VRK rk, ZMet zm, double betadx, int nlev, int kchunk,
+__global__ __launch_bounds__(64 * RJT, WPE) void k_explicit_wave(VGrid g, const double *__restrict__ rowc, const double *__restrict__ pcrt, VRK rk, ZMet zm, int nlev, int kchunk,
                                                   const double *__restrict__ q1, const double *__restrict__ q2,
                                                   const double *__restrict__ q3, const double *__restrict__ prg1,
                                                   const double *__restrict__ prg2, const double *__restrict__ prg3,
@@ -439,36 +417,16 @@ __global__ __launch_bounds__(64 * RJT, WPE) void k_explicit_wave(VGrid g, VCoef 
   const int j0 = 1 + bx * RJ;
   const int kb = 1 + by * kchunk, ke = min(kb + kchunk - 1, nz);
   const int LRW = RJ + 2, PL = LRW * NTP;
-  double *pcr = reinterpret_cast<double *>(smem_raw);             // [RJ][nlev][2] + [RJ][2]
-  double *fin = pcr + RJ * nlev * 2;
-  TC *cfs = reinterpret_cast<TC *>(fin + RJ * 2);                 // [RJ][kRowCoefs]
+  const int prow = kPcrHead + 2 * nlev;
+  double *pcr = reinterpret_cast<double *>(smem_raw);             // [RJ][prow]
+  TC *cfs = reinterpret_cast<TC *>(pcr + RJ * prow);              // [RJ][kRowCoefs]
   TC *ring = cfs + RJ * kRowCoefs;                                // [3 slots][3 arrays][LRW][NTP]
   TC *fb = ring + 9 * PL;                                         // [2][3][RJ][NTP]
   const int j = j0 + tj;
   const int jc = (j <= nr) ? j : nr;
-  // PCR ratios of this row (one lane per row)
-  if (lane == 0) {
-    double a1 = -(betadx * c.s1t11[jc]), b1 = 1.0 + 2.0 * (betadx * c.s1t11[jc]);
-    double a2 = -(betadx * c.s2t11[jc]), b2 = 1.0 + 2.0 * (betadx * c.s2t11[jc]);
-    for (int lvl = 0; lvl < nlev; ++lvl) {
-      const double al1 = -a1 / b1, al2 = -a2 / b2;
-      pcr[(tj * nlev + lvl) * 2] = al1;
-      pcr[(tj * nlev + lvl) * 2 + 1] = al2;
-      b1 = b1 + 2.0 * al1 * a1; a1 = al1 * a1;
-      b2 = b2 + 2.0 * al2 * a2; a2 = al2 * a2;
-    }
-    const bool pow2 = nt >= 2 && (nt & (nt - 1)) == 0;
-    fin[tj * 2] = 1.0 / (pow2 ? b1 + 2.0 * a1 : b1);
-    fin[tj * 2 + 1] = 1.0 / (pow2 ? b2 + 2.0 * a2 : b2);
-    const int jm = (jc == 1) ? 1 : jc - 1;
-    TC *cf = cfs + tj * kRowCoefs;
-    cf[0] = (TC)c.h1d11[jc]; cf[1] = (TC)c.h1d22d[jc]; cf[2] = (TC)c.h1d22n[jc]; cf[3] = (TC)c.h1dare[jc];
-    cf[4] = (TC)c.h2d11[jc]; cf[5] = (TC)c.h2d22p[jc]; cf[6] = (TC)c.h2d22m[jc]; cf[7] = (TC)c.h2dare[jc];
-    cf[8] = (TC)c.s1t11[jc]; cf[9] = (TC)c.s1t2n[jc]; cf[10] = (TC)c.s1t2s[jc]; cf[11] = (TC)c.s1t2c[jc];
-    cf[12] = (TC)c.s2t11[jc]; cf[13] = (TC)c.s2t2p[jc]; cf[14] = (TC)c.s2t2c[jc]; cf[15] = (TC)c.s2t2m[jc];
-    cf[16] = (TC)c.s3t2n[jc]; cf[17] = (TC)c.s3t2s[jc];
-    cf[18] = (TC)(1.0 / c.rm[jc + 1]); cf[19] = (TC)(1.0 / c.rm[jc]); cf[20] = (TC)(1.0 / c.rm[jm]);
-  }
+  // this row's coefficients, and its reduction ratios, depth and last factors
+  if (lane < kRowCoefs) cfs[tj * kRowCoefs + lane] = (TC)rowc[(size_t)jc * kRowCoefs + lane];
+  for (int q = lane; q < prow; q += 64) pcr[tj * prow + q] = pcrt[(size_t)jc * kPcrRow + q];
   // plane fetch: element e = tid + l*NTH of the (LRW x NTP) tile, three arrays
   constexpr int NL = (CPL * (RJT + 2) + RJT - 1) / RJT;  // ceil((RJ + 2) NTP / (64 RJ))
   long goff[NL];
@@ -677,8 +635,10 @@ __global__ __launch_bounds__(64 * RJT, WPE) void k_explicit_wave(VGrid g, VCoef 
     }
     wave_sync();
     int sm = 1 % nt;
-    for (int lvl = 0; lvl < nlev; ++lvl) {
-      const TC al1 = (TC)pcr[(tj * nlev + lvl) * 2], al2 = (TC)pcr[(tj * nlev + lvl) * 2 + 1];
+    const double *pr = pcr + tj * prow;
+    const int mylev = __builtin_amdgcn_readfirstlane((int)pr[2]);
+    for (int lvl = 0; lvl < mylev; ++lvl) {
+      const TC al1 = (TC)pr[kPcrHead + 2 * lvl], al2 = (TC)pr[kPcrHead + 2 * lvl + 1];
       TC n1[CPL], n2[CPL], n3[CPL];
 #pragma unroll
       for (int cc = 0; cc < CPL; cc++) {
@@ -703,7 +663,7 @@ __global__ __launch_bounds__(64 * RJT, WPE) void k_explicit_wave(VGrid g, VCoef 
       }
       wave_sync();
     }
-    const TC d1 = (TC)fin[tj * 2], d2 = (TC)fin[tj * 2 + 1];
+    const TC d1 = (TC)pr[0], d2 = (TC)pr[1];
 #pragma unroll
     for (int cc = 0; cc < CPL; cc++) {
       const int ti = lane + 64 * cc;
@@ -740,8 +700,14 @@ __global__ __launch_bounds__(64 * RJT, WPE) void k_explicit_wave(VGrid g, VCoef 
 #undef irmm
 }
 
-template <typename TW, typename TC, bool ZS>
-__global__ __launch_bounds__(1024) void k_explicit_cell(VGrid g, VCoef c, VRK rk, ZMet zm, double betadx, int nlev,
+// Variant with one z plane per block (no z marching): every stencil operand
+// is read through L1/L2.  Fewer registers and LDS than the marching form;
+// the autotuner picks whichever is faster for the precision and grid.
+// ROWW = 32, 64: rows of that many lanes, solved within the wavefront (no
+// block barrier); 0: rows of several wavefronts.
+template <typename TW, typename TC, bool ZS, int ROWW>
+__global__ __launch_bounds__(512) void k_explicit_cell(VGrid g, const double *__restrict__ rowc,
+                                                   const double *__restrict__ pcrt, VRK rk, ZMet zm,
                                                    const double *__restrict__ q1, const double *__restrict__ q2,
                                                    const double *__restrict__ q3, const double *__restrict__ prg1,
                                                    const double *__restrict__ prg2, const double *__restrict__ prg3,
@@ -755,7 +721,10 @@ __global__ __launch_bounds__(1024) void k_explicit_cell(VGrid g, VCoef c, VRK rk
   const int j = bx * RJ + tj + 1;
   const int k = by + 1;
   const bool cell = (i <= g.nt) && (j <= g.nr);
-  const int jc = cell ? j : 1;  // coefficient row for idle threads
+  // the row's tables; a row of whole wavefronts is uniform in each of them
+  int jc = min(j, g.nr);
+  if (ROWW != 32) jc = __builtin_amdgcn_readfirstlane(jc);
+  const double *cf = rowc + (size_t)jc * kRowCoefs, *pr = pcrt + (size_t)jc * kPcrRow;
   TC v1 = (TC)0, v2 = (TC)0, v3 = (TC)0;
   if (cell) {
   const int ip = (i == g.nt) ? 1 : i + 1, im = (i == 1) ? g.nt : i - 1;
@@ -774,27 +743,27 @@ __global__ __launch_bounds__(1024) void k_explicit_cell(VGrid g, VCoef c, VRK rk
   // ---- q1 at (theta_c, r_m, z_m) ----
   {
     TC qnn = Q1(dip) + Q1(0), qss = Q1(dim) + Q1(0);
-    TC h11 = (qnn * qnn - qss * qss) * (TC)c.h1d11[j];
+    TC h11 = (qnn * qnn - qss * qss) * (TC)cf[0];
     qnn = (Q2(sj) + Q2(dim + sj)) * (Q1(sj) + Q1(0));
     qss = (Q1(0) + Q1(djm)) * (Q2(0) + Q2(dim));
-    TC h12d = (qnn - qss) * (TC)c.h1d22d[j];
+    TC h12d = (qnn - qss) * (TC)cf[1];
     qnn = (Q1(dip) + Q1(0)) * (Q2(sj) + Q2(0));
     qss = (Q1(0) + Q1(dim)) * (Q2(dim + sj) + Q2(dim));
-    TC h12n = (qnn + qss) * (TC)c.h1d22n[j];
+    TC h12n = (qnn + qss) * (TC)cf[2];
     qnn = (TC)0.25 * (Q3(sk) + Q3(dim + sk)) * (Q1(sk) + Q1(0));
     qss = (k == 1) ? (TC)0 : (TC)0.25 * (Q3(0) + Q3(dim)) * (Q1(0) + Q1(-sk));
     TC h13 = (qnn - qss) * zmk;
     qnn = Q2(sj) + Q2(0);
     qss = Q2(dim + sj) + Q2(dim);
-    TC d1q2 = (qnn - qss) * (TC)c.h1dare[j];
+    TC d1q2 = (qnn - qss) * (TC)cf[3];
     TC H1 = d1q2 - (h11 + (h12d + h12n) + h13);
-    TC d11 = (Q1(dip) - (TC)2 * Q1(0) + Q1(dim)) * (TC)c.s1t11[j];
+    TC d11 = (Q1(dip) - (TC)2 * Q1(0) + Q1(dim)) * (TC)cf[8];
     TC d33 = zs ? zd2c<TC>(zm, k, Q1(-sk), Q1(0), Q1(sk))
                 : (k == 1) ? (TC)(4.0 / 3.0) * (Q1(sk) - (TC)3 * Q1(0)) * dx3q
                            : (Q1(sk) - (TC)2 * Q1(0) + Q1(-sk)) * dx3q;
-    TC qn2 = (Q1(sj) / (TC)c.rm[j + 1] - Q1(0) / (TC)c.rm[j]) * (TC)c.s1t2n[j];
-    TC qs2 = (Q1(0) / (TC)c.rm[j] - Q1(djm) / (TC)c.rm[jm]) * (TC)c.s1t2s[j];
-    TC d22 = (qn2 - qs2) * (TC)c.s1t2c[j];
+    TC qn2 = (Q1(sj) * (TC)cf[18] - Q1(0) * (TC)cf[19]) * (TC)cf[9];
+    TC qs2 = (Q1(0) * (TC)cf[19] - Q1(djm) * (TC)cf[20]) * (TC)cf[10];
+    TC d22 = (qn2 - qs2) * (TC)cf[11];
     v1 = (ga * H1 + ro * (use_ru ? ru1[o] : (TC)0) - al * prg1[pc] + aRe * (d11 + d33 + d22)) * dt;
     ru1[o] = H1;
   }
@@ -802,10 +771,10 @@ __global__ __launch_bounds__(1024) void k_explicit_cell(VGrid g, VCoef c, VRK rk
   if (j >= 2) {
     TC qnn = (Q1(dip) + Q1(dip - sj)) * (Q2(dip) + Q2(0));
     TC qss = (Q1(0) + Q1(-sj)) * (Q2(0) + Q2(dim));
-    TC h21 = (qnn - qss) * (TC)c.h2d11[j];
+    TC h21 = (qnn - qss) * (TC)cf[4];
     qnn = Q2(sj) + Q2(0);
     qss = Q2(0) + Q2(-sj);
-    TC h22 = qnn * qnn * (TC)c.h2d22p[j] - qss * qss * (TC)c.h2d22m[j];
+    TC h22 = qnn * qnn * (TC)cf[5] - qss * qss * (TC)cf[6];
     qnn = (TC)0.5 * (Q1(0) + Q1(dip));
     qss = (TC)0.5 * (Q1(-sj) + Q1(dip - sj));
     TC h11n = (TC)0.25 * (qnn + qss) * (qnn + qss);
@@ -814,13 +783,13 @@ __global__ __launch_bounds__(1024) void k_explicit_cell(VGrid g, VCoef c, VRK rk
     TC h23 = (qnn - qss) * zmk;
     qnn = Q1(dip) + Q1(dip - sj);
     qss = Q1(0) + Q1(-sj);
-    TC d1q1 = -((qnn - qss) * (TC)c.h2dare[j]);
+    TC d1q1 = -((qnn - qss) * (TC)cf[7]);
     TC H2 = d1q1 - (h21 + h22 + h23 - h11n);
-    TC d11 = (Q2(dip) - (TC)2 * Q2(0) + Q2(dim)) * (TC)c.s2t11[j];
+    TC d11 = (Q2(dip) - (TC)2 * Q2(0) + Q2(dim)) * (TC)cf[12];
     TC d33 = zs ? zd2c<TC>(zm, k, Q2(-sk), Q2(0), Q2(sk))
                 : (k == 1) ? (TC)(4.0 / 3.0) * (Q2(sk) - (TC)3 * Q2(0)) * dx3q
                            : (Q2(sk) - (TC)2 * Q2(0) + Q2(-sk)) * dx3q;
-    TC d22 = Q2(sj) * (TC)c.s2t2p[j] - Q2(0) * (TC)c.s2t2c[j] + Q2(-sj) * (TC)c.s2t2m[j];
+    TC d22 = Q2(sj) * (TC)cf[13] - Q2(0) * (TC)cf[14] + Q2(-sj) * (TC)cf[15];
     v2 = (ga * H2 + ro * (use_ru ? ru2[o] : (TC)0) - al * prg2[pc] + aRe * (d11 + d33 + d22)) * dt;
     ru2[o] = H2;
   }
@@ -828,18 +797,18 @@ __global__ __launch_bounds__(1024) void k_explicit_cell(VGrid g, VCoef c, VRK rk
   if (k >= 2) {
     TC qnn = (Q3(sj) + Q3(0)) * (Q2(sj) + Q2(sj - sk));
     TC qss = (Q3(djm) + Q3(0)) * (Q2(0) + Q2(-sk));
-    TC h32 = (qnn - qss) * (TC)c.h1d22d[j];
+    TC h32 = (qnn - qss) * (TC)cf[1];
     qnn = (Q3(0) + Q3(dip)) * (Q1(dip) + Q1(dip - sk));
     qss = (Q3(dim) + Q3(0)) * (Q1(0) + Q1(-sk));
-    TC h31 = (qnn - qss) * (TC)c.h1d11[j];
+    TC h31 = (qnn - qss) * (TC)cf[0];
     qnn = (TC)0.25 * (Q3(0) + Q3(sk)) * (Q3(0) + Q3(sk));
     qss = (TC)0.25 * (Q3(0) + Q3(-sk)) * (Q3(0) + Q3(-sk));
     TC h33 = (qnn - qss) * zck;
     TC H3 = -(h31 + h32 + h33);
-    TC d11 = (Q3(dip) - (TC)2 * Q3(0) + Q3(dim)) * (TC)c.s1t11[j];
+    TC d11 = (Q3(dip) - (TC)2 * Q3(0) + Q3(dim)) * (TC)cf[8];
     TC d33 = zs ? zd2f<TC>(zm, k, Q3(-sk), Q3(0), Q3(sk)) : (Q3(sk) - (TC)2 * Q3(0) + Q3(-sk)) * dx3q;
-    TC qn2 = (Q3(sj) - Q3(0)) * (TC)c.s3t2n[j];
-    TC qs2 = (Q3(0) - Q3(djm)) * (TC)c.s3t2s[j];
+    TC qn2 = (Q3(sj) - Q3(0)) * (TC)cf[16];
+    TC qs2 = (Q3(0) - Q3(djm)) * (TC)cf[17];
     TC d22 = qn2 - qs2;
     v3 = (ga * H3 + ro * (use_ru ? ru3[o] : (TC)0) - al * prg3[pc] + aRe * (d11 + d33 + d22)) * dt;
     ru3[o] = H3;
@@ -855,39 +824,48 @@ __global__ __launch_bounds__(1024) void k_explicit_cell(VGrid g, VCoef c, VRK rk
   TC *f2 = f1 + (size_t)RJ * NTP;
   TC *f3 = f2 + (size_t)RJ * NTP;
   f1[ti] = v1; f2[ti] = v2; f3[ti] = v3;
-  double a1 = -(betadx * c.s1t11[jc]), b1 = 1.0 + 2.0 * (betadx * c.s1t11[jc]);
-  double a2 = -(betadx * c.s2t11[jc]), b2 = 1.0 + 2.0 * (betadx * c.s2t11[jc]);
-  const int N = g.nt;
-  const bool pow2 = N >= 2 && (N & (N - 1)) == 0;
-  __syncthreads();
-  // ping-pong buffers: one barrier per reduction level
+  const int N = g.nt, mylev = (int)pr[2];
+  int blev = mylev;  // the depth that the lanes which meet at the syncs share
+  if (ROWW == 0) {
+    for (int r = 0; r < RJ; r++) blev = max(blev, (int)pcrt[(size_t)min(bx * RJ + r + 1, g.nr) * kPcrRow + 2]);
+  } else if (ROWW == 32) {
+    blev = max(mylev, __shfl_xor(mylev, 32));
+  }
+  auto sync = [&]() {
+    if (ROWW == 0) {
+      __syncthreads();
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  };
+  sync();
+  // ping-pong buffers: one sync per reduction level
   const long S3 = 3L * RJ * NTP;
   int sm = 1 % N;
-  for (int lvl = 0; lvl < nlev; ++lvl) {
-    const double al1 = -a1 / b1, al2 = -a2 / b2;
+  for (int lvl = 0; lvl < blev; ++lvl) {
     TC n1 = v1, n2 = v2, n3 = v3;
-    if (ti < N) {
+    if (ti < N && lvl < mylev) {
+      const TC al1 = (TC)pr[kPcrHead + 2 * lvl], al2 = (TC)pr[kPcrHead + 2 * lvl + 1];
       int imv = ti - sm; if (imv < 0) imv += N;
       int ipv = ti + sm; if (ipv >= N) ipv -= N;
-      n1 = v1 + (TC)al1 * (f1[imv] + f1[ipv]);
-      n2 = v2 + (TC)al2 * (f2[imv] + f2[ipv]);
-      n3 = v3 + (TC)al1 * (f3[imv] + f3[ipv]);
+      n1 = v1 + al1 * (f1[imv] + f1[ipv]);
+      n2 = v2 + al2 * (f2[imv] + f2[ipv]);
+      n3 = v3 + al1 * (f3[imv] + f3[ipv]);
     }
-    b1 = b1 + 2.0 * al1 * a1; a1 = al1 * a1;
-    b2 = b2 + 2.0 * al2 * a2; a2 = al2 * a2;
     sm = (2 * sm) % N;
     const long flip = (lvl & 1) ? -S3 : S3;
     f1 += flip; f2 += flip; f3 += flip;
     f1[ti] = n1; f2[ti] = n2; f3[ti] = n3;
     v1 = n1; v2 = n2; v3 = n3;
-    __syncthreads();
+    sync();
   }
   if (!cell) return;
-  const double d1 = pow2 ? b1 + 2.0 * a1 : b1, d2 = pow2 ? b2 + 2.0 * a2 : b2;
+  const TC d1 = (TC)pr[0], d2 = (TC)pr[1];
   const long o = hidx(g, i, j, k);
-  r1[o] = (TC)(v1 / (TC)d1);
-  if (j >= 2) r2[o] = (TC)(v2 / (TC)d2);
-  if (k >= 2) r3[o] = (TC)(v3 / (TC)d1);
+  r1[o] = v1 * d1;
+  if (j >= 2) r2[o] = v2 * d2;
+  if (k >= 2) r3[o] = v3 * d1;
 }
 
 // ---------------------------------------------------------------------------
@@ -1959,36 +1937,59 @@ template <typename TW> void launch_explicit(vrh_t *h, int irk) {
   // compute type of the stencils: the work type (FP32 in the mixed path)
   using TC = TW;
   const VGrid &g = h->g;
-  int ntp = 1;
-  while (ntp < g.nt) ntp <<= 1;
-  if (ntp < 64) ntp = 64;
-  const double betadx = 0.5 * h->rk[irk].a * h->dt / h->Re;
+  const int ntp = (g.nt + 63) / 64 * 64;  // lanes of a theta row
   const int nlev = h->theta_levels[irk];
-  const int var = h->explicit_variant >= 0 ? h->explicit_variant : (sizeof(TW) == 8 ? 0 : 1);
+  const double *rowc = h->d_rowc, *pcrt = h->pcrt(irk);
+  // The default form (the tuner times all four).  us, the best chunk length of each:
+  //   FP64   64x128x256: plane 72, marching 98, wave 84; 128x256x512: 628, 459, 387;
+  //          256x128x256: 326, 268, 850 (its registers spill)
+  //   mixed  64x128x256: marching 53, wave 41; 128x256x512: 349, 295;
+  //          129x128x128: 68, 58 (four rows of 192 lanes); 256x128x256: 179, 193
+  // so rows of up to 64 lanes take the plane form in FP64 and the wave form in
+  // mixed, up to 128 the wave form, beyond the marching form, or in mixed up to
+  // 192 the wave form.  The mixed default leaves the plane form out: its
+  // contraction of q3's terms rounds differently from the others', which agree
+  // bit for bit.
+  const bool f64 = sizeof(TW) == 8;
+  const int var = h->explicit_variant >= 0 ? h->explicit_variant
+                  : g.nt <= 64             ? (f64 ? 0 : 2)
+                  : g.nt <= 128            ? 3
+                  : g.nt <= 192            ? (f64 ? 1 : 2)
+                                           : 1;
   KTimer kt(h, KT_EXPLICIT);
+#define EXPL_ARGS                                                                                                    \
+  h->f.q1, h->f.q2, h->f.q3, h->f.prg1, h->f.prg2, h->f.prg3, (TW *)h->f.ru1, (TW *)h->f.ru2, (TW *)h->f.ru3,        \
+      (TW *)h->f.r1, (TW *)h->f.r2, (TW *)h->f.r3
   if (var == 0) {
     // one z plane per block
-    int rj = 256 / ntp;
-    if (rj < 1) rj = 1;
-    dim3 blk(ntp, rj), grd((g.nr + rj - 1) / rj, g.nz);
-    const size_t sh = sizeof(TC) * 6 * (size_t)rj * ntp;
-    auto kern = h->zmet.m3 ? k_explicit_cell<TW, TC, true> : k_explicit_cell<TW, TC, false>;
-    hipLaunchKernelGGL(kern, grd, blk, sh, h->stream, g, h->coef, h->rk[irk], h->zmet, betadx, nlev,
-                       h->f.q1, h->f.q2, h->f.q3, h->f.prg1, h->f.prg2,
-                       h->f.prg3, (TW *)h->f.ru1, (TW *)h->f.ru2, (TW *)h->f.ru3, (TW *)h->f.r1,
-                       (TW *)h->f.r2, (TW *)h->f.r3);
+    const int roww = g.nt <= 32 ? 32 : g.nt <= 64 ? 64 : 0, rl = roww ? roww : ntp;
+    const int rj = rl <= 128 ? 256 / rl : 1;
+    dim3 blk(rl, rj), grd((g.nr + rj - 1) / rj, g.nz);
+    const size_t sh = sizeof(TC) * 6 * (size_t)rj * rl;
+    const bool zs = h->zmet.m3 != nullptr;
+    auto kern = roww == 32   ? (zs ? k_explicit_cell<TW, TC, true, 32> : k_explicit_cell<TW, TC, false, 32>)
+                : roww == 64 ? (zs ? k_explicit_cell<TW, TC, true, 64> : k_explicit_cell<TW, TC, false, 64>)
+                             : (zs ? k_explicit_cell<TW, TC, true, 0> : k_explicit_cell<TW, TC, false, 0>);
+    hipLaunchKernelGGL(kern, grd, blk, sh, h->stream, g, rowc, pcrt, h->rk[irk], h->zmet, EXPL_ARGS);
     return;
   }
+  // Planes per block: each block first loads three planes of its rows, so
+  // long chunks, as far as they leave four blocks per CU (us at 4, 8, 16, 32
+  // planes: mixed 33x96x200 31, 34, 44, 78; 128x96x256 65, 61, 76, 123;
+  // 128x256x512 310, 299, 295, 332; 256x512x1024 2939, 2642, 2483, 2428).
+  auto chunk = [&](int rows) {
+    const long rb = (g.nr + rows - 1) / rows;
+    int kc = 32;
+    while (kc > 4 && rb * ((g.nz + kc - 1) / kc) < 1024) kc /= 2;
+    return kc;
+  };
   // z marching: rows per block for 512 threads within 64 KB of LDS
-  auto lds = [&](int rj) {
-    return sizeof(double) * (size_t)rj * (kMaxPcrLevels * 2 + 2) +
+  auto lds = [&](int rj, int prow) {
+    return sizeof(double) * (size_t)rj * prow +
            sizeof(TC) * ((size_t)rj * kRowCoefs + (size_t)9 * (rj + 2) * ntp + (size_t)6 * rj * ntp);
   };
-  int rj = 512 / ntp;
-  if (rj < 1) rj = 1;
-  const int kchunk = 16;
-  // the wave form's PCR ratio table holds this substep's levels only
-  auto lds_w = [&](int rw) { return lds(rw) - sizeof(double) * (size_t)rw * 2 * (kMaxPcrLevels - nlev); };
+  // the wave form's ratio table holds this substep's levels only
+  auto lds_w = [&](int rw) { return lds(rw, kPcrHead + 2 * nlev); };
   if (var == 2 || var == 3) {
     // one wavefront per r row.  Form 2: the most rows (<= 8) whose LDS fits
     // 64 KB.  Form 3: among the instantiated row counts, the one that keeps
@@ -2000,12 +2001,12 @@ template <typename TW> void launch_explicit(vrh_t *h, int irk) {
     int rw = 8;
     size_t lim = 65536;
     if (var == 2) {
-      while (rw > 1 && lds(rw) > lim) rw--;
+      while (rw > 1 && lds(rw, kPcrRow) > lim) rw--;
     } else {
       lim = (size_t)h->lds_block;
-      const int cand1[] = {8, 6}, cand2[] = {6, 4, 2}, cand4[] = {2};
-      const int *cd = cpl == 1 ? cand1 : cpl == 2 ? cand2 : cand4;
-      const int ncd = cpl == 1 ? 2 : cpl == 2 ? 3 : 1;
+      const int cand1[] = {8, 6}, cand2[] = {6, 4, 2}, cand3[] = {4, 2}, cand4[] = {2};
+      const int *cd = cpl == 1 ? cand1 : cpl == 2 ? cand2 : cpl == 3 ? cand3 : cand4;
+      const int ncd = cpl == 1 ? 2 : cpl == 2 ? 3 : cpl == 3 ? 2 : 1;
       int best = 0;
       rw = 0;
       for (int i = 0; i < ncd; i++) {
@@ -2016,33 +2017,34 @@ template <typename TW> void launch_explicit(vrh_t *h, int irk) {
       }
       if (rw == 0) rw = 1;
     }
+    const int kchunk = chunk(rw);
     dim3 grd((g.nr + rw - 1) / rw, (g.nz + kchunk - 1) / kchunk);
-    bool done = rw > 1 && (var == 2 ? lds(rw) : lds_w(rw)) <= lim;
-#define EXPL_WAVE(C, R, W)                                                                                          \
+    bool done = rw > 1 && (var == 2 ? lds(rw, kPcrRow) : lds_w(rw)) <= lim;
+#define EXPL_WAVE(C, R, W)                                                                                            \
   hipLaunchKernelGGL((h->zmet.m3 ? k_explicit_wave<TW, TC, C, R, W, true> : k_explicit_wave<TW, TC, C, R, W, false>), \
-                     grd, dim3(64, R), lds_w(R), h->stream, g, h->coef, h->rk[irk],                                     \
-                     h->zmet, betadx, nlev, kchunk, h->f.q1, h->f.q2, h->f.q3, h->f.prg1, h->f.prg2, \
-                     h->f.prg3, (TW *)h->f.ru1, (TW *)h->f.ru2, (TW *)h->f.ru3, (TW *)h->f.r1,          \
-                     (TW *)h->f.r2, (TW *)h->f.r3)
+                     grd, dim3(64, R), lds_w(R), h->stream, g, rowc, pcrt, h->rk[irk], h->zmet, nlev, kchunk, EXPL_ARGS)
     if (done) {
       if (cpl == 1 && rw == 8) EXPL_WAVE(1, 8, 4);
       else if (cpl == 1 && rw == 6) EXPL_WAVE(1, 6, 3);
       else if (cpl == 2 && rw == 6) EXPL_WAVE(2, 6, 3);
       else if (cpl == 2 && rw == 4) EXPL_WAVE(2, 4, 2);
       else if (cpl == 2 && rw == 2) EXPL_WAVE(2, 2, 2);
+      else if (cpl == 3 && rw == 4) EXPL_WAVE(3, 4, 2);
+      else if (cpl == 3 && rw == 2) EXPL_WAVE(3, 2, 2);
       else if (cpl == 4 && rw == 2) EXPL_WAVE(4, 2, 2);
       else done = false;
     }
 #undef EXPL_WAVE
     if (done) return;
   }
-  while (rj > 1 && lds(rj) > 65536) rj--;
+  int rj = 512 / ntp;
+  if (rj < 1) rj = 1;
+  while (rj > 1 && lds(rj, kPcrRow) > 65536) rj--;
+  const int kchunk = chunk(rj);
   dim3 blk(ntp, rj), grd((g.nr + rj - 1) / rj, (g.nz + kchunk - 1) / kchunk);
   auto kern = h->zmet.m3 ? k_explicit_march<TW, TC, true> : k_explicit_march<TW, TC, false>;
-  hipLaunchKernelGGL(kern, grd, blk, lds(rj), h->stream, g, h->coef, h->rk[irk], h->zmet, betadx, nlev,
-                     kchunk, h->f.q1, h->f.q2, h->f.q3, h->f.prg1, h->f.prg2,
-                     h->f.prg3, (TW *)h->f.ru1, (TW *)h->f.ru2, (TW *)h->f.ru3, (TW *)h->f.r1,
-                     (TW *)h->f.r2, (TW *)h->f.r3);
+  hipLaunchKernelGGL(kern, grd, blk, lds(rj, kPcrRow), h->stream, g, rowc, pcrt, h->rk[irk], h->zmet, kchunk, EXPL_ARGS);
+#undef EXPL_ARGS
 }
 
 // Blocks of the explicit kernel's one-wave-per-row form and tuned z-DCT
@@ -2064,24 +2066,32 @@ void lds_optin(vrh_t *h) {
         reinterpret_cast<const void *>(&k_explicit_wave<double, double, 2, 6, 3, false>),
         reinterpret_cast<const void *>(&k_explicit_wave<double, double, 2, 4, 2, false>),
         reinterpret_cast<const void *>(&k_explicit_wave<double, double, 2, 2, 2, false>),
+        reinterpret_cast<const void *>(&k_explicit_wave<double, double, 3, 4, 2, false>),
+        reinterpret_cast<const void *>(&k_explicit_wave<double, double, 3, 2, 2, false>),
         reinterpret_cast<const void *>(&k_explicit_wave<double, double, 4, 2, 2, false>),
         reinterpret_cast<const void *>(&k_explicit_wave<float, float, 1, 8, 4, false>),
         reinterpret_cast<const void *>(&k_explicit_wave<float, float, 1, 6, 3, false>),
         reinterpret_cast<const void *>(&k_explicit_wave<float, float, 2, 6, 3, false>),
         reinterpret_cast<const void *>(&k_explicit_wave<float, float, 2, 4, 2, false>),
         reinterpret_cast<const void *>(&k_explicit_wave<float, float, 2, 2, 2, false>),
+        reinterpret_cast<const void *>(&k_explicit_wave<float, float, 3, 4, 2, false>),
+        reinterpret_cast<const void *>(&k_explicit_wave<float, float, 3, 2, 2, false>),
         reinterpret_cast<const void *>(&k_explicit_wave<float, float, 4, 2, 2, false>),
         reinterpret_cast<const void *>(&k_explicit_wave<double, double, 1, 8, 4, true>),
         reinterpret_cast<const void *>(&k_explicit_wave<double, double, 1, 6, 3, true>),
         reinterpret_cast<const void *>(&k_explicit_wave<double, double, 2, 6, 3, true>),
         reinterpret_cast<const void *>(&k_explicit_wave<double, double, 2, 4, 2, true>),
         reinterpret_cast<const void *>(&k_explicit_wave<double, double, 2, 2, 2, true>),
+        reinterpret_cast<const void *>(&k_explicit_wave<double, double, 3, 4, 2, true>),
+        reinterpret_cast<const void *>(&k_explicit_wave<double, double, 3, 2, 2, true>),
         reinterpret_cast<const void *>(&k_explicit_wave<double, double, 4, 2, 2, true>),
         reinterpret_cast<const void *>(&k_explicit_wave<float, float, 1, 8, 4, true>),
         reinterpret_cast<const void *>(&k_explicit_wave<float, float, 1, 6, 3, true>),
         reinterpret_cast<const void *>(&k_explicit_wave<float, float, 2, 6, 3, true>),
         reinterpret_cast<const void *>(&k_explicit_wave<float, float, 2, 4, 2, true>),
         reinterpret_cast<const void *>(&k_explicit_wave<float, float, 2, 2, 2, true>),
+        reinterpret_cast<const void *>(&k_explicit_wave<float, float, 3, 4, 2, true>),
+        reinterpret_cast<const void *>(&k_explicit_wave<float, float, 3, 2, 2, true>),
         reinterpret_cast<const void *>(&k_explicit_wave<float, float, 4, 2, 2, true>),
         reinterpret_cast<const void *>(&k_dctz<float>),
         reinterpret_cast<const void *>(&k_dctz<double>)};
