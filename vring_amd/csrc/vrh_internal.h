@@ -66,6 +66,17 @@ struct LineCoef {
   int n, P;
 };
 
+// Work-group order across the eight XCDs: the dispatcher hands work group p
+// (linear id) to XCD p mod 8, and each XCD has its own L2.  xcd_tile maps p
+// to a logical tile so that XCD x runs one contiguous range of tiles, in
+// order, one dispatch round apart: neighbouring tiles meet in one L2.  A
+// bijection on [0, nblk) for any nblk.
+__device__ __forceinline__ long xcd_tile(long b, long nblk) {
+  constexpr long kX = 8;
+  const long q = nblk / kX, rem = nblk % kX, x = b % kX, r = b / kX;
+  return x < rem ? x * (q + 1) + r : rem * (q + 1) + (x - rem) * q + r;
+}
+
 // Tables of the explicit kernels (explicit_tables), one row per r index j =
 // 0..nr: kRowCoefs metric coefficients (cf[...] in the kernels), and per
 // substep kPcrRow numbers of the theta solves: the factors 1/diagonal of the

@@ -17,16 +17,6 @@ namespace {
 
 template <typename T> __device__ __forceinline__ T ldg(const T *p) { return __builtin_nontemporal_load(p); }
 
-// Work-group order across the eight XCDs: the dispatcher hands work group p
-// (linear id) to XCD p mod 8, and each XCD has its own L2.  xcd_tile maps p
-// to a logical tile so that XCD x runs one contiguous range of tiles, in
-// order, one dispatch round apart: neighbouring tiles meet in one L2.  A
-// bijection on [0, nblk) for any nblk.
-__device__ __forceinline__ long xcd_tile(long b, long nblk) {
-  constexpr long kX = 8;
-  const long q = nblk / kX, rem = nblk % kX, x = b % kX, r = b / kX;
-  return x < rem ? x * (q + 1) + r : rem * (q + 1) + (x - rem) * q + r;
-}
 // The block's logical (x, y, z) coordinates of a 2-D or 3-D grid in the
 // order of xcd_tile, x fastest: tiles adjacent in x (whose halo rows
 // overlap) share an L2.

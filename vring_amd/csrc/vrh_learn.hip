@@ -18,7 +18,7 @@
 #include <string>
 #include <vector>
 
-#include "vrh_learn.h"
+#include "vrh_internal.h"
 
 namespace {
 
@@ -47,27 +47,39 @@ __device__ __forceinline__ float bf2f(bf16_t h) { return __uint_as_float(((unsig
 struct Geo {
   int nr, nz, S;
   double dr;
-  const double *rm, *rf, *dz, *izm;  // rf: nr+1 face factors rface/dr (0 at both ends); izm: nz+1 (0 at ends)
+  // rf: nr+1 face factors rface/dr (0 at both ends); izm: nz+1 (0 at ends);
+  // drm: dr/rm; rv: rm dr
+  const double *rm, *rf, *dz, *izm, *drm, *rv;
   const int *m;
 };
 
-__device__ __forceinline__ double vol(const Geo &g, int k, int j) { return g.dz[k] * (g.rm[j] * g.dr); }
+__device__ __forceinline__ double vol(const Geo &g, int k, int j) { return g.dz[k] * g.rv[j]; }
+// diagonal and rows of S, the fused operations written out so that every
+// kernel rounds alike
 __device__ __forceinline__ double sdiag(const Geo &g, int b, int k, int j) {
+#pragma clang fp contract(off)
   const double mm = (double)g.m[b] * (double)g.m[b];
-  return mm * (g.dz[k] * (g.dr / g.rm[j])) + g.dz[k] * (g.rf[j] + g.rf[j + 1]) +
-         (g.rm[j] * g.dr) * (g.izm[k] + g.izm[k + 1]);
+  return __builtin_fma(g.rv[j], g.izm[k] + g.izm[k + 1],
+                       __builtin_fma(mm, g.dz[k] * g.drm[j], g.dz[k] * (g.rf[j] + g.rf[j + 1])));
+}
+// the same diagonal as the initial residual's kernel rounds it
+__device__ __forceinline__ double sdiag0(const Geo &g, int b, int k, int j) {
+#pragma clang fp contract(off)
+  const double mm = (double)g.m[b] * (double)g.m[b];
+  return __builtin_fma(g.rv[j], g.izm[k] + g.izm[k + 1],
+                       __builtin_fma(g.dz[k], g.rf[j] + g.rf[j + 1], mm * (g.dz[k] * g.drm[j])));
 }
 // (S x)(c) with neighbours read through `at`
 template <typename F>
 __device__ __forceinline__ double sapply(const Geo &g, int b, int k, int j, F at) {
+#pragma clang fp contract(off)
   const double xc = at(k, j);
   const double mm = (double)g.m[b] * (double)g.m[b];
-  double y = mm * (g.dz[k] * (g.dr / g.rm[j])) * xc;
-  if (j > 0) y += g.dz[k] * g.rf[j] * (xc - at(k, j - 1));
-  if (j < g.nr - 1) y += g.dz[k] * g.rf[j + 1] * (xc - at(k, j + 1));
-  const double rv = g.rm[j] * g.dr;
-  if (k > 0) y += rv * g.izm[k] * (xc - at(k - 1, j));
-  if (k < g.nz - 1) y += rv * g.izm[k + 1] * (xc - at(k + 1, j));
+  double y = mm * (g.dz[k] * g.drm[j]) * xc;
+  if (j > 0) y = __builtin_fma(g.dz[k] * g.rf[j], xc - at(k, j - 1), y);
+  if (j < g.nr - 1) y = __builtin_fma(g.dz[k] * g.rf[j + 1], xc - at(k, j + 1), y);
+  if (k > 0) y = __builtin_fma(g.rv[j] * g.izm[k], xc - at(k - 1, j), y);
+  if (k < g.nz - 1) y = __builtin_fma(g.rv[j] * g.izm[k + 1], xc - at(k + 1, j), y);
   return y;
 }
 
@@ -79,9 +91,9 @@ __device__ __forceinline__ double psum(const double *part, int nq, int b, int q)
   return s;
 }
 
-// Block reduction of NQ values; thread 0 writes partials.
+// Block reduction of NQ values; thread 0 writes the partials of block bx.
 template <int NQ>
-__device__ __forceinline__ void block_partials(double (&v)[NQ], double *part, int nq, int b) {
+__device__ __forceinline__ void block_partials(double (&v)[NQ], double *part, int nq, int b, int bx) {
   __shared__ double red[NQ][256 / 64];
   for (int q = 0; q < NQ; q++) {
     double x = v[q];
@@ -91,16 +103,35 @@ __device__ __forceinline__ void block_partials(double (&v)[NQ], double *part, in
   __syncthreads();
   if (threadIdx.x == 0)
     for (int q = 0; q < NQ; q++)
-      part[((long)b * kRedBlocks + blockIdx.x) * nq + q] = red[q][0] + red[q][1] + red[q][2] + red[q][3];
+      part[((long)b * kRedBlocks + bx) * nq + q] = red[q][0] + red[q][1] + red[q][2] + red[q][3];
+}
+template <int NQ> __device__ __forceinline__ void block_partials(double (&v)[NQ], double *part, int nq, int b) {
+  block_partials<NQ>(v, part, nq, b, (int)blockIdx.x);
 }
 
+// The cells of one thread of block bx: bx 256 + thread, then every
+// kRedBlocks 256-th; (k, j) advance with the cell, one division per thread.
+struct CellIt {
+  int i, k, j, n, nr, dk, dj;
+  __device__ __forceinline__ CellIt(const Geo &g, int bx) {
+    n = g.nz * g.nr; nr = g.nr;
+    i = bx * 256 + (int)threadIdx.x;
+    k = i / nr; j = i - k * nr;
+    dk = 256 * kRedBlocks / nr; dj = 256 * kRedBlocks - dk * nr;
+  }
+  __device__ __forceinline__ bool in() const { return i < n; }
+  __device__ __forceinline__ void next() {
+    i += 256 * kRedBlocks; k += dk; j += dj;
+    if (j >= nr) { j -= nr; k++; }
+  }
+};
 // grid (kRedBlocks, S), 256 threads: cell loop of slot b
 #define CELL_LOOP(g, b, c, k, j)                                                   \
   const long ncs = (long)(g).nz * (g).nr;                                          \
-  for (long c_ = (long)blockIdx.x * 256 + threadIdx.x; c_ < ncs; c_ += 256L * kRedBlocks) \
+  for (CellIt it_((g), (int)blockIdx.x); it_.in(); it_.next())                     \
     for (int once_ = 1; once_; once_ = 0)                                          \
-      for (const long c = (long)(b) * ncs + c_; once_; once_ = 0)                  \
-        for (const int k = (int)(c_ / (g).nr), j = (int)(c_ - (long)k * (g).nr); once_; once_ = 0)
+      for (const long c = (long)(b) * ncs + it_.i; once_; once_ = 0)               \
+        for (const int k = it_.k, j = it_.j; once_; once_ = 0)
 
 // ---------------------------------------------------------------------------
 // elementary kernels
@@ -164,76 +195,225 @@ __global__ void k_resid(Geo g, const double *__restrict__ rhs, const double *__r
 // Jacobi-preconditioned CG (textbook form), all slots together; per-slot
 // scalars live on the device, each kernel sums the partials it needs.
 // ---------------------------------------------------------------------------
-// r = b - S x, z = D^-1 r, p = z; partials (r.z, r.r, b.b)
+// r = b - S x, z = D^-1 r; partials (r.z, r.r, b.b)
 __global__ void k_cg_init(Geo g, const double *__restrict__ rhs, const double *__restrict__ x, double *__restrict__ r,
-                          double *__restrict__ z, double *__restrict__ p, double *part) {
+                          double *__restrict__ z, double *part) {
   const int b = blockIdx.y;
   double v[3] = {0.0, 0.0, 0.0};
   CELL_LOOP(g, b, c, k, j) {
     const double *xb = x + (long)b * ncs;
     const double rr = rhs[c] - sapply(g, b, k, j, [&](int kk, int jj) { return xb[(long)kk * g.nr + jj]; });
-    const double zz = rr / sdiag(g, b, k, j);
-    r[c] = rr; z[c] = zz; p[c] = zz;
+    const double zz = rr / sdiag0(g, b, k, j);
+    r[c] = rr; z[c] = zz;
     v[0] += rr * zz; v[1] += rr * rr; v[2] += rhs[c] * rhs[c];
   }
   block_partials<3>(v, part, 3, b);
 }
-__global__ void k_cg_start(int S, const double *part, double *sc, double tol2) {
+// Scalars of a slot's iteration, kept twice: a kernel reads one set while its
+// first block writes the other.
+struct CgSc { double rz, bb, done, it; };
+
+__global__ void k_cg_start(int S, const double *part, CgSc *sc, double tol2) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= S) return;
-  sc[b * kNsc + SC_RZ] = psum(part, 3, b, 0);
-  sc[b * kNsc + SC_BB] = psum(part, 3, b, 2);
-  sc[b * kNsc + SC_DONE] = (psum(part, 3, b, 1) <= tol2 * sc[b * kNsc + SC_BB]) ? 1.0 : 0.0;
-  sc[b * kNsc + SC_IT] = 0.0;
+  const double bb = psum(part, 3, b, 2);
+  sc[b] = CgSc{psum(part, 3, b, 0), bb, (psum(part, 3, b, 1) <= tol2 * bb) ? 1.0 : 0.0, 0.0};
 }
-// after an update: r.z of the new residual, iteration count, done flag
-__global__ void k_cg_fold(int S, const double *part_rz, double *sc, double tol2) {
+// the scalars after an update: r.z of the new residual, iteration count, done flag
+__device__ __forceinline__ CgSc cg_fold(const CgSc &o, const double *part_rz, int b, double tol2) {
+  if (o.done != 0.0) return o;
+  return CgSc{psum(part_rz, 2, b, 0), o.bb, psum(part_rz, 2, b, 1) <= tol2 * o.bb ? 1.0 : 0.0, o.it + 1.0};
+}
+__global__ void k_cg_end(int S, const double *part_rz, const CgSc *sc, double *out, double tol2, int fold) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= S) return;
-  double *s = sc + b * kNsc;
-  if (s[SC_DONE] != 0.0) return;
-  s[SC_RZ] = psum(part_rz, 3, b, 0);
-  s[SC_IT] += 1.0;
-  if (psum(part_rz, 3, b, 1) <= tol2 * s[SC_BB]) s[SC_DONE] = 1.0;
+  const CgSc s = fold ? cg_fold(sc[b], part_rz, b, tol2) : sc[b];
+  double *o = out + b * kNsc;
+  o[SC_RZ] = s.rz; o[SC_BB] = s.bb; o[SC_DONE] = s.done; o[SC_IT] = s.it;
 }
-// q = S p; partial p.q
-__global__ void k_cg_q(Geo g, const double *__restrict__ p, double *__restrict__ q, double *part_pq) {
-  const int b = blockIdx.y;
+
+// An iteration is two kernels, each a pass over its slot's cells; nothing but
+// p, x, r and z passes through memory.
+//   direction: p = z + beta p (beta = (r.z)_new / (r.z)_old; p = z at first)
+//     formed at the cell and its neighbours from the old p, so that S p and
+//     the partial p.Sp come in the same pass;
+//   update: S p again from p, x += a p, r -= a S p, z = D^-1 r; partials
+//     (r.z, r.r).
+// The partial sums are those of 64 blocks of 256 threads, thread t of block bx
+// adding the cells bx 256 + t + 16384 i in order of i.  A block here has four
+// times the threads, each pass over eight i's: every thread forms two cells,
+// and the first 256 add the products from LDS in that order (a solve's last
+// thousand iterations have few slots left, and a thread that walked its eight
+// cells alone waited for each in turn).  Only the slots of the list `act` run.
+// Work group p goes to XCD p mod 8, which takes the blocks bx = 8 (p mod 8) ..
+// + 7 of every slot: neighbouring rows meet in one L2 and any number of slots
+// loads the XCDs evenly.
+// 64 slots of 256x512 to 1e-8 (2302 iterations, 11 slots on average): 95 ms, 260
+// with S p, update and direction as kernels of their own (12 passes instead of
+// 9) over all slots.  A kernel takes 95 us with all 64 slots (62 at the copy
+// rate; bound by the latencies of a block's phases, two blocks to a CU) and 10
+// with one or two (launch and those latencies).
+struct CgBlock {
+  int b, bx, n;
+  __device__ __forceinline__ CgBlock(const Geo &g, const int *act) {
+    const int p = (int)blockIdx.x, x = p & 7, r = p >> 3;
+    b = act[r >> 3];
+    bx = 8 * x + (r & 7);
+    n = g.nz * g.nr;
+  }
+};
+static_assert(kRedBlocks == 64, "CgBlock deals 8 x 8 blocks of a slot");
+// A cell and its four neighbours (itself where there is none: its coefficient
+// is zero there)
+struct CgNb {
+  int c, l, r, d, u, k, j;
+  __device__ __forceinline__ CgNb(const Geo &g, int cell) {
+    c = cell; k = c / g.nr; j = c - k * g.nr;
+    l = j > 0 ? c - 1 : c; r = j < g.nr - 1 ? c + 1 : c;
+    d = k > 0 ? c - g.nr : c; u = k < g.nz - 1 ? c + g.nr : c;
+  }
+};
+// sapply on values at hand (the terms that sapply leaves out have zero factors here)
+__device__ __forceinline__ double cg_row(const Geo &g, double mm, const CgNb &n, double xc, double xl, double xr, double xd,
+                                         double xu) {
+#pragma clang fp contract(off)
+  const double dz = g.dz[n.k], rv = g.rv[n.j];
+  double y = mm * (dz * g.drm[n.j]) * xc;
+  y = __builtin_fma(dz * g.rf[n.j], xc - xl, y);
+  y = __builtin_fma(dz * g.rf[n.j + 1], xc - xr, y);
+  y = __builtin_fma(rv * g.izm[n.k], xc - xd, y);
+  return __builtin_fma(rv * g.izm[n.k + 1], xc - xu, y);
+}
+// Cells of a block, eight per thread of the first 256 at a time: `load` fetches
+// what a cell needs (called before `scal`, which the first wave runs alone,
+// so that the loads are under way meanwhile), `form` gives the products u v
+// to add (with SQ, u u too).
+template <bool SQ, typename V, typename LOAD, typename SCAL, typename FORM>
+__device__ __forceinline__ void cg_cells(const CgBlock &q, double (&v)[SQ ? 2 : 1], LOAD load, SCAL scal, FORM form) {
+  __shared__ double lu[8][256], lv[8][256];
+  const int t = threadIdx.x & 255, sub = threadIdx.x >> 8;
+  constexpr int kStride = 256 * kRedBlocks;
+  bool have = false;
+  for (int c0 = q.bx * 256; c0 < q.n; c0 += 8 * kStride) {
+    V raw[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) raw[h] = load(min(c0 + t + (sub + 4 * h) * kStride, q.n - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    if (!have) {
+      if (threadIdx.x < 64) scal();
+      __syncthreads();
+      have = true;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const int i = sub + 4 * h, c = c0 + t + i * kStride;
+      double u = 0.0, w = 0.0;
+      if (c < q.n) form(c, raw[h], u, w);
+      lu[i][t] = u;
+      lv[i][t] = w;
+    }
+    __syncthreads();
+    if (sub == 0) {
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const double u = lu[i][t];
+        v[0] = __builtin_fma(u, lv[i][t], v[0]);
+        if (SQ) v[SQ ? 1 : 0] = __builtin_fma(u, u, v[SQ ? 1 : 0]);
+      }
+    }
+    __syncthreads();
+  }
+}
+// block_partials of the first 256 threads
+template <int NQ> __device__ __forceinline__ void cg_partials(double (&v)[NQ], double *part, const CgBlock &q) {
+  __shared__ double red[NQ][4];
+  if (threadIdx.x < 256) {
+#pragma unroll
+    for (int n = 0; n < NQ; n++) {
+      double x = v[n];
+      for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+      if ((threadIdx.x & 63) == 0) red[n][threadIdx.x >> 6] = x;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < NQ) {
+    const double *r = red[threadIdx.x];
+    part[((long)q.b * kRedBlocks + q.bx) * NQ + threadIdx.x] = r[0] + r[1] + r[2] + r[3];
+  }
+}
+struct CgV5 { double c, l, r, d, u; };
+__device__ __forceinline__ CgV5 cg_load5(const double *__restrict__ x, const CgNb &n) {
+  return CgV5{x[n.c], x[n.l], x[n.r], x[n.d], x[n.u]};
+}
+__global__ __launch_bounds__(1024, 8) void k_cg_direction(Geo g, const int *__restrict__ act, const double *__restrict__ z,
+                                                          const double *__restrict__ po, double *__restrict__ pn,
+                                                          const double *__restrict__ part_rz,
+                                                          double *__restrict__ part_pq, const CgSc *__restrict__ sc,
+                                                          CgSc *__restrict__ scn, double tol2, int first) {
+  __shared__ double sh[2];
+  const CgBlock q(g, act);
+  const CgSc o = sc[q.b];
+  if (o.done != 0.0) {
+    if (q.bx == 0 && threadIdx.x == 0) scn[q.b] = o;
+    return;
+  }
+  const long base = (long)q.b * q.n;
+  const double *zb = z + base, *pb = first ? zb : po + base;
+  const double mm = (double)g.m[q.b] * (double)g.m[q.b];
   double v[1] = {0.0};
-  CELL_LOOP(g, b, c, k, j) {
-    const double *pb = p + (long)b * ncs;
-    const double y = sapply(g, b, k, j, [&](int kk, int jj) { return pb[(long)kk * g.nr + jj]; });
-    q[c] = y;
-    v[0] += p[c] * y;
-  }
-  block_partials<1>(v, part_pq, 1, b);
+  struct V { CgV5 z, p; };
+  cg_cells<false, V>(
+      q, v,
+      [&](int c) {
+        const CgNb n(g, c);
+        return V{cg_load5(zb, n), cg_load5(pb, n)};
+      },
+      [&]() {
+        const CgSc s = first ? o : cg_fold(o, part_rz, q.b, tol2);
+        if (threadIdx.x == 0) {
+          if (q.bx == 0) scn[q.b] = s;
+          sh[0] = first ? 0.0 : s.rz / o.rz;
+        }
+      },
+      [&](int c, const V &w, double &p, double &y) {
+        // p = z at first: beta = 0 (and the old p read is z itself)
+        const double be = sh[0];
+        p = __builtin_fma(be, w.p.c, w.z.c);
+        y = cg_row(g, mm, CgNb(g, c), p, __builtin_fma(be, w.p.l, w.z.l), __builtin_fma(be, w.p.r, w.z.r),
+                   __builtin_fma(be, w.p.d, w.z.d), __builtin_fma(be, w.p.u, w.z.u));
+        pn[base + c] = p;
+      });
+  cg_partials<1>(v, part_pq, q);
 }
-// x += a p, r -= a q, z = D^-1 r; partials (r.z, r.r, 0)
-__global__ void k_cg_update(Geo g, double *__restrict__ x, double *__restrict__ r, double *__restrict__ z,
-                            const double *__restrict__ p, const double *__restrict__ q, const double *part_pq,
-                            double *part_rz, const double *sc) {
-  const int b = blockIdx.y;
-  const double *s = sc + b * kNsc;
-  const bool done = s[SC_DONE] != 0.0;
-  const double pq = psum(part_pq, 1, b, 0);
-  const double a = (done || pq == 0.0) ? 0.0 : s[SC_RZ] / pq;
-  double v[3] = {0.0, 0.0, 0.0};
-  CELL_LOOP(g, b, c, k, j) {
-    const double rr = r[c] - a * q[c];
-    const double zz = rr / sdiag(g, b, k, j);
-    if (!done) { x[c] += a * p[c]; r[c] = rr; z[c] = zz; }
-    v[0] += rr * zz; v[1] += rr * rr;
-  }
-  block_partials<3>(v, part_rz, 3, b);
-}
-// p = z + beta p with beta = (r.z)_new / (r.z)_old (the scalars still hold the old value)
-__global__ void k_cg_dir(Geo g, const double *__restrict__ z, double *__restrict__ p, const double *part_rz,
-                         const double *sc) {
-  const int b = blockIdx.y;
-  const double *s = sc + b * kNsc;
-  if (s[SC_DONE] != 0.0) return;
-  const double beta = psum(part_rz, 3, b, 0) / s[SC_RZ];
-  CELL_LOOP(g, b, c, k, j) { p[c] = z[c] + beta * p[c]; }
+__global__ __launch_bounds__(1024, 8) void k_cg_update(Geo g, const int *__restrict__ act, double *__restrict__ x,
+                                                       double *__restrict__ r, double *__restrict__ z,
+                                                       const double *__restrict__ p, const double *__restrict__ part_pq,
+                                                       double *__restrict__ part_rz, const CgSc *__restrict__ sc) {
+  __shared__ double sh[1];
+  const CgBlock q(g, act);
+  const CgSc s = sc[q.b];
+  if (s.done != 0.0) return;
+  const long base = (long)q.b * q.n;
+  const double *pb = p + base;
+  const double mm = (double)g.m[q.b] * (double)g.m[q.b];
+  double v[2] = {0.0, 0.0};
+  struct V { CgV5 p; double x, r; };
+  cg_cells<true, V>(
+      q, v, [&](int c) { return V{cg_load5(pb, CgNb(g, c)), x[base + c], r[base + c]}; },
+      [&]() {
+        const double pq = psum(part_pq, 1, q.b, 0);
+        if (threadIdx.x == 0) sh[0] = pq == 0.0 ? 0.0 : s.rz / pq;
+      },
+      [&](int c, const V &w, double &rr, double &zz) {
+        const double a = sh[0];
+        const CgNb n(g, c);
+        rr = __builtin_fma(-a, cg_row(g, mm, n, w.p.c, w.p.l, w.p.r, w.p.d, w.p.u), w.r);
+        zz = rr / sdiag(g, q.b, n.k, n.j);
+        x[base + c] = __builtin_fma(a, w.p.c, w.x);
+        r[base + c] = rr;
+        z[base + c] = zz;
+      });
+  cg_partials<2>(v, part_rz, q);
 }
 
 // ---------------------------------------------------------------------------
@@ -905,7 +1085,7 @@ struct vrh_hz_s {
   std::vector<double> zf, zm, dz, rm;
   std::vector<int> hm;
   // geometry
-  double *d_rm = nullptr, *d_rf = nullptr, *d_dz = nullptr, *d_izm = nullptr, *d_zm = nullptr;
+  double *d_rm = nullptr, *d_rf = nullptr, *d_dz = nullptr, *d_izm = nullptr, *d_zm = nullptr, *d_drm = nullptr, *d_rv = nullptr;
   int *d_m = nullptr;
   // direct solve: V (column q = z eigenvector, W-orthonormal), eigenvalues
   double *d_V = nullptr, *d_lam = nullptr;
@@ -923,7 +1103,7 @@ struct vrh_hz_s {
   Geo geo() const {
     Geo g;
     g.nr = nr; g.nz = nz; g.S = S; g.dr = dr;
-    g.rm = d_rm; g.rf = d_rf; g.dz = d_dz; g.izm = d_izm; g.m = d_m;
+    g.rm = d_rm; g.rf = d_rf; g.dz = d_dz; g.izm = d_izm; g.m = d_m; g.drm = d_drm; g.rv = d_rv;
     return g;
   }
   size_t ncell() const { return (size_t)S * nz * nr; }
@@ -1088,34 +1268,54 @@ int sync_scalars(vrh_hz_t *h, std::vector<double> &sc) {
   return 0;
 }
 
-// PCG from x (device arrays rhs, x); returns iterations per slot in its
+// PCG from x (device arrays rhs, x); returns iterations per slot in its.  The
+// done flags are looked at every 32 iterations, one iteration behind (a
+// converged slot's blocks return at once), and the converged slots leave the
+// list.  The last residual stays in vec[2].
 int pcg_dev(vrh_hz_t *h, const double *rhs, double *x, double tol, int maxit, std::vector<int> &its) {
   Geo g = h->geo();
-  double *r = h->vec[2], *z = h->vec[3], *p = h->vec[4], *q = h->vec[5];
-  double *part_rz = h->d_part, *part_pq = h->d_part + (size_t)h->S * kRedBlocks * 4;
+  const int S = h->S;
+  double *r = h->vec[2], *z = h->vec[3], *p[2] = {h->vec[4], h->vec[5]};
+  const size_t np = (size_t)S * kRedBlocks;
+  double *part0 = h->d_part, *part_pq = h->d_part + np * 4, *part_rz = h->d_part + np * 12;
+  // scalars and slot list in the partials' spare room
+  CgSc *cg[2] = {reinterpret_cast<CgSc *>(h->d_part + np * 8), reinterpret_cast<CgSc *>(h->d_part + np * 8) + S};
+  int *act = reinterpret_cast<int *>(cg[1] + S);
   const double tol2 = tol * tol;
-  const dim3 sg((h->S + 63) / 64), sb(64);
-  hipLaunchKernelGGL(k_cg_init, red_grid(h), dim3(256), 0, h->stream, g, rhs, x, r, z, p, part_rz);
-  hipLaunchKernelGGL(k_cg_start, sg, sb, 0, h->stream, h->S, part_rz, h->d_sc, tol2);
-  std::vector<double> sc;
-  for (int it = 0; it < maxit; it++) {
-    hipLaunchKernelGGL(k_cg_q, red_grid(h), dim3(256), 0, h->stream, g, p, q, part_pq);
-    hipLaunchKernelGGL(k_cg_update, red_grid(h), dim3(256), 0, h->stream, g, x, r, z, p, q, part_pq, part_rz,
-                       h->d_sc);
-    hipLaunchKernelGGL(k_cg_dir, red_grid(h), dim3(256), 0, h->stream, g, z, p, part_rz, h->d_sc);
-    hipLaunchKernelGGL(k_cg_fold, sg, sb, 0, h->stream, h->S, part_rz, h->d_sc, tol2);
-    if ((it & 15) == 15) {
-      int rc = sync_scalars(h, sc);
-      if (rc) return rc;
-      bool all = true;
-      for (int b = 0; b < h->S; b++) all = all && sc[(size_t)b * kNsc + SC_DONE] != 0.0;
-      if (all) break;
+  const dim3 sg((S + 63) / 64), sb(64), blk(1024);
+  std::vector<int> list(S);
+  for (int b = 0; b < S; b++) list[b] = b;
+  int nact = S;
+  HZCHK(h, hipMemcpyAsync(act, list.data(), S * sizeof(int), hipMemcpyHostToDevice, h->stream));
+  hipLaunchKernelGGL(k_cg_init, red_grid(h), dim3(256), 0, h->stream, g, rhs, x, r, z, part0);
+  hipLaunchKernelGGL(k_cg_start, sg, sb, 0, h->stream, S, part0, cg[0], tol2);
+  std::vector<CgSc> hc(S);
+  int it = 0;
+  for (; it < maxit && nact > 0; it++) {
+    const int e = it & 1;
+    const dim3 grd((unsigned)(nact * kRedBlocks));
+    hipLaunchKernelGGL(k_cg_direction, grd, blk, 0, h->stream, g, act, z, p[e], p[1 - e], part_rz, part_pq, cg[e],
+                       cg[1 - e], tol2, it == 0 ? 1 : 0);
+    hipLaunchKernelGGL(k_cg_update, grd, blk, 0, h->stream, g, act, x, r, z, p[1 - e], part_pq, part_rz, cg[1 - e]);
+    if ((it & 31) == 31) {
+      // a slot that leaves the list keeps its scalars in both sets
+      HZCHK(h, hipMemcpyAsync(cg[e], cg[1 - e], S * sizeof(CgSc), hipMemcpyDeviceToDevice, h->stream));
+      HZCHK(h, hipMemcpyAsync(hc.data(), cg[e], S * sizeof(CgSc), hipMemcpyDeviceToHost, h->stream));
+      HZCHK(h, hipStreamSynchronize(h->stream));
+      const int before = nact;
+      nact = 0;
+      for (int b = 0; b < S; b++)
+        if (hc[b].done == 0.0) list[nact++] = b;
+      if (nact > 0 && nact < before)
+        HZCHK(h, hipMemcpyAsync(act, list.data(), nact * sizeof(int), hipMemcpyHostToDevice, h->stream));
     }
   }
+  hipLaunchKernelGGL(k_cg_end, sg, sb, 0, h->stream, S, part_rz, cg[it & 1], h->d_sc, tol2, it > 0 ? 1 : 0);
+  std::vector<double> sc;
   int rc = sync_scalars(h, sc);
   if (rc) return rc;
-  its.resize(h->S);
-  for (int b = 0; b < h->S; b++)
+  its.resize(S);
+  for (int b = 0; b < S; b++)
     its[b] = sc[(size_t)b * kNsc + SC_DONE] != 0.0 ? (int)sc[(size_t)b * kNsc + SC_IT] : -1;
   HZCHK(h, hipGetLastError());
   return 0;
@@ -1463,13 +1663,17 @@ int vrh_hz_create(const vrh_hz_grid *gr, vrh_hz_t **out) {
                               : h->zmax * k / nz;
   for (int k = 0; k < nz; k++) { h->zm[k] = 0.5 * (h->zf[k] + h->zf[k + 1]); h->dz[k] = h->zf[k + 1] - h->zf[k]; }
   for (int j = 0; j < nr; j++) h->rm[j] = (j + 0.5) * h->dr;
-  std::vector<double> rf(nr + 1, 0.0), izm(nz + 1, 0.0);
+  std::vector<double> rf(nr + 1, 0.0), izm(nz + 1, 0.0), drm(nr), rv(nr);
+  for (int j = 0; j < nr; j++) { drm[j] = h->dr / h->rm[j]; rv[j] = h->rm[j] * h->dr; }
   for (int j = 1; j < nr; j++) rf[j] = (j * h->dr) / h->dr;
   for (int k = 1; k < nz; k++) izm[k] = 1.0 / (h->zm[k] - h->zm[k - 1]);
   int rc;
   if ((rc = halloc(h, &h->d_rm, nr)) || (rc = halloc(h, &h->d_rf, nr + 1)) || (rc = halloc(h, &h->d_dz, nz)) ||
-      (rc = halloc(h, &h->d_izm, nz + 1)) || (rc = halloc(h, &h->d_zm, nz)) || (rc = halloc(h, &h->d_m, h->S)))
+      (rc = halloc(h, &h->d_izm, nz + 1)) || (rc = halloc(h, &h->d_zm, nz)) || (rc = halloc(h, &h->d_m, h->S)) ||
+      (rc = halloc(h, &h->d_drm, nr)) || (rc = halloc(h, &h->d_rv, nr)))
     return rc;
+  if ((rc = hz_h2d(h, h->d_drm, drm.data(), nr * sizeof(double)))) return rc;
+  if ((rc = hz_h2d(h, h->d_rv, rv.data(), nr * sizeof(double)))) return rc;
   if ((rc = hz_h2d(h, h->d_rm, h->rm.data(), nr * sizeof(double)))) return rc;
   if ((rc = hz_h2d(h, h->d_rf, rf.data(), (nr + 1) * sizeof(double)))) return rc;
   if ((rc = hz_h2d(h, h->d_dz, h->dz.data(), nz * sizeof(double)))) return rc;
@@ -1525,7 +1729,7 @@ int vrh_hz_create(const vrh_hz_grid *gr, vrh_hz_t **out) {
 int vrh_hz_destroy(vrh_hz_t *h) {
   if (!h) return -1;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  void *ptrs[] = {h->d_rm, h->d_rf, h->d_dz, h->d_izm, h->d_zm, h->d_m, h->d_V, h->d_lam, h->d_part, h->d_sc,
+  void *ptrs[] = {h->d_drm, h->d_rv, h->d_rm, h->d_rf, h->d_dz, h->d_izm, h->d_zm, h->d_m, h->d_V, h->d_lam, h->d_part, h->d_sc,
                   h->d_w, h->d_g, h->d_m1, h->d_m2, h->d_wf, h->d_wb, h->d_x0, h->d_a[0], h->d_a[1], h->d_a[2],
                   h->d_g4, h->d_gt[0], h->d_gt[1], h->d_out, h->d_loss, h->d_dwpart};
   for (void *p : ptrs) if (p) (void)hipFree(p);
