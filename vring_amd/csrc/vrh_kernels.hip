@@ -1170,7 +1170,7 @@ __host__ __device__ constexpr size_t al16(size_t b) { return (b + 15) & ~(size_t
 // power of two: two real lines per complex FFT in LDS (other ntheta: k_divdft).
 // In mixed mode the packed positions 0..4 (m = 0,1,2) are also produced in
 // double from the double divergence into S64 (layout (5, nr, nz)).
-template <typename TW>
+template <typename TW, bool SPLIT>
 __global__ __launch_bounds__(256) void k_divfft(VGrid g, VCoef c, ZMet zm, double inv_adt, const double *__restrict__ dq1,
                                                 const double *__restrict__ dq2, const double *__restrict__ dq3,
                                                 const double *__restrict__ ext, TW *__restrict__ S,
@@ -1214,25 +1214,28 @@ __global__ __launch_bounds__(256) void k_divfft(VGrid g, VCoef c, ZMet zm, doubl
   const int TPL = nth / LB, lpt = tid / TPL, tl = tid - lpt * TPL;
   const int NU = (N + TPL - 1) / TPL;
   const bool lvalid = l0 + lpt < nlines;
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0;
-  auto put = [&](int ii, double val) {
+  // partial sums of the FP64 low modes: with SPLIT a thread keeps those of its
+  // even and odd angles apart (see launch_poisson)
+  double sm[SPLIT ? 2 : 1][5] = {};
+  auto put = [&](int ii, int u, double val) {
     const int pos = (lpt >> 1) * N + ii;
     if (lpt & 1) im[pos] = (TW)val; else re[pos] = (TW)val;
     if (S64) {  // cos and sin sums of wavenumbers 0, 1, 2
       int q2 = 2 * ii;
       if (q2 >= N) q2 -= N;
-      s0 += val;
-      s1 += val * tw[ii];
-      s2 += val * tw[N + ii];
-      s3 += val * tw[q2];
-      s4 += val * tw[N + q2];
+      double *s = sm[SPLIT ? u & 1 : 0];
+      s[0] += val;
+      s[1] += val * tw[ii];
+      s[2] += val * tw[N + ii];
+      s[3] += val * tw[q2];
+      s[4] += val * tw[N + q2];
     }
   };
   const int jl = jk[2 * lpt], kl = jk[2 * lpt + 1];
   if (ext) {
     for (int u = 0; u < NU; ++u) {
       const int ii = tl + TPL * u;
-      if (ii < N) put(ii, lvalid ? ext[cidx(g, ii + 1, jl, kl)] : 0.0);
+      if (ii < N) put(ii, u, lvalid ? ext[cidx(g, ii + 1, jl, kl)] : 0.0);
     }
   } else {
     // the loads of U angles are all issued before the first is used;
@@ -1260,7 +1263,7 @@ __global__ __launch_bounds__(256) void k_divfft(VGrid g, VCoef c, ZMet zm, doubl
         const int ii = tl + TPL * (ub + u);
         if (ii < N) {
           const double rhs = divq_rhs(b1[u] - a1[u], g.dx1 * g.axsym, b2[u] - a2[u], rdv, rmv, b3[u] - a3[u], zkv, inv_adt);
-          put(ii, lvalid ? rhs : 0.0);
+          put(ii, u, lvalid ? rhs : 0.0);  // ub is a multiple of U: u has the parity of ub + u
         }
       }
     }
@@ -1269,16 +1272,16 @@ __global__ __launch_bounds__(256) void k_divfft(VGrid g, VCoef c, ZMet zm, doubl
     // the line's TPL lanes: a fixed butterfly within each wave (deterministic
     // order), then one partial per wave into LDS
     const int grp = TPL < 64 ? TPL : 64;
-    for (int o = grp >> 1; o > 0; o >>= 1) {
-      s0 += __shfl_xor(s0, o, grp);
-      s1 += __shfl_xor(s1, o, grp);
-      s2 += __shfl_xor(s2, o, grp);
-      s3 += __shfl_xor(s3, o, grp);
-      s4 += __shfl_xor(s4, o, grp);
-    }
+    if (SPLIT)
+#pragma unroll
+      for (int w = 0; w < 5; w++) sm[0][w] += sm[SPLIT ? 1 : 0][w];
+    for (int o = grp >> 1; o > 0; o >>= 1)
+#pragma unroll
+      for (int w = 0; w < 5; w++) sm[0][w] += __shfl_xor(sm[0][w], o, grp);
     if ((tl & (grp - 1)) == 0) {
       double *pp = part + (size_t)lpt * 10 + tl / grp;
-      pp[0] = s0; pp[2] = s1; pp[4] = s2; pp[6] = s3; pp[8] = s4;
+#pragma unroll
+      for (int w = 0; w < 5; w++) pp[2 * w] = sm[0][w];
     }
   }
   __syncthreads();
@@ -1318,8 +1321,11 @@ __global__ __launch_bounds__(256) void k_divfft(VGrid g, VCoef c, ZMet zm, doubl
 // lines per block, nz a power of two (other nz: k_zdense); lines are contiguous in memory (line stride 1, position
 // stride nl).  Makhoul's reordering turns each pair of real lines into one
 // complex FFT of length nz.  dir=+1 forward, -1 inverse (REDFT01).
+// FP32: at most 64 VGPRs, so that two 1024-lane blocks share a CU, one
+// loading while the other transforms (us forward/inverse, without and with:
+// 256x512x1024 758/749, 482/456; 128x256x512 54/49, 50/48).
 template <typename TW>
-__global__ __launch_bounds__(1024) void k_dctz(TW *__restrict__ S, long nl, int n, int logn, int TL, int logtl, int dir,
+__global__ __launch_bounds__(1024, sizeof(TW) == 4 ? 8 : 1) void k_dctz(TW *__restrict__ S, long nl, int n, int logn, int TL, int logtl, int dir,
                                               const double *__restrict__ twr, const double *__restrict__ twi,
                                               const double *__restrict__ er, const double *__restrict__ ei) {
   extern __shared__ unsigned char smem_raw[];
@@ -2290,11 +2296,16 @@ template <typename TW> void launch_poisson(vrh_t *h, int irk, const double *ext_
   TW *S = (TW *)h->f.S;
   double *S64 = (h->prec == VRH_MIXED) ? h->f.S64 : nullptr;
   const double adt = h->rk[irk].a * h->dt;
-  int LB = h->fft_lines > 0 ? h->fft_lines : 1024 / N;
-  if (LB > 16) LB = 16;
-  // butterflies per thread of the LDS FFT: (LB/2) N / rmin <= qt * 256
+  // Lines per block: 16, or 8 of 256 angles (butterflies per thread of the LDS
+  // FFT: (LB/2) N / rmin <= qt 256).  us forward/inverse with 4, 8, 16 lines:
+  // mixed 128x256x512 289/124, 179/84, 150/68; FP64 255/124, 162/84, 144/79;
+  // with 2, 4, 8 of mixed 256x512x1024 2310/1080, 1348/710, 1089/536.
+  int LB = h->fft_lines > 0 ? h->fft_lines : 16;
   while (LB > 2 && (LB / 2) * N / fft_min_radix(logn) > 256 * fft_qt<TW>()) LB /= 2;
-  if (LB < 2) LB = 2;
+  // The low modes' sums run over 256 / LB lanes; the default keeps the order of
+  // N / 4 lanes (of 1024 / N lines), two of whose sums a lane then holds
+  // apart, so that the mixed path's results do not depend on LB.
+  const bool split = S64 && h->fft_lines <= 0 && 2 * (256 / LB) == N / 4;
   const dim3 fgrd((unsigned)((nlines + LB - 1) / LB));
   {
     KTimer kt(h, KT_DIVFFT);
@@ -2302,7 +2313,7 @@ template <typename TW> void launch_poisson(vrh_t *h, int irk, const double *ext_
       size_t sh = al16(sizeof(TW) * LB * N);
       if (S64) sh = al16(sh + sizeof(double) * (2 * (size_t)N + 10 * (size_t)LB));
       sh = al16(al16(sh + sizeof(TW) * N) + sizeof(int) * 2 * LB) + sizeof(double) * 2 * LB;
-      hipLaunchKernelGGL(k_divfft<TW>, fgrd, dim3(256), sh, h->stream, g, h->coef, h->zmet, 1.0 / adt, h->f.dq1,
+      hipLaunchKernelGGL((split ? k_divfft<TW, true> : k_divfft<TW, false>), fgrd, dim3(256), sh, h->stream, g, h->coef, h->zmet, 1.0 / adt, h->f.dq1,
                          h->f.dq2, h->f.dq3, ext_rhs, S, S64, h->d_twt, h->d_twt + N, LB, logn);
     } else {
       launch_divdft<TW>(h, 1.0 / adt, ext_rhs, S, S64);
