@@ -1,0 +1,74 @@
+"""The substep at the edges of the rules that pick its kernels from the grid:
+theta lengths around the explicit kernels' row widths (32 and 64 lanes, 2, 3
+and 4 cells a lane) in every form, and the segment lengths of the grouped r
+and z sweeps, with and without lanes and waves to spare, against the single
+sweeps' results and the oracle."""
+import numpy as np
+import pytest
+
+import vring_amd
+from gpu_common import compare, make_pair, seed_fields, seed_random
+
+pytestmark = pytest.mark.gpu
+
+
+def substeps(o, s):
+    """To the 1e-11 of the other phase tests."""
+    for irk in (1, 2, 3):
+        for p in ["ucoeff", "coesys", "hdnbc", "hdnl1", "hdnl2", "hdnl3", "step"]:
+            assert o.phase(p, irk) == 0
+        for p in ["hdnbc", "explicit", "adi"]:
+            s.phase(p, irk)
+        compare(o, s, ["dq1", "dq2", "dq3", "ru1", "ru2", "ru3"], 1e-11)
+        for p in ["divq", "laplace", "upsol", "uppres"]:
+            assert o.phase(p, irk) == 0
+        for p in ["poisson", "project"]:
+            s.phase(p, irk)
+        compare(o, s, ["dph", "q1", "q2", "q3", "pres", "prg"], 1e-11)
+
+
+@pytest.mark.parametrize("nt", [4, 31, 32, 63, 64, 65, 127, 129, 191, 192, 193, 255, 256])
+@pytest.mark.parametrize("form", [-1, 0, 1, 2, 3])
+def test_explicit_row_widths_match_oracle(nt, form):
+    nr, nz = 5, 7
+    print(f"case explicit nt={nt} form={form}", flush=True)
+    o, s = make_pair(nt, nr, nz)
+    s.set_tuning(explicit_form=form)
+    seed_random(o, s, seed=nt)
+    o.set_time(0.13)
+    s.set_time(0.13)
+    substeps(o, s)
+
+
+# r segments 16 and 24, z segments 16, 24 and 40; the last two run one by one
+@pytest.mark.parametrize("nt,nr,nz", [(5, 15, 16), (7, 16, 15), (9, 255, 30), (3, 17, 256), (8, 264, 31), (5, 271, 256),
+                                      (4, 12, 520), (3, 271, 512), (3, 300, 20), (4, 9, 700)])
+def test_sweeps_of_all_segments_match_oracle(nt, nr, nz):
+    print(f"case sweeps {nt}x{nr}x{nz}", flush=True)
+    o, s = make_pair(nt, nr, nz, slip=0.25)
+    seed_random(o, s, seed=nr + nz)
+    o.set_time(0.13)
+    s.set_time(0.13)
+    substeps(o, s)
+
+
+@pytest.mark.parametrize("nt,nr,nz,M", [(33, 16, 200, 0), (16, 32, 300, 0), (8, 16, 513, 0), (16, 32, 60, 32),
+                                        (16, 32, 60, 48)])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_whole_steps_grouped_and_single(nt, nr, nz, M, precision):
+    """hdnbc rides in the grouped sweeps of a whole step (M = 0: the default
+    segments) and runs by itself beside single ones; 5 steps of a ring, FP64
+    to the 1e-10 of the 100-step test, mixed to its 1e-6."""
+    print(f"case whole step {nt}x{nr}x{nz} M={M} {precision}", flush=True)
+    rmax, zmax = 4.0, 12.0
+    q1, q2, q3 = vring_amd.ring_initial_condition(nt, nr, nz, rmax, zmax, [(1.0, 3.0, 0.4, 1.0)])
+    dt = vring_amd.cfl_dt(nt, nr, nz, rmax, zmax, q1, q2, q3, cfl=0.3, ujet=1.0)
+    o, s = make_pair(nt, nr, nz, rmax, zmax, Re=500.0, dt=dt, precision=precision)
+    if M:
+        s.set_tuning(M=(M,) * 6)
+    seed_fields(o, s, q1, q2, q3)
+    for _ in range(5):
+        assert o.rk3_step() == 0
+    s.step(5)
+    vscale = max(np.abs(o.field("q2")).max(), np.abs(o.field("q3")).max())
+    compare(o, s, ["q1", "q2", "q3"], 1e-10 if precision == "fp64" else 1e-6, scale=vscale)

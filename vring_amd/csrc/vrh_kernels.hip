@@ -29,29 +29,6 @@ __device__ __forceinline__ void xcd_block(int &bx, int &by, int &bz) {
   bz = (int)(r / ny);
 }
 
-// ---------------------------------------------------------------------------
-// hdnbc: outlet convective condition and mass correction, one thread per
-// (theta, r) outlet point (momentum_terms_swirl.F90:225-291).  zm3n: the
-// outlet cell's z difference dx3/dmz(nz) on an axial mesh, 0 on the uniform one.
-// ---------------------------------------------------------------------------
-__global__ void k_hdnbc(VGrid g, VCoef c, double zm3n, double gam, double rom, double cor, const double *__restrict__ cor_dev,
-                        const double *__restrict__ q3, double *__restrict__ csort, double *__restrict__ dq3no,
-                        double *__restrict__ corr3n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  int j = blockIdx.y + 1;  // 1..nrc
-  if (i > g.nt) return;
-  if (cor_dev) cor = *cor_dev;
-  long p = (long)(i - 1) + (long)g.nt * j;
-  double qn = q3[hidx(g, i, j, g.nzc)], qm = q3[hidx(g, i, j, g.nz)];
-  double cs = csort[p];
-  if (j <= g.nr && qn > 0.0) cs = (double)0.6f * qn;
-  csort[p] = cs;
-  double tconv = -(cs * (zm3n > 0.0 ? zm3n : g.dx3)) * (qn - qm);
-  double c3n = (gam * tconv + rom * dq3no[p]) * g.dt;
-  dq3no[p] = tconv;
-  corr3n[p] = c3n + c.qc[j] * cor;
-}
-
 // Inlet time profile (gen_tools_swirl.F90:159-175): smooth ramp to 1 over
 // 0.1n, hold until n, ramp down (n = 2).
 __device__ __host__ inline double profile_fn(double t) {
@@ -856,140 +833,6 @@ __global__ __launch_bounds__(512) void k_explicit_cell(VGrid g, const double *__
   r1[o] = v1 * d1;
   if (j >= 2) r2[o] = v2 * d2;
   if (k >= 2) r3[o] = v3 * d1;
-}
-
-// ---------------------------------------------------------------------------
-// Partitioned Thomas solve of the r and z sweeps (solqj/solqk with
-// solve_lap_par/solve_lap_thom, step.F90:266-485; tripar.F90:11-145).
-// A block owns 64 lines (one per lane, consecutive theta -> coalesced) and P
-// waves; wave s owns positions [s*M, s*M+M) of every line and keeps them in
-// registers.  The two linear recurrences of the Thomas algorithm are closed
-// across segments with precomputed carry products (one LDS exchange each).
-// ---------------------------------------------------------------------------
-struct LineArgs {
-  LineCoef lc;
-  VGrid g;
-  long nlines;
-  int j0;                      // first r index of z-lines
-  double slip;
-  const double *q;             // state component (z sweeps / q2 r sweep)
-  double *dq;                  // predictor output (z sweeps of q1,q3 / r sweep of q2)
-  void *r;                     // qrhs of the component (TW)
-  const double *corr3n;        // outlet row of the q3 z sweep
-  double c3s;                  // inlet row value of the q3 z sweep (uniform in theta)
-  const double *c3s_dev;       // same value read from the device (captured steps), or null
-  int jlim;                    // inlet rows: j <= jlim
-};
-
-template <typename TW, int M, int MODE>
-__global__ __attribute__((amdgpu_flat_work_group_size(64, 1024), amdgpu_waves_per_eu(1, 4))) void k_line(LineArgs a) {
-  __shared__ TW sh_a[16][64];
-  const int lane = threadIdx.x & 63;
-  const int s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const long L = (long)blockIdx.x * 64 + lane;
-  const bool act = L < a.nlines;
-  const long Lc = act ? L : a.nlines - 1;  // addresses stay in bounds; results of !act lanes are dropped
-  const VGrid &g = a.g;
-  const int n = a.lc.n, P = a.lc.P;
-  const int p0 = s * M;
-  const int len = min(M, n - p0);
-  TW *rr = reinterpret_cast<TW *>(a.r);
-  // the coefficients in the work type (the mixed path's float copies)
-  auto cw = [](const double *d, const float *f) {
-    if constexpr (sizeof(TW) == 4) { (void)d; return f; } else { (void)f; return d; }
-  };
-  const TW *cA = cw(a.lc.A, a.lc.Af), *cB = cw(a.lc.B, a.lc.Bf), *cC = cw(a.lc.C, a.lc.Cf);
-  const TW *cPk = cw(a.lc.Pk, a.lc.Pkf), *cQk = cw(a.lc.Qk, a.lc.Qkf);
-  const TW *cPs = cw(a.lc.Pseg, a.lc.Psegf), *cQs = cw(a.lc.Qseg, a.lc.Qsegf);
-  // line -> (i, second index)
-  const int i = (int)(Lc % g.nt) + 1;
-  const int l2 = (int)(Lc / g.nt);
-  long base;  // address of position 0 of the line
-  long step;  // address stride between positions
-  if (MODE <= SW_R2) { base = hidx(g, i, 1, l2 + 1); step = g.sj; }      // r lines at k = l2+1
-  else { base = hidx(g, i, l2 + a.j0, 1); step = g.sk; }                  // z lines at j = l2+j0
-  const int jz = l2 + a.j0;
-  // every load of the segment is issued before the first use (positions
-  // beyond the line clamp to its last one and are masked afterwards)
-  TW x[M];
-#pragma unroll
-  for (int t = 0; t < M; ++t) x[t] = rr[base + step * min(p0 + t, n - 1)];
-  TW rlast = (TW)0;
-  if (MODE == SW_Z3) rlast = (TW)a.corr3n[(long)(i - 1) + (long)g.nt * jz];
-  __builtin_amdgcn_sched_barrier(0);
-  TW gp = (TW)0;
-#pragma unroll
-  for (int t = 0; t < M; ++t) {
-    const int p = p0 + t;
-    TW rv = x[t];
-    if (MODE == SW_R2 || MODE == SW_Z1 || MODE == SW_Z2) {
-      if (p == 0 || p == n - 1) rv = (TW)0;
-    } else if (MODE == SW_Z3) {
-      if (p == 0) rv = (jz <= a.jlim) ? (TW)(a.c3s_dev ? *a.c3s_dev : a.c3s) : (TW)0;
-      else if (p == n - 1) rv = rlast;
-    }
-    const TW v = cA[p] * rv + cB[p] * gp;
-    const bool in = t < len;
-    x[t] = in ? v : (TW)0;
-    gp = in ? v : gp;
-  }
-  sh_a[s][lane] = gp;
-  __syncthreads();
-  TW G = (TW)0;
-  for (int s2 = 0; s2 < s; ++s2) G = sh_a[s2][lane] + cPs[s2] * G;
-  __syncthreads();
-  TW xp = (TW)0;
-#pragma unroll
-  for (int t = M - 1; t >= 0; --t) {
-    const int p = p0 + t;
-    const TW v = x[t] + cPk[p] * G - cC[p] * xp;
-    const bool in = t < len;
-    x[t] = in ? v : x[t];
-    xp = in ? v : xp;
-  }
-  sh_a[s][lane] = xp;
-  __syncthreads();
-  TW X = (TW)0;
-  for (int s2 = P - 1; s2 > s; --s2) X = sh_a[s2][lane] + cQs[s2] * X;
-#pragma unroll
-  for (int t = 0; t < M; ++t) x[t] = x[t] + cQk[p0 + t] * X;
-  if (MODE == SW_R1 || MODE == SW_R3 || MODE == SW_Z2) {
-    if (!act) return;
-#pragma unroll
-    for (int t = 0; t < M; ++t)
-      if (t < len) rr[base + step * (p0 + t)] = x[t];
-  } else {
-    // dq = q + x, in chunks of 8 positions whose q loads go out together
-    // before their stores
-    constexpr int CH = 8;
-#pragma unroll
-    for (int c0 = 0; c0 < M; c0 += CH) {
-      double qv[CH];
-#pragma unroll
-      for (int u = 0; u < CH; ++u)
-        qv[u] = (c0 + u < M) ? a.q[base + step * min(p0 + c0 + u, n - 1)] : 0.0;
-      __builtin_amdgcn_sched_barrier(0);
-      if (act) {
-#pragma unroll
-        for (int u = 0; u < CH; ++u) {
-          const int t = c0 + u;
-          if (t < M && t < len) {
-            const int p = p0 + t;
-            const long ad = base + step * p;
-            if (MODE == SW_R2) {
-              // dq2 = x + q2 for j = 1..nr; dq2(nrc) = 0 (step.F90:330-333, 183-187)
-              a.dq[ad] = (p == n - 1) ? 0.0 : (double)x[t] + qv[u];
-            } else {
-              // dq = q + x for k = 1..nzc; slip row at nrc (step.F90:84-88, 133-138)
-              const double d = qv[u] + (double)x[t];
-              a.dq[ad] = d;
-              if (jz == g.nr) a.dq[ad + g.sj] = a.slip * d;
-            }
-          }
-        }
-      }
-    }
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1907,18 +1750,6 @@ __global__ void k_analysis_sum(const double *__restrict__ part, int nblk, double
 // ===========================================================================
 #define CHECK_LAUNCH() (void)hipGetLastError()
 
-static void hdnbc_on(vrh_t *h, int irk, double cor, const double *cor_dev, hipStream_t st) {
-  const VGrid &g = h->g;
-  dim3 blk(64), grd((g.nt + 63) / 64, g.nrc);
-  KTimer kt(h, KT_HDNBC);
-  const double zm3n = h->zmesh[2].empty() ? 0.0 : g.dx3 / h->zmesh[2][g.nz];
-  hipLaunchKernelGGL(k_hdnbc, grd, blk, 0, st, g, h->coef, zm3n, h->rk[irk].g, h->rk[irk].r, cor, cor_dev, h->f.q3,
-                     h->f.csort, h->f.dq3no, h->f.corr3n);
-}
-template <typename TW> void launch_hdnbc(vrh_t *h, int irk, double cor, const double *cor_dev) {
-  hdnbc_on(h, irk, cor, cor_dev, h->stream);
-}
-
 void launch_scalars(vrh_t *h) {
   hipLaunchKernelGGL(k_scalars, dim3(1), dim3(64), 0, h->stream, h->d_sc, h->dt, h->rk[1].a, h->rk[2].a,
                      h->rk[3].a, h->inlet_area, h->cor_red, 1, 0.0);
@@ -2098,72 +1929,6 @@ void lds_optin(vrh_t *h) {
   if (lb > 65536) ok = ok && dense_lds_optin(lb);
   (void)hipGetLastError();
   if (ok) { h->lds_block = lb; h->lds_cu = lc; }
-}
-
-template <typename TW, int MODE>
-static void line_launch(vrh_t *h, const LineArgs &a, int M, hipStream_t st) {
-  const int P = a.lc.P;
-  dim3 blk(64 * P), grd((unsigned)((a.nlines + 63) / 64));
-  KTimer kt(h, MODE <= SW_R2 ? KT_LINE_R : KT_LINE_Z);
-  switch (M) {
-    case 16: hipLaunchKernelGGL((k_line<TW, 16, MODE>), grd, blk, 0, st, a); break;
-    case 24: hipLaunchKernelGGL((k_line<TW, 24, MODE>), grd, blk, 0, st, a); break;
-    case 32: hipLaunchKernelGGL((k_line<TW, 32, MODE>), grd, blk, 0, st, a); break;
-    case 40: hipLaunchKernelGGL((k_line<TW, 40, MODE>), grd, blk, 0, st, a); break;
-    case 48: hipLaunchKernelGGL((k_line<TW, 48, MODE>), grd, blk, 0, st, a); break;
-    case 72: hipLaunchKernelGGL((k_line<TW, 72, MODE>), grd, blk, 0, st, a); break;
-    default: hipLaunchKernelGGL((k_line<TW, 64, MODE>), grd, blk, 0, st, a); break;
-  }
-}
-
-template <typename TW> void launch_sweeps(vrh_t *h, int irk, double c3s, const double *c3s_dev, bool hdnbc,
-                                          double cor, const double *cor_dev) {
-  const VGrid &g = h->g;
-  LineArgs a{};
-  a.g = g;
-  a.slip = h->slip;
-  a.jlim = h->jlim;
-  a.c3s = c3s;
-  a.c3s_dev = c3s_dev;
-  a.corr3n = h->f.corr3n;
-  // The three components' chains are independent: q3 and q2 run on the
-  // side streams, forked from and joined back into the handle's stream
-  // (captured steps record the fork as graph branches).  With the kernel
-  // timer on, and inside an ensemble graph (whose members already run side
-  // by side), all run in order on the handle's stream.
-  const bool par = !h->kt_on && !h->serial_sweeps;
-  hipStream_t s1 = par ? h->side[0] : h->stream, s2 = par ? h->side[1] : h->stream;
-  const int ie = (irk >= 1 && irk <= 3) ? irk : 0;
-  if (par) {
-    (void)hipEventRecord(h->fork_ev[ie], h->stream);
-    (void)hipStreamWaitEvent(s1, h->fork_ev[ie], 0);
-    (void)hipStreamWaitEvent(s2, h->fork_ev[ie], 0);
-  }
-  // q1: r then z (step.F90:75-78)
-  a.lc = h->lc[irk][SW_R1]; a.nlines = (long)g.nt * g.nz; a.r = h->f.r1;
-  line_launch<TW, SW_R1>(h, a, h->Msw[SW_R1], h->stream);
-  a.lc = h->lc[irk][SW_Z1]; a.nlines = (long)g.nt * g.nr; a.j0 = 1; a.q = h->f.q1; a.dq = h->f.dq1;
-  line_launch<TW, SW_Z1>(h, a, h->Msw[SW_Z1], h->stream);
-  // q3: r then z (step.F90:124-127).  In a whole step the outlet rows of
-  // hdnbc (csort, dq3no, corr3n: read only by the q3 z sweep; computed from
-  // q3, which the explicit kernel leaves alone) head this chain, off the
-  // critical path.
-  if (hdnbc) hdnbc_on(h, irk, cor, cor_dev, s1);
-  a.lc = h->lc[irk][SW_R3]; a.nlines = (long)g.nt * g.nz; a.r = h->f.r3;
-  line_launch<TW, SW_R3>(h, a, h->Msw[SW_R3], s1);
-  a.lc = h->lc[irk][SW_Z3]; a.nlines = (long)g.nt * g.nr; a.j0 = 1; a.q = h->f.q3; a.dq = h->f.dq3;
-  line_launch<TW, SW_Z3>(h, a, h->Msw[SW_Z3], s1);
-  // q2: z then r (step.F90:171-177)
-  a.lc = h->lc[irk][SW_Z2]; a.nlines = (long)g.nt * (g.nr - 1); a.j0 = 2; a.r = h->f.r2;
-  line_launch<TW, SW_Z2>(h, a, h->Msw[SW_Z2], s2);
-  a.lc = h->lc[irk][SW_R2]; a.nlines = (long)g.nt * g.nzc; a.q = h->f.q2; a.dq = h->f.dq2;
-  line_launch<TW, SW_R2>(h, a, h->Msw[SW_R2], s2);
-  if (par) {
-    (void)hipEventRecord(h->join_ev[ie][0], s1);
-    (void)hipEventRecord(h->join_ev[ie][1], s2);
-    (void)hipStreamWaitEvent(h->stream, h->join_ev[ie][0], 0);
-    (void)hipStreamWaitEvent(h->stream, h->join_ev[ie][1], 0);
-  }
 }
 
 static int ilog2(int n) { int l = 0; while ((1 << l) < n) ++l; return l; }
@@ -2441,9 +2206,7 @@ double *analysis_scratch(int dev) {
 }
 
 #define INST(TW)                                                   \
-  template void launch_hdnbc<TW>(vrh_t *, int, double, const double *); \
   template void launch_explicit<TW>(vrh_t *, int);                 \
-  template void launch_sweeps<TW>(vrh_t *, int, double, const double *, bool, double, const double *); \
   template void launch_poisson<TW>(vrh_t *, int, const double *, double *); \
   template void launch_project<TW>(vrh_t *, int);
 INST(double)
