@@ -1481,11 +1481,15 @@ __global__ __launch_bounds__(256) void k_ifft(VGrid g, const TW *__restrict__ S,
 // side), so each dph value is fetched from HBM about once; the gradient
 // components qcap are recomputed from the ring where the reference stores
 // them.  Everything that depends on the thread's r row only (metric ratios,
-// reciprocals of rm) is hoisted out of the z loop.
+// reciprocals of rm) is hoisted out of the z loop; a wavefront of a 64-wide
+// tile has one row and holds these in scalar registers, which leaves room for
+// a fourth wave per SIMD (64x128x256: 64.5 -> 60 us).  Bound by memory: 15
+// arrays, 5.2 TB/s at 128x256x512.
 // ---------------------------------------------------------------------------
 template <int W, int R, bool ZS>
-__global__ __launch_bounds__(W * R) void k_project(VGrid g, VCoef c, ZMet zm, double adt, double be, int kchunk,
-                                                    const double *__restrict__ dph, const double *__restrict__ dq1,
+__global__ __launch_bounds__(W * R, W == 64 ? 4 : 3) void k_project(VGrid g, VCoef c, ZMet zm, double adt, double be,
+                                                    int kchunk, int xcd, const double *__restrict__ dph,
+                                                    const double *__restrict__ dq1,
                                                     const double *__restrict__ dq2, const double *__restrict__ dq3,
                                                     double *__restrict__ q1, double *__restrict__ q2,
                                                     double *__restrict__ q3, double *__restrict__ prg1,
@@ -1494,12 +1498,19 @@ __global__ __launch_bounds__(W * R) void k_project(VGrid g, VCoef c, ZMet zm, do
   constexpr int LC = W + 3, LR = R + 3, NE = LR * LC, NT = W * R;
   constexpr int NL = (NE + NT - 1) / NT;
   __shared__ double ring[4][LR][LC + 1];
-  const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * W + tx;
+  // a wavefront has one r row (W = 64): its coefficients sit in scalar registers
+  const int tx = threadIdx.x, ty = W == 64 ? __builtin_amdgcn_readfirstlane(threadIdx.y) : threadIdx.y, tid = ty * W + tx;
+  auto uni = [](double v) {
+    if (W != 64) return v;
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)), __builtin_amdgcn_readfirstlane(__double2loint(v)));
+  };
   const int nt = g.nt, nr = g.nr, nz = g.nz, nrc = g.nrc, nzc = g.nzc;
   const long sj = g.sj, sk = g.sk;
-  const int i0 = blockIdx.x * W;  // 0-based theta of the tile's first column
-  const int j0 = blockIdx.y * R;  // rows 0..nrc (row 0 only takes the inlet copy of q3)
-  const int kb = 1 + blockIdx.z * kchunk;
+  int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
+  if (xcd) xcd_block(bx, by, bz);
+  const int i0 = bx * W;  // 0-based theta of the tile's first column
+  const int j0 = by * R;  // rows 0..nrc (row 0 only takes the inlet copy of q3)
+  const int kb = 1 + bz * kchunk;
   const int ke = min(kb + kchunk - 1, nzc);
   // ring fill: element e = tid + l*NT of the (LR x LC) plane tile
   long goff[NL];
@@ -1545,14 +1556,14 @@ __global__ __launch_bounds__(W * R) void k_project(VGrid g, VCoef c, ZMet zm, do
   const int jq = (jr >= 1 && jr <= nr) ? jr : 1;  // rows of the uppres coefficients
   const int djp = (jq == nr) ? 0 : 1, djm = (jq == 1) ? 0 : -1;
   // radial gradient rc dx2 / dcr (divergence.F90:132, 327)
-  const double a1 = adt * g.dx1 / c.rm[jq], a2 = adt * c.rc[jr] * g.dx2 / c.dcr[jr], a3 = adt * g.dx3;
-  const double irm = 1.0 / c.rm[jq], irmp = 1.0 / c.rm[jq + djp], irmm = 1.0 / c.rm[jq + djm];
-  const double irmn = 1.0 / c.rm[jq + 1];
+  const double a1 = uni(adt * g.dx1 / c.rm[jq]), a2 = uni(adt * c.rc[jr] * g.dx2 / c.dcr[jr]), a3 = adt * g.dx3;
+  const double irm = uni(1.0 / c.rm[jq]), irmp = uni(1.0 / c.rm[jq + djp]), irmm = uni(1.0 / c.rm[jq + djm]);
+  const double irmn = uni(1.0 / c.rm[jq + 1]);
   const double s1t11 = c.s1t11[jq], s1t2n = c.s1t2n[jq], s1t2s = c.s1t2s[jq], s1t2c = c.s1t2c[jq];
   const double s2t11 = c.s2t11[jq], s2t2p = c.s2t2p[jq], s2t2m = c.s2t2m[jq];
   const double s3t2n = c.s3t2n[jq], s3t2s = c.s3t2s[jq];
   const int jqp = min(jq + 1, nrc), jqm = max(jq - 1, 1);
-  const double rcj = c.rc[jq] / c.dcr[jq], rcp = c.rc[jqp] / c.dcr[jqp], rcm = c.rc[jqm] / c.dcr[jqm];
+  const double rcj = uni(c.rc[jq] / c.dcr[jq]), rcp = uni(c.rc[jqp] / c.dcr[jqp]), rcm = uni(c.rc[jqm] / c.dcr[jqm]);
   const double dx1 = g.dx1, dx2 = g.dx2, dx3 = g.dx3, dx3q = g.dx3q, slip = g.slip;
   const int cx = tx + 2, cy = ty + 2;
   // the streamed operands of the next plane are loaded while this one is computed
@@ -1576,13 +1587,20 @@ __global__ __launch_bounds__(W * R) void k_project(VGrid g, VCoef c, ZMet zm, do
     n_pres = pres[oo];
   };
   load_cell(kb);
+  // the plane's axial metric terms, read one plane ahead as well
+  struct ZM { double c3, c3p, c3m, cp, cm, fp, fm; };
+  auto load_zm = [&](int k) { return ZM{zm.c3[k], zm.c3[k + 1], zm.c3[k - 1], zm.cp[k], zm.cm[k], zm.fp[k], zm.fm[k]}; };
+  ZM z{};
+  if (ZS) z = load_zm(kb);
   for (int k = kb; k <= ke; k++) {
+    const ZM zk = z;
     stash(k + 1);
     const double c_dq1 = n_dq1, c_dq2 = n_dq2, c_dq3 = n_dq3, c_pres = n_pres;
     const double c_p1 = n_p1, c_p2 = n_p2, c_p3 = n_p3;
     __syncthreads();
     fetch(k + 2);
     load_cell(k + 1);
+    if (ZS) z = load_zm(min(k + 1, ke));
     if (act) {
       const double(*P0)[LC + 1] = ring[k & 3];
       const double(*Pm)[LC + 1] = ring[(k - 1) & 3];
@@ -1595,7 +1613,7 @@ __global__ __launch_bounds__(W * R) void k_project(VGrid g, VCoef c, ZMet zm, do
       // axial mesh: the z gradient at faces k, k+1, k-1 and the z-gradient
       // factor of upsol; the uniform mesh keeps dx3
       constexpr bool zs = ZS;  // axial mesh (a separate instantiation)
-      const double zc0 = zs ? zm.c3[k] : dx3, zcp = zs ? zm.c3[k + 1] : dx3, zcm = zs ? zm.c3[k - 1] : dx3;
+      const double zc0 = zs ? zk.c3 : dx3, zcp = zs ? zk.c3p : dx3, zcm = zs ? zk.c3m : dx3;
       const double a3k = zs ? adt * zc0 : a3;
       // ---- upsol ----
       if (j >= 1 && j <= nr) {
@@ -1623,7 +1641,7 @@ __global__ __launch_bounds__(W * R) void k_project(VGrid g, VCoef c, ZMet zm, do
           const double qjp = (P0[cy + djp][cx] - P0[cy + djp][cx - 1]) * dx1 * irmp;
           const double qjm = (P0[cy + djm][cx] - P0[cy + djm][cx - 1]) * dx1 * irmm;
           const double d11 = (qip - 2.0 * qc0 + qim) * s1t11;
-          const double d33 = zs ? (qkp - qc0) * zm.cp[k] - (qc0 - qkm) * zm.cm[k] : (qkp - 2.0 * qc0 + qkm) * dx3q;
+          const double d33 = zs ? (qkp - qc0) * zk.cp - (qc0 - qkm) * zk.cm : (qkp - 2.0 * qc0 + qkm) * dx3q;
           const double qnn = qjp * irmn - qc0 * irm;
           const double qss = qc0 * irm - qjm * irmm;
           const double d22 = (qnn * s1t2n - qss * s1t2s) * s1t2c;
@@ -1639,7 +1657,7 @@ __global__ __launch_bounds__(W * R) void k_project(VGrid g, VCoef c, ZMet zm, do
           const double qjp = (j + 1 < nrc) ? (P0[cy + 1][cx] - p0) * dx2 * rcp : 0.0;
           const double qjm = (j - 1 > 1) ? (P0[cy - 1][cx] - P0[cy - 2][cx]) * dx2 * rcm : 0.0;
           const double d11 = (qip - 2.0 * qc0 + qim) * s2t11;
-          const double d33 = zs ? (qkp - qc0) * zm.cp[k] - (qc0 - qkm) * zm.cm[k] : (qkp - 2.0 * qc0 + qkm) * dx3q;
+          const double d33 = zs ? (qkp - qc0) * zk.cp - (qc0 - qkm) * zk.cm : (qkp - 2.0 * qc0 + qkm) * dx3q;
           const double d22 = (qjp - qc0) * s2t2p - (qc0 - qjm) * s2t2m;
           prg2[pc] = c_p2 + qc0 - be * (d11 + d22 + d33);
         }
@@ -1655,7 +1673,7 @@ __global__ __launch_bounds__(W * R) void k_project(VGrid g, VCoef c, ZMet zm, do
             const double qjp = (P0[cy + djp][cx] - Pm[cy + djp][cx]) * zc0;
             const double qjm = (P0[cy + djm][cx] - Pm[cy + djm][cx]) * zc0;
             const double d11 = (qip - 2.0 * qc0 + qim) * s1t11;
-            const double d33 = zs ? (qkp - qc0) * zm.fp[k] - (qc0 - qkm) * zm.fm[k] : (qkp - 2.0 * qc0 + qkm) * dx3q;
+            const double d33 = zs ? (qkp - qc0) * zk.fp - (qc0 - qkm) * zk.fm : (qkp - 2.0 * qc0 + qkm) * dx3q;
             const double d22 = (qjp - qc0) * s3t2n - (qc0 - qjm) * s3t2s;
             prg3[pc] = c_p3 + qc0 - be * (d11 + d22 + d33);
           }
@@ -1663,7 +1681,7 @@ __global__ __launch_bounds__(W * R) void k_project(VGrid g, VCoef c, ZMet zm, do
         {
           const double d11 = (P0[cy][cx + 1] + P0[cy][cx - 1] - 2.0 * p0) * s1t11;
           const double d22 = (P0[cy + djp][cx] - p0) * s3t2n - (p0 - P0[cy + djm][cx]) * s3t2s;
-          const double d33 = zs ? (Pp[cy][cx] - p0) * zm.cp[k] - (p0 - Pkm[cy][cx]) * zm.cm[k]
+          const double d33 = zs ? (Pp[cy][cx] - p0) * zk.cp - (p0 - Pkm[cy][cx]) * zk.cm
                                 : (Pp[cy][cx] + Pkm[cy][cx] - 2.0 * p0) * dx3q;
           pres[o] = c_pres + p0 - be * (d11 + d22 + d33);
         }
@@ -2153,19 +2171,26 @@ template <typename TW> void launch_project(vrh_t *h, int irk) {
   const double adt = h->rk[irk].a * h->dt;
   const double be = 0.5 * (h->rk[irk].a * h->dt) / h->Re;
   // Planes per block: 8 (a block re-reads three planes of phi, 2 % of its
-  // bytes; its waves' first loads are exposed once per chunk).  us at 4, 8, 16, 32 planes:
-  // 128x256x512 411, 387, 391, 412; 129x128x128 80, 77, 87, 88;
-  // 32x64x128 19, 21, 27, 45.  4 where 8 leaves fewer than 2 blocks per CU.
-  // Up to 32 angles a tile of 32 x 8 idles no lanes (32x64x128: 15.5 us
-  // with 4 planes).
-  const int W = g.nt <= 32 ? 32 : 64, R = 256 / W;
-  const long cols = (long)((g.nt + W - 1) / W) * ((g.nrc + 1 + R - 1) / R);
-  const int kchunk = cols * ((g.nzc + 7) / 8) < 512 ? 4 : 8;
+  // bytes; its waves' first loads are exposed once per chunk), 4 up to 20 MB
+  // a component, where 8 leave too few blocks.  us at 8 and 4 planes:
+  // 32x64x128 18.4, 16.0; 64x128x256 60.0, 58.1 (tanh mesh 69, 63);
+  // 129x128x128 79.6, 77.5; 200x96x160 92.1, 94.7; 128x192x256 149.1, 150.8;
+  // 128x256x512 388, 406.
+  // Tiles of 32 x 8 where they idle fewer lanes, up to 32 and from 65 to 96
+  // angles: 64 x 4 against 32 x 8 take 18.8 and 16.0 at 32x64x128, 48.4 and
+  // 44.4 at 96x64x256, but 73 and 82 at 129x128x128 and 65 and 72 at 100x96x200.
+  const int W = g.nt <= 32 || (g.nt > 64 && g.nt <= 96) ? 32 : 64, R = 256 / W;
+  const int kchunk = (long)sizeof(double) * g.ncomp <= (20L << 20) ? 4 : 8;
+  // Neighbouring tiles on one XCD where rows are not whole 64-byte pieces, so
+  // that the pieces two tiles share are joined in one L2: 77.5 -> 72.1 us at
+  // 129x128x128, 65.2 -> 62.3 at 100x96x200, 225 -> 213 at 255x128x256.  Whole
+  // pieces are better spread over all XCDs: 66.4 against 69.9 at 144x96x160.
+  const int xcd = g.nt % 8 != 0;
   dim3 blk(W, R), grd((g.nt + W - 1) / W, (g.nrc + 1 + R - 1) / R, (g.nzc + kchunk - 1) / kchunk);
   KTimer kt(h, KT_PROJECT);
   auto kern = W == 64 ? (h->zmet.m3 ? k_project<64, 4, true> : k_project<64, 4, false>)
                       : (h->zmet.m3 ? k_project<32, 8, true> : k_project<32, 8, false>);
-  hipLaunchKernelGGL(kern, grd, blk, 0, h->stream, g, h->coef, h->zmet, adt, be, kchunk, h->f.dph, h->f.dq1,
+  hipLaunchKernelGGL(kern, grd, blk, 0, h->stream, g, h->coef, h->zmet, adt, be, kchunk, xcd, h->f.dph, h->f.dq1,
                      h->f.dq2, h->f.dq3, h->f.q1, h->f.q2, h->f.q3, h->f.prg1, h->f.prg2,
                      h->f.prg3, h->f.pres, h->f.flag);
 }
