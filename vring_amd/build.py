@@ -7,7 +7,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libvrh.so")
-SOURCES = ["vrh_api.cpp", "vrh_host.cpp", "vrh_kernels.hip", "vrh_lines.hip", "vrh_dense.hip", "vrh_particles.hip", "vrh_learn.hip"]
+SOURCES = ["vrh_api.cpp", "vrh_host.cpp", "vrh_copy.cpp", "vrh_kernels.hip", "vrh_lines.hip", "vrh_dense.hip", "vrh_particles.hip", "vrh_learn.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17",
          # packed FP32 instructions are disabled for all device code

@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "vrh.h"
+#include "vrh_copy.h"
 #include "vrh_learn.h"
 
 #define VRH_HD __host__ __device__ __forceinline__
@@ -271,6 +272,8 @@ struct vrh_s {
   // stream while stepping continues
   double *d_snap = nullptr, *h_snap = nullptr;
   double *d_anl = nullptr;  // vrh_analysis block partials and result (first use)
+  HostCopy down;            // staging of large downloads
+  double *d_poi = nullptr;  // vrh_poisson_solve's right-hand side and solution (first use)
   hipStream_t copy_stream = nullptr;
   hipEvent_t snap_ev = nullptr;
   bool snap_pending = false;

@@ -1080,6 +1080,7 @@ struct vrh_hz_s {
   int nr = 0, nz = 0, S = 0, pool = 1;
   double rmax = 0, zmax = 0, stretch = 0, dr = 0;
   hipStream_t stream = nullptr;
+  HostCopy down;  // staging of large downloads
   rocblas_handle blas = nullptr;
   std::string err;
   std::vector<double> zf, zm, dz, rm;
@@ -1150,8 +1151,7 @@ int upload_host(vrh_hz_t *h, double *d, const double *src) {
   return 0;
 }
 int download_host(vrh_hz_t *h, double *dst, const double *d) {
-  HZCHK(h, hipMemcpyAsync(dst, d, h->ncell() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-  HZCHK(h, hipStreamSynchronize(h->stream));
+  HZCHK(h, host_download(h->down, h->stream, dst, d, h->ncell() * sizeof(double)));
   return 0;
 }
 
@@ -1734,6 +1734,7 @@ int vrh_hz_destroy(vrh_hz_t *h) {
                   h->d_g4, h->d_gt[0], h->d_gt[1], h->d_out, h->d_loss, h->d_dwpart};
   for (void *p : ptrs) if (p) (void)hipFree(p);
   for (double *v : h->vec) if (v) (void)hipFree(v);
+  host_copy_free(h->down);
   if (h->blas) rocblas_destroy_handle(h->blas);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;

@@ -877,14 +877,14 @@ int vrh_particles_download(vrh_t *h, int batch, long n, double *u, int *alive) {
   if (rc) return rc;
   // rows in the shown order, formed on the device (physical slot p holds shown
   // slot slot[p], a permutation of [0, cap)): 10^6 trilinear particles took
-  // 28 ms with the arrays copied down and scattered by the host, now 5 (2 of
-  // them the first touch of fresh host pages)
+  // 28 ms with the arrays copied down and scattered by the host, 5 with one
+  // copy of the rows, 2.1 with the staged one
   int *bad = B.lflag, hbad = 0;
   (void)hipMemsetAsync(bad, 0, sizeof(int), h->stream);
   hipLaunchKernelGGL(k_rows_out, dim3((unsigned)((B.cap + 63) / 64)), dim3(256), 0, h->stream, B.u, B.alive, B.slot,
                      B.cap, n, nvar, B.u_tmp, B.alive_tmp, bad);
   if (hipGetLastError() != hipSuccess ||
-      (n > 0 && hipMemcpyAsync(u, B.u_tmp, sizeof(double) * nvar * n, hipMemcpyDeviceToHost, h->stream) != hipSuccess) ||
+      (n > 0 && host_download(h->down, h->stream, u, B.u_tmp, sizeof(double) * nvar * n) != hipSuccess) ||
       (n > 0 && alive &&
        hipMemcpyAsync(alive, B.alive_tmp, sizeof(int) * n, hipMemcpyDeviceToHost, h->stream) != hipSuccess) ||
       hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, h->stream) != hipSuccess ||
