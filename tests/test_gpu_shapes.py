@@ -72,3 +72,23 @@ def test_whole_steps_grouped_and_single(nt, nr, nz, M, precision):
     s.step(5)
     vscale = max(np.abs(o.field("q2")).max(), np.abs(o.field("q3")).max())
     compare(o, s, ["q1", "q2", "q3"], 1e-10 if precision == "fp64" else 1e-6, scale=vscale)
+
+
+# a chosen z tile width runs the mixed path's FP64 low modes by themselves
+@pytest.mark.parametrize("nt,nr,nz", [(8, 15, 16), (32, 64, 128), (16, 17, 64), (9, 33, 40), (4, 256, 33), (64, 40, 512),
+                                      (16, 12, 1024), (8, 257, 32)])
+def test_mixed_modes_in_one_launch_and_apart_agree(nt, nr, nz):
+    """Bit for bit: the same sums, whichever launch they are in."""
+    print(f"case mixed modes {nt}x{nr}x{nz}", flush=True)
+    q1, q2, q3 = vring_amd.ring_initial_condition(nt, nr, nz, 4.0, 12.0, [(1.0, 3.0, 0.4, 1.0)])
+    dt = vring_amd.cfl_dt(nt, nr, nz, 4.0, 12.0, q1, q2, q3, cfl=0.3, ujet=1.0)
+    got = []
+    for lines in (0, 16):
+        s = vring_amd.Solver(nt, nr, nz, 4.0, 12.0, 500.0, dt, precision="mixed")
+        s.set_tuning(dct_lines=lines)
+        for n, a in (("q1", q1), ("q2", q2), ("q3", q3)):
+            s.upload(n, a)
+        s.step(3)
+        got.append([s.download(n) for n in ("q1", "q2", "q3", "pres")])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)

@@ -39,12 +39,12 @@ constexpr int kGrp = 8;
 // 18 us a transform, where a direct sum with a cosine per term took 460.
 // ---------------------------------------------------------------------------
 template <typename TW, int NT>
-__global__ __launch_bounds__(512) void k_zdense(TW *__restrict__ S, long nl, int n, DenseMat m, double div) {
-  extern __shared__ double x[];
+__device__ __forceinline__ void zdense_block(unsigned blk, double *x, TW *__restrict__ S, long nl, int n, const DenseMat &m,
+                                             double div) {
   constexpr int TN = 16 * NT, NTH = 512, RS = NTH / TN;  // RS rows per pass of the block
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const long l0 = (long)blockIdx.x * TN;
+  const long l0 = (long)blk * TN;
   {
     const int c = tid % TN, r0 = tid / TN;
     const TW *src = S + min(l0 + c, nl - 1);
@@ -95,6 +95,20 @@ __global__ __launch_bounds__(512) void k_zdense(TW *__restrict__ S, long nl, int
       }
     }
   }
+}
+
+template <typename TW, int NT>
+__global__ __launch_bounds__(512) void k_zdense(TW *__restrict__ S, long nl, int n, DenseMat m, double div) {
+  extern __shared__ double x[];
+  zdense_block<TW, NT>(blockIdx.x, x, S, nl, n, m, div);
+}
+// the mixed path's FP64 low modes (first na blocks) and its FP32 lines
+template <int NT>
+__global__ __launch_bounds__(512) void k_zdense2(double *__restrict__ S64, long nl64, unsigned na, float *__restrict__ S,
+                                                 long nl, int n, DenseMat m, double div) {
+  extern __shared__ double x[];
+  if (blockIdx.x < na) zdense_block<double, 1>(blockIdx.x, x, S64, nl64, n, m, div);
+  else zdense_block<float, NT>(blockIdx.x - na, x, S, nl, n, m, div);
 }
 
 // ---------------------------------------------------------------------------
@@ -470,6 +484,17 @@ template <typename TW> void launch_zdense(vrh_t *h, hipStream_t st, TW *S, long 
   else hipLaunchKernelGGL((k_zdense<TW, 1>), grd, blk, sh, st, S, nl, n, m, div);
 }
 
+// cosine transforms of the mixed path's low modes and of its FP32 lines
+void launch_zdense2(vrh_t *h, double *S64, long nl64, float *S, long nl, int dir) {
+  const DenseMat &m = h->zdct[dir > 0 ? 0 : 1];
+  const int n = h->nz, nt = nl >= 32 * 256 && n <= 320 ? 2 : 1;
+  const double div = dir > 0 ? (double)n : 1.0;
+  const unsigned na = (unsigned)((nl64 + 15) / 16), nb = (unsigned)((nl + 16 * nt - 1) / (16 * nt));
+  const size_t sh = sizeof(double) * 16 * nt * (size_t)n;
+  if (nt == 2) hipLaunchKernelGGL(k_zdense2<2>, dim3(na + nb), dim3(512), sh, h->stream, S64, nl64, na, S, nl, n, m, div);
+  else hipLaunchKernelGGL(k_zdense2<1>, dim3(na + nb), dim3(512), sh, h->stream, S64, nl64, na, S, nl, n, m, div);
+}
+
 template <typename TW>
 void launch_divdft(vrh_t *h, double inv_adt, const double *ext, TW *S, double *S64) {
   const VGrid &g = h->g;
@@ -495,6 +520,7 @@ size_t dense_lds_need(int nt, int nz) {
 bool dense_lds_optin(int bytes) {
   const void *fns[] = {reinterpret_cast<const void *>(&k_zdense<double, 1>), reinterpret_cast<const void *>(&k_zdense<double, 2>),
                        reinterpret_cast<const void *>(&k_zdense<float, 1>), reinterpret_cast<const void *>(&k_zdense<float, 2>),
+                       reinterpret_cast<const void *>(&k_zdense2<1>), reinterpret_cast<const void *>(&k_zdense2<2>),
                        reinterpret_cast<const void *>(&k_divdft<double>), reinterpret_cast<const void *>(&k_divdft<float>),
                        reinterpret_cast<const void *>(&k_idft<double>), reinterpret_cast<const void *>(&k_idft<float>)};
   for (const void *f : fns)

@@ -340,6 +340,7 @@ int dense_axial(vrh_t *h, const std::vector<double> &vi, const std::vector<doubl
 size_t dense_lds_need(int nt, int nz);
 bool dense_lds_optin(int bytes);
 template <typename TW> void launch_zdense(vrh_t *h, hipStream_t st, TW *S, long nl, int dir);
+void launch_zdense2(vrh_t *h, double *S64, long nl64, float *S, long nl, int dir);
 template <typename TW> void launch_divdft(vrh_t *h, double inv_adt, const double *ext, TW *S, double *S64);
 template <typename TW> void launch_idft(vrh_t *h, const TW *S, const double *S64, double *phi_out, double *dph);
 template <typename TW> void launch_project(vrh_t *h, int irk);

@@ -1168,9 +1168,10 @@ __global__ __launch_bounds__(256) void k_divfft(VGrid g, VCoef c, ZMet zm, doubl
 // loading while the other transforms (us forward/inverse, without and with:
 // 256x512x1024 758/749, 482/456; 128x256x512 54/49, 50/48).
 template <typename TW>
-__global__ __launch_bounds__(1024, sizeof(TW) == 4 ? 8 : 1) void k_dctz(TW *__restrict__ S, long nl, int n, int logn, int TL, int logtl, int dir,
-                                              const double *__restrict__ twr, const double *__restrict__ twi,
-                                              const double *__restrict__ er, const double *__restrict__ ei) {
+__device__ __forceinline__ void dctz_block(unsigned blk, unsigned nblk, TW *__restrict__ S, long nl, int n, int logn, int TL,
+                                           int logtl, int dir, const double *__restrict__ twr,
+                                           const double *__restrict__ twi, const double *__restrict__ er,
+                                           const double *__restrict__ ei) {
   extern __shared__ unsigned char smem_raw[];
   TW *re = reinterpret_cast<TW *>(smem_raw);
   // sequences at stride n + 1 in LDS: the line-to-sequence transposes
@@ -1187,7 +1188,7 @@ __global__ __launch_bounds__(1024, sizeof(TW) == 4 ? 8 : 1) void k_dctz(TW *__re
   auto ecos = [&](int k) { return lds_tw ? etw[k] : (TW)er[k]; };
   auto esin = [&](int k) { return lds_tw ? etw[n + k] : (TW)ei[k]; };
   const int tid = threadIdx.x, nth = blockDim.x;
-  const long l0 = xcd_tile(blockIdx.x, gridDim.x) * TL;
+  const long l0 = xcd_tile(blk, nblk) * TL;
   for (int q = tid; q < n / 2; q += nth) { twl[q] = (TW)twr[q]; twl[n / 2 + q] = (TW)twi[q]; }
   if (lds_tw)
     for (int q = tid; q < n; q += nth) { etw[q] = (TW)er[q]; etw[n + q] = (TW)ei[q]; }
@@ -1272,19 +1273,45 @@ __global__ __launch_bounds__(1024, sizeof(TW) == 4 ? 8 : 1) void k_dctz(TW *__re
   }
 }
 
+struct DctzTab { const double *twr, *twi, *er, *ei; };
+template <typename TW> struct DctzLines {
+  TW *S;
+  long nl;
+  int TL, logtl;
+  unsigned nb;  // blocks
+};
+template <typename TW>
+__global__ __launch_bounds__(1024, sizeof(TW) == 4 ? 8 : 1) void k_dctz(DctzLines<TW> a, DctzTab t, int n, int logn, int dir) {
+  dctz_block<TW>(blockIdx.x, a.nb, a.S, a.nl, n, logn, a.TL, a.logtl, dir, t.twr, t.twi, t.er, t.ei);
+}
+// the mixed path's FP64 low modes (first blocks) and its FP32 lines
+__global__ __launch_bounds__(1024) void k_dctz2(DctzLines<double> a, DctzLines<float> b, DctzTab t, int n, int logn, int dir) {
+  if (blockIdx.x < a.nb) dctz_block<double>(blockIdx.x, a.nb, a.S, a.nl, n, logn, a.TL, a.logtl, dir, t.twr, t.twi, t.er, t.ei);
+  else dctz_block<float>(blockIdx.x - a.nb, b.nb, b.S, b.nl, n, logn, b.TL, b.logtl, dir, t.twr, t.twi, t.er, t.ei);
+}
+
 // Radial tridiagonal solves of every (mode, kz) system (solve_radial,
 // poisson_solve.F90:270-323) with precomputed inverse pivots ib; lanes over
 // the packed mode index (contiguous), P waves of M rows each.
 // FP32: at most 64 VGPRs, so that two 1024-lane blocks share a CU.
 template <typename T, int M>
-__global__ __launch_bounds__(1024, sizeof(T) == 4 ? 8 : 1) void k_radial(T *__restrict__ S, const T *__restrict__ ib, long nm, long nlines,
-                                                 int nr, const T *__restrict__ aab, const T *__restrict__ ccb) {
-  __shared__ T sh_v[16][64];
-  __shared__ T sh_p[16][64];
+__device__ __forceinline__ void radial_block(unsigned blk, T (&sh_v)[16][64], T (&sh_p)[16][64], T *__restrict__ S,
+                                             const T *__restrict__ ib, long nm, long nlines, int nr,
+                                             const T *__restrict__ aab, const T *__restrict__ ccb) {
+  // 16 rows a wave (the body of two kernels): the sums are rounded the one way
+  // in both, fused or not as written
+  auto fma_t = [](T x, T y, T z) {
+    if constexpr (sizeof(T) == 4) return __builtin_fmaf(x, y, z); else return __builtin_fma(x, y, z);
+  };
+  auto add_t = [](T z, T x, T y) {
+#pragma clang fp contract(off)
+    const T p = x * y;
+    return z + p;
+  };
   const int lane = threadIdx.x & 63;
   const int s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int P = blockDim.x >> 6;
-  const long L = (long)blockIdx.x * 64 + lane;
+  const long L = (long)blk * 64 + lane;
   const bool act = L < nlines;
   const long Lc = act ? L : nlines - 1;  // addresses stay in bounds; results of !act lanes are dropped
   const long pos = Lc % nm, kz = Lc / nm;
@@ -1307,7 +1334,7 @@ __global__ __launch_bounds__(1024, sizeof(T) == 4 ? 8 : 1) void k_radial(T *__re
     const bool in = t < len;
     const T ibv = w[t];
     const T B = -aab[pc + 1] * ibv * (T)(p > 0);
-    const T v = ibv * x[t] + B * gp;
+    const T v = M == 16 ? fma_t(ibv, x[t], B * gp) : ibv * x[t] + B * gp;
     x[t] = in ? v : (T)0;
     gp = in ? v : gp;
     Pacc = in ? Pacc * B : Pacc;
@@ -1324,7 +1351,7 @@ __global__ __launch_bounds__(1024, sizeof(T) == 4 ? 8 : 1) void k_radial(T *__re
     const int p = p0 + t, pc = min(p, nr - 1);
     const bool in = t < len;
     Pr = in ? Pr * (-aab[pc + 1] * w[t] * (T)(p > 0)) : Pr;
-    x[t] = in ? x[t] + Pr * G : x[t];
+    x[t] = !in ? x[t] : M > 16 ? x[t] + Pr * G : t < M - 1 ? add_t(x[t], Pr, G) : fma_t(Pr, G, x[t]);
   }
   T xp = (T)0, Qacc = (T)1;
 #pragma unroll
@@ -1352,6 +1379,30 @@ __global__ __launch_bounds__(1024, sizeof(T) == 4 ? 8 : 1) void k_radial(T *__re
       S[base + nm * p] = x[t] + Qr * X;
     }
   }
+}
+
+template <typename T> struct RadialLines {
+  T *S;
+  const T *ib, *aab, *ccb;
+  long nm, nlines;
+};
+template <typename T, int M>
+__global__ __launch_bounds__(1024, sizeof(T) == 4 ? 8 : 1) void k_radial(RadialLines<T> a, int nr) {
+  __shared__ T sh_v[16][64];
+  __shared__ T sh_p[16][64];
+  radial_block<T, M>(blockIdx.x, sh_v, sh_p, a.S, a.ib, a.nm, a.nlines, nr, a.aab, a.ccb);
+}
+// the mixed path's FP64 low modes (first blocks) and its FP32 lines, up to 256
+// rows
+__global__ __launch_bounds__(1024) void k_radial2(RadialLines<double> a, RadialLines<float> b, int nr) {
+  __shared__ double sh_v[16][64];
+  __shared__ double sh_p[16][64];
+  const unsigned na = (unsigned)((a.nlines + 63) / 64);
+  if (blockIdx.x < na)
+    radial_block<double, 16>(blockIdx.x, sh_v, sh_p, a.S, a.ib, a.nm, a.nlines, nr, a.aab, a.ccb);
+  else
+    radial_block<float, 16>(blockIdx.x - na, reinterpret_cast<float(&)[16][64]>(sh_v),
+                           reinterpret_cast<float(&)[16][64]>(sh_p), b.S, b.ib, b.nm, b.nlines, nr, b.aab, b.ccb);
 }
 
 // fft_ftp_multi (fastfouriertransform.F90:74-82) + copy into dph
@@ -1951,25 +2002,36 @@ void lds_optin(vrh_t *h) {
 
 static int ilog2(int n) { int l = 0; while ((1 << l) < n) ++l; return l; }
 
+// rows per wave of the radial solves: 16 keeps the segment's rhs and pivots
+// in registers (a 1024-lane block allows 128 VGPRs) up to nr = 256; 32 beyond
+// (P <= 16)
+static int radial_rows(const VGrid &g) { return g.nr <= 256 ? 16 : 32; }
+// the radial base coefficients in the solve's type (float copies rounded as
+// the device conversion)
+static RadialLines<double> radial_lines(vrh_t *h, double *S, const double *ib, long nm) {
+  return {S, ib, h->d_aab, h->d_ccb, nm, nm * h->g.nz};
+}
+static RadialLines<float> radial_lines(vrh_t *h, float *S, const float *ib, long nm) {
+  return {S, ib, h->d_aabf, h->d_ccbf, nm, nm * h->g.nz};
+}
 template <typename T>
 static void radial_launch(vrh_t *h, T *S, const T *ib, long nm, hipStream_t st) {
   const VGrid &g = h->g;
-  // rows per wave: 16 keeps the segment's rhs and pivots in registers (a
-  // 1024-lane block allows 128 VGPRs) up to nr = 256; 32 beyond (P <= 16)
-  const int M = g.nr <= 256 ? 16 : 32;
-  const int P = (g.nr + M - 1) / M;
-  const long nlines = nm * g.nz;
-  dim3 blk(64 * P), grd((unsigned)((nlines + 63) / 64));
-  // the radial base coefficients in the solve's type (float copies rounded
-  // as the device conversion)
-  const T *ra, *rc;
-  if constexpr (sizeof(T) == 4) { ra = h->d_aabf; rc = h->d_ccbf; }
-  else { ra = h->d_aab; rc = h->d_ccb; }
+  const int M = radial_rows(g), P = (g.nr + M - 1) / M;
+  const RadialLines<T> a = radial_lines(h, S, ib, nm);
+  dim3 blk(64 * P), grd((unsigned)((a.nlines + 63) / 64));
   KTimer kt(h, KT_RADIAL);
-  if (M == 16)
-    hipLaunchKernelGGL((k_radial<T, 16>), grd, blk, 0, st, S, ib, nm, nlines, g.nr, ra, rc);
-  else
-    hipLaunchKernelGGL((k_radial<T, 32>), grd, blk, 0, st, S, ib, nm, nlines, g.nr, ra, rc);
+  if (M == 16) hipLaunchKernelGGL((k_radial<T, 16>), grd, blk, 0, st, a, g.nr);
+  else hipLaunchKernelGGL((k_radial<T, 32>), grd, blk, 0, st, a, g.nr);
+}
+static void radial_launch2(vrh_t *h, double *S64, const double *ib64, float *S, const float *ib) {
+  const VGrid &g = h->g;
+  const int P = (g.nr + 15) / 16;
+  const RadialLines<double> a = radial_lines(h, S64, ib64, 5);
+  const RadialLines<float> b = radial_lines(h, S, ib, g.nt);
+  dim3 blk(64 * P), grd((unsigned)((a.nlines + 63) / 64 + (b.nlines + 63) / 64));
+  KTimer kt(h, KT_RADIAL);
+  hipLaunchKernelGGL(k_radial2, grd, blk, 0, h->stream, a, b, g.nr);
 }
 
 // z transform of the mixed path's pressure solve on an axial mesh (FP64 path:
@@ -2047,16 +2109,13 @@ __global__ __launch_bounds__(256) void k_hz_scatter(const double *__restrict__ x
   }
 }
 
-// One z transform of the pressure solve, in place on nl lines: the cosine
-// transform by FFT (nz a power of two) or as a dense product, or on an axial
-// mesh the product with its eigenvectors.
-template <typename T> static void z_transform(vrh_t *h, hipStream_t st, T *S, long nl, int dir, int want) {
+// shape of a cosine transform by FFT: a power of two of lines per block, data
+// + twiddles within 64 KB of LDS (a tuned width may take the device's larger
+// per-block LDS: 32 FP32 lines read whole 128-byte rows of the strided
+// layout), one FFT butterfly per thread with up to 1024 threads
+struct DctzShape { int tl, nth; size_t sh; };
+template <typename T> static DctzShape dctz_shape(vrh_t *h, int want) {
   const int nz = h->g.nz, lz = ilog2(nz);
-  if (h->zmet.m3 || (nz & (nz - 1)) != 0) { launch_zdense<T>(h, st, S, nl, dir); return; }
-  // lines per block: a power of two, data + twiddles within 64 KB of LDS
-  // (a tuned width may take the device's larger per-block LDS: 32 FP32
-  // lines read whole 128-byte rows of the strided layout), one FFT
-  // butterfly per thread with up to 1024 threads
   const size_t es = sizeof(T), lim = want > 0 ? (size_t)h->lds_block : 65536;
   const int tmax = want > 0 ? 32 : 16;
   int tl = 2;
@@ -2066,9 +2125,32 @@ template <typename T> static void z_transform(vrh_t *h, hipStream_t st, T *S, lo
   if (want > 0) while (tl > 2 && tl > want) tl /= 2;
   const int b = (tl / 2) * nz / fft_min_radix(lz), nth = b > 512 ? 1024 : b > 256 ? 512 : 256;
   // tile lines, FFT twiddles, and in FP32 the Makhoul twiddles
-  const size_t sh = es * ((size_t)tl * (nz + 1) + (size_t)(es == 4 ? 3 : 1) * nz);
-  hipLaunchKernelGGL(k_dctz<T>, dim3((unsigned)((nl + tl - 1) / tl)), dim3(nth), sh, st, S, nl, nz, lz, tl, ilog2(tl),
-                     dir, h->d_twz, h->d_twz + nz, h->d_ez, h->d_ez + nz);
+  return {tl, nth, es * ((size_t)tl * (nz + 1) + (size_t)(es == 4 ? 3 : 1) * nz)};
+}
+template <typename T> static DctzLines<T> dctz_lines(const DctzShape &p, T *S, long nl) {
+  return {S, nl, p.tl, ilog2(p.tl), (unsigned)((nl + p.tl - 1) / p.tl)};
+}
+
+// One z transform of the pressure solve, in place on nl lines: the cosine
+// transform by FFT (nz a power of two) or as a dense product, or on an axial
+// mesh the product with its eigenvectors.
+template <typename T> static void z_transform(vrh_t *h, hipStream_t st, T *S, long nl, int dir, int want) {
+  const int nz = h->g.nz, lz = ilog2(nz);
+  if (h->zmet.m3 || (nz & (nz - 1)) != 0) { launch_zdense<T>(h, st, S, nl, dir); return; }
+  const DctzShape p = dctz_shape<T>(h, want);
+  const DctzLines<T> a = dctz_lines(p, S, nl);
+  hipLaunchKernelGGL(k_dctz<T>, dim3(a.nb), dim3(p.nth), p.sh, st, a, DctzTab{h->d_twz, h->d_twz + nz, h->d_ez, h->d_ez + nz},
+                     nz, lz, dir);
+}
+// that of the mixed path's FP64 low modes and FP32 lines in one launch
+static void z_transform2(vrh_t *h, double *S64, long nl64, float *S, long nl, int dir) {
+  const int nz = h->g.nz, lz = ilog2(nz);
+  if ((nz & (nz - 1)) != 0) { launch_zdense2(h, S64, nl64, S, nl, dir); return; }
+  const DctzShape p = dctz_shape<double>(h, 0), q = dctz_shape<float>(h, h->dct_lines);
+  const DctzLines<double> a = dctz_lines(p, S64, nl64);
+  const DctzLines<float> b = dctz_lines(q, S, nl);
+  hipLaunchKernelGGL(k_dctz2, dim3(a.nb + b.nb), dim3(std::max(p.nth, q.nth)), std::max(p.sh, q.sh), h->stream, a, b,
+                     DctzTab{h->d_twz, h->d_twz + nz, h->d_ez, h->d_ez + nz}, nz, lz, dir);
 }
 
 template <typename TW> void launch_poisson(vrh_t *h, int irk, const double *ext_rhs, double *phi_out) {
@@ -2107,7 +2189,15 @@ template <typename TW> void launch_poisson(vrh_t *h, int irk, const double *ext_
   // a side stream, forked and joined between them, beside the FP32
   // transforms.  With the kernel timer on, or inside an ensemble graph, it
   // stays in order on the handle's stream.
-  const bool par = S64 && !h->kt_on && !h->serial_sweeps;
+  // On grids of up to 14 MB a component (FP32) and 256 rows the two chains
+  // share launches instead: three kernels instead of six with a fork and a
+  // join, whose gaps took 14 us of a substep.  us a step, side by side ->
+  // shared: 32x64x128 307 -> 267, 33x96x200 524 -> 477, 64x96x256 551 -> 521,
+  // 100x128x200 1245 -> 1205, 64x128x400 1459 -> 1435, 64x192x256 even; the
+  // FP32 lines then run with the FP64 kernel's registers, and 128x192x256
+  // (25 MB) took 1642 instead of 1625.
+  const bool pair = S64 && !h->zmet.m3 && radial_rows(g) == 16 && h->dct_lines <= 0 && 4 * g.ncomp <= 14L << 20;
+  const bool par = S64 && !pair && !h->kt_on && !h->serial_sweeps;
   hipStream_t s64 = par ? h->side[0] : h->stream;
   const int ie = (irk >= 1 && irk <= 3) ? irk : 0;
   if (par) {
@@ -2118,7 +2208,7 @@ template <typename TW> void launch_poisson(vrh_t *h, int irk, const double *ext_
     zgemm(h, s64, S64, h->S2_64, nl64, 1);
     radial_launch<double>(h, h->S2_64, h->f.ib64, 5, s64);
     zgemm(h, s64, h->S2_64, S64, nl64, -1);
-  } else if (S64) {
+  } else if (S64 && !pair) {
     z_transform<double>(h, s64, S64, nl64, 1, 0);
     radial_launch<double>(h, S64, h->f.ib64, 5, s64);
     z_transform<double>(h, s64, S64, nl64, -1, 0);
@@ -2136,6 +2226,11 @@ template <typename TW> void launch_poisson(vrh_t *h, int irk, const double *ext_
       { KTimer kt(h, KT_DCT_FWD); zgemm(h, h->stream, S, S2, nl, 1); }
       radial_launch<TW>(h, S2, (const TW *)h->f.ib, N, h->stream);
       { KTimer kt(h, KT_DCT_INV); zgemm(h, h->stream, S2, S, nl, -1); }
+      done = true;
+    } else if (pair) {
+      { KTimer kt(h, KT_DCT_FWD); z_transform2(h, S64, nl64, S, nl, 1); }
+      radial_launch2(h, S64, h->f.ib64, S, (const TW *)h->f.ib);
+      { KTimer kt(h, KT_DCT_INV); z_transform2(h, S64, nl64, S, nl, -1); }
       done = true;
     }
   }
