@@ -250,7 +250,7 @@ __global__ __launch_bounds__(kThThreads) void k_divdft(VGrid g, VCoef c, ZMet zm
 // ---------------------------------------------------------------------------
 // fft_ftp_multi (fastfouriertransform.F90:74-82), the copy into dph
 // (poisson_solve.F90:29) and dph(nzc) = dph(nz) (divergence.F90:93-99) for
-// ntheta no power of two.  One lane per line (64 lines per block in LDS, odd
+// ntheta no power of two, mixed path.  One lane per line (64 lines per block in LDS, odd
 // stride), kIdT angles per wave at a time: a coefficient pair read from LDS
 // serves kIdT angles, and the cosines and sines, the same for all lanes, come
 // as scalar loads from a table in their order of use.  A term is
@@ -267,8 +267,7 @@ __device__ __forceinline__ double id_term(double v, double a, double c, double b
 
 constexpr int kIdLines = 64, kIdT = 4, kIdWaves = 16;
 
-template <typename TW>
-__global__ __launch_bounds__(64 * kIdWaves) void k_idft(VGrid g, const TW *__restrict__ S,
+__global__ __launch_bounds__(64 * kIdWaves) void k_idft(VGrid g, const float *__restrict__ S,
                                                         const double *__restrict__ S64, double *__restrict__ phi_out,
                                                         double *__restrict__ dph, const double *__restrict__ tab) {
   extern __shared__ double x[];
@@ -279,12 +278,12 @@ __global__ __launch_bounds__(64 * kIdWaves) void k_idft(VGrid g, const TW *__res
   constexpr int NTH = 64 * kIdWaves;
   {
     // the block's lines are contiguous in S; (line, position) advances by NTH
-    const TW *src = S + (size_t)N * l0;
+    const float *src = S + (size_t)N * l0;
     const int dl = NTH / N, dp = NTH - dl * N;
     constexpr int U = 8;
     int lp = tid / N, pos = tid - lp * N;
     for (int eb = tid; eb < tot; eb += U * NTH) {
-      TW v[U];
+      float v[U];
 #pragma unroll
       for (int u = 0; u < U; u++) v[u] = src[min(eb + u * NTH, tot - 1)];
       __builtin_amdgcn_sched_barrier(0);
@@ -349,6 +348,96 @@ __global__ __launch_bounds__(64 * kIdWaves) void k_idft(VGrid g, const TW *__res
   __syncthreads();
   // a wave per line
   for (int lp = wave; lp < nln; lp += kIdWaves) {
+    const long l = l0 + lp;
+    const int j = (int)(l % g.nr) + 1, k = (int)(l / g.nr) + 1;
+    for (int ii = lane; ii < N; ii += 64) {
+      const double y = x[lp * ldn + ii];
+      if (phi_out) phi_out[cidx(g, ii + 1, j, k)] = y;
+      if (dph) {
+        dph[hidx(g, ii + 1, j, k)] = y;
+        if (k == g.nz) dph[hidx(g, ii + 1, j, g.nzc)] = y;
+      }
+    }
+  }
+}
+
+// The same for the FP64 path, as a product with the matrix of the cosines and
+// sines on the matrix cores: tiles and lines as in k_divdft.  129x128x128:
+// 30 us, 45 with the vector units above (whose order of terms the mixed
+// path's results hold to); 8 at the FP64 matrix rate, 7 at the copy rate.
+// Four partial sums a tile keep the products from waiting for each other and
+// the chains of roundings shorter than the vector units'.
+__global__ __launch_bounds__(kThThreads) void k_idft64(VGrid g, const double *__restrict__ S, double *__restrict__ phi_out,
+                                                       double *__restrict__ dph, DenseMat m) {
+  extern __shared__ double x[];
+  const int N = g.nt, ldn = N | 1, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const long nlines = (long)g.nr * g.nz, l0 = (long)blockIdx.x * kThLines;
+  const int nln = (int)min((long)kThLines, nlines - l0), tot = nln * N;
+  {
+    // the block's lines are contiguous in S; (line, position) advances by kThThreads
+    const double *src = S + (size_t)N * l0;
+    const int dl = kThThreads / N, dp = kThThreads - dl * N;
+    constexpr int U = 8;
+    int lp = tid / N, pos = tid - lp * N;
+    for (int eb = tid; eb < tot; eb += U * kThThreads) {
+      double v[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) v[u] = src[min(eb + u * kThThreads, tot - 1)];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        if (eb + u * kThThreads < tot) x[lp * ldn + pos] = v[u];
+        lp += dl;
+        pos += dp;
+        if (pos >= N) { pos -= N; lp++; }
+      }
+    }
+    // lines past the last one: zeros
+    for (int e = tot + tid; e < kThLines * N; e += kThThreads) x[(e / N) * ldn + e % N] = 0.0;
+  }
+  __syncthreads();
+  constexpr int TPW = 4;  // N < 256: at most 2 x 16 tiles on eight waves
+  d4 acc[TPW];
+  const int kq = lane >> 4;
+#pragma unroll
+  for (int u = 0; u < TPW; u++) {
+    d4 part[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) part[q] = d4{0.0, 0.0, 0.0, 0.0};
+    const int t = wave + kThWaves * u;  // angles of tile t / 2, lines of half t % 2
+    if (t >= 2 * m.mt) continue;
+    const double *ap = m.a + (size_t)(t >> 1) * m.ks * 64 + lane;
+    const double *xl = x + ((t & 1) * 16 + (lane & 15)) * ldn;
+    double cur[kGrp], nxt[kGrp];
+#pragma unroll
+    for (int s = 0; s < kGrp; s++) cur[s] = ap[s * 64];
+    for (int s0 = 0; s0 < m.ks; s0 += kGrp) {
+      const double *np = ap + min(s0 + kGrp, m.ks - kGrp) * 64;
+#pragma unroll
+      for (int s = 0; s < kGrp; s++) nxt[s] = np[s * 64];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < kGrp; s++)
+        part[s & 3] = __builtin_amdgcn_mfma_f64_16x16x4f64(cur[s], xl[min(4 * (s0 + s) + kq, N - 1)], part[s & 3], 0, 0, 0);
+#pragma unroll
+      for (int s = 0; s < kGrp; s++) cur[s] = nxt[s];
+    }
+    acc[u] = (part[0] + part[1]) + (part[2] + part[3]);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < TPW; u++) {
+    const int t = wave + kThWaves * u;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int i = (t >> 1) * 16 + 4 * v + kq;
+      if (i < N) x[((t & 1) * 16 + (lane & 15)) * ldn + i] = acc[u][v];
+    }
+  }
+  __syncthreads();
+  // a wave per line
+  for (int lp = wave; lp < nln; lp += kThWaves) {
     const long l = l0 + lp;
     const int j = (int)(l % g.nr) + 1, k = (int)(l / g.nr) + 1;
     for (int ii = lane; ii < N; ii += 64) {
@@ -439,6 +528,18 @@ int dense_create(vrh_t *h) {
       const int k = (pos + 1) / 2, ph = (int)(((long)k * i) % N);
       return pos == 0 || (pos & 1) ? cs[ph] : sn[ph];
     });
+    if (h->prec != VRH_MIXED) {
+      // inverse: row i, columns as the packed positions
+      size_t ai;
+      h->itdft = pack_dense(pk, ai, N, N, [&](int i, int pos) {
+        const int k = (pos + 1) / 2, ph = (int)(((long)k * i) % N);
+        return pos == 0 ? 1.0 : !(pos & 1) ? sn[ph] : 2 * k == N ? 0.5 * cs[ph] : cs[ph];
+      });
+      if ((rc = upload_pack(h, &h->d_tdft, pk))) return rc;
+      h->tdft.a = h->d_tdft + at;
+      h->itdft.a = h->d_tdft + ai;
+      return 0;
+    }
     // inverse: (cos, sin) of wavenumber kk at kIdT angles, tile by tile
     const size_t ti = pk.size();
     const int nk = N / 2;
@@ -507,8 +608,12 @@ template <typename TW>
 void launch_idft(vrh_t *h, const TW *S, const double *S64, double *phi_out, double *dph) {
   const VGrid &g = h->g;
   const long nlines = (long)g.nr * g.nz;
-  hipLaunchKernelGGL(k_idft<TW>, dim3((unsigned)((nlines + kIdLines - 1) / kIdLines)), dim3(64 * kIdWaves),
-                     sizeof(double) * kIdLines * (g.nt | 1), h->stream, g, S, S64, phi_out, dph, h->idft_tab);
+  if constexpr (sizeof(TW) == 8)
+    hipLaunchKernelGGL(k_idft64, dim3((unsigned)((nlines + kThLines - 1) / kThLines)), dim3(kThThreads),
+                       sizeof(double) * kThLines * (g.nt | 1), h->stream, g, S, phi_out, dph, h->itdft);
+  else
+    hipLaunchKernelGGL(k_idft, dim3((unsigned)((nlines + kIdLines - 1) / kIdLines)), dim3(64 * kIdWaves),
+                       sizeof(double) * kIdLines * (g.nt | 1), h->stream, g, S, S64, phi_out, dph, h->idft_tab);
 }
 
 // LDS that a grid's dense kernels need beyond the default limit, and their opt-in
@@ -522,7 +627,7 @@ bool dense_lds_optin(int bytes) {
                        reinterpret_cast<const void *>(&k_zdense<float, 1>), reinterpret_cast<const void *>(&k_zdense<float, 2>),
                        reinterpret_cast<const void *>(&k_zdense2<1>), reinterpret_cast<const void *>(&k_zdense2<2>),
                        reinterpret_cast<const void *>(&k_divdft<double>), reinterpret_cast<const void *>(&k_divdft<float>),
-                       reinterpret_cast<const void *>(&k_idft<double>), reinterpret_cast<const void *>(&k_idft<float>)};
+                       reinterpret_cast<const void *>(&k_idft64), reinterpret_cast<const void *>(&k_idft)};
   for (const void *f : fns)
     if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) return false;
   return true;

@@ -209,9 +209,9 @@ struct vrh_s {
   double *d_zeig = nullptr;
   DenseMat zeig[2] = {};  // [0] forward, [1] inverse
   // lengths that are no power of two: the z cosine matrices, the forward
-  // theta matrix and the inverse theta transform's table
+  // theta matrix and the inverse theta transform's (FP64) or its table (mixed)
   double *d_zcos = nullptr, *d_tdft = nullptr;
-  DenseMat zdct[2] = {}, tdft = {};
+  DenseMat zdct[2] = {}, tdft = {}, itdft = {};
   const double *idft_tab = nullptr;
   // per-mode iterative pressure solve (vrh_set_mode_solver): theta
   // positions pos >= hz_pos0 (modes m >= mmin) are solved by the Helmholtz
