@@ -92,3 +92,14 @@ def test_mixed_modes_in_one_launch_and_apart_agree(nt, nr, nz):
         got.append([s.download(n) for n in ("q1", "q2", "q3", "pres")])
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+def test_kernel_timer_times_the_kernels_alone():
+    """Nine r and z sweeps, three outlet rows and six radial solves a step, on
+    a grid whose untimed steps group them."""
+    s = vring_amd.Solver(16, 24, 32, 4.0, 12.0, 500.0, 0.01, precision="mixed")
+    s.step(1)
+    s.enable_ktimer(True)
+    s.step(2)
+    n = {k: cnt for k, (_, cnt) in s.kernel_times().items()}
+    assert (n["line_r"], n["line_z"], n["hdnbc"], n["radial"]) == (18, 18, 6, 12), n

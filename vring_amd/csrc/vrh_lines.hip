@@ -268,7 +268,6 @@ template <typename TW, int PHASE> void group_launch(vrh_t *h, SweepGroup &w, int
   w.b2 = w.b1 + nb(w.a[1]);
   w.b3 = w.b2 + nb(w.a[2]);
   const int hb = hdnbc ? (g.nt * g.nrc + 64 * P - 1) / (64 * P) : 0;
-  KTimer kt(h, PHASE == 0 ? KT_LINE_R : KT_LINE_Z);
   const dim3 grd((unsigned)(w.b3 + hb)), blk(64 * P);
   auto go = [&](auto *kern) { hipLaunchKernelGGL(kern, grd, blk, 0, h->stream, w); };
   if (mr == 16 && mz == 16) go(k_sweeps<TW, PHASE, 16, 16>);
@@ -312,7 +311,8 @@ template <typename TW> void launch_sweeps(vrh_t *h, int irk, double c3s, const d
   // at 128x128x192 mixed.  Beyond it the single sweeps' fewer registers (7
   // waves a SIMD against 4) win: 1021 -> 1052 at 96x96x200 FP64 (15 MB), 1183
   // -> 1224 at 129x128x128 FP64; 128x192x256 is even in both precisions.
-  if ((long)sizeof(TW) * g.ncomp <= (14L << 20) && h->Msw[SW_R3] == mr && h->Msw[SW_Z2] == mz && h->Msw[SW_Z3] == mz &&
+  // The kernel timer's entries are those of the kernels alone.
+  if (!h->kt_on && (long)sizeof(TW) * g.ncomp <= (14L << 20) && h->Msw[SW_R3] == mr && h->Msw[SW_Z2] == mz && h->Msw[SW_Z3] == mz &&
       group_has<TW>(mr, mz) && group_has<TW>(mr2, mz)) {
     SweepGroup w{s, {z2, r1, r3}, 0, 0, 0, hdnbc_args(h, irk, cor, cor_dev)};
     SweepGroup v{s, {z1, z3, r2}, 0, 0, 0, w.hd};
