@@ -1298,8 +1298,8 @@ template <typename T, int M>
 __device__ __forceinline__ void radial_block(unsigned blk, T (&sh_v)[16][64], T (&sh_p)[16][64], T *__restrict__ S,
                                              const T *__restrict__ ib, long nm, long nlines, int nr,
                                              const T *__restrict__ aab, const T *__restrict__ ccb) {
-  // 16 rows a wave (the body of two kernels): the sums are rounded the one way
-  // in both, fused or not as written
+  // the sums are rounded the one way in every kernel this is the body of,
+  // fused or not as written
   auto fma_t = [](T x, T y, T z) {
     if constexpr (sizeof(T) == 4) return __builtin_fmaf(x, y, z); else return __builtin_fma(x, y, z);
   };
@@ -1334,7 +1334,7 @@ __device__ __forceinline__ void radial_block(unsigned blk, T (&sh_v)[16][64], T 
     const bool in = t < len;
     const T ibv = w[t];
     const T B = -aab[pc + 1] * ibv * (T)(p > 0);
-    const T v = M == 16 ? fma_t(ibv, x[t], B * gp) : ibv * x[t] + B * gp;
+    const T v = fma_t(ibv, x[t], B * gp);
     x[t] = in ? v : (T)0;
     gp = in ? v : gp;
     Pacc = in ? Pacc * B : Pacc;
@@ -1351,7 +1351,7 @@ __device__ __forceinline__ void radial_block(unsigned blk, T (&sh_v)[16][64], T 
     const int p = p0 + t, pc = min(p, nr - 1);
     const bool in = t < len;
     Pr = in ? Pr * (-aab[pc + 1] * w[t] * (T)(p > 0)) : Pr;
-    x[t] = !in ? x[t] : M > 16 ? x[t] + Pr * G : t < M - 1 ? add_t(x[t], Pr, G) : fma_t(Pr, G, x[t]);
+    x[t] = !in ? x[t] : t < M - 1 ? add_t(x[t], Pr, G) : fma_t(Pr, G, x[t]);
   }
   T xp = (T)0, Qacc = (T)1;
 #pragma unroll
