@@ -59,3 +59,27 @@ def test_downloads_of_handles_in_threads():
     for t in th:
         t.join()
     assert not bad, bad
+
+
+def test_downloads_of_one_handle_in_threads():
+    nt, nr, nz = 64, 61, 270
+    print("case downloads of one handle in threads", flush=True)
+    s = vring_amd.Solver(nt, nr, nz, 4.0, 12.0, 1000.0, 0.01)
+    want = {n: np.random.default_rng(q).standard_normal((nt, nr + 3, nz + 3)) for q, n in enumerate(("q1", "q2", "q3"))}
+    for n, a in want.items():
+        s.upload(n, a)
+    bad = []
+
+    def work(n):
+        try:
+            for _ in range(4):
+                assert np.array_equal(s.download(n), want[n]), n
+        except BaseException as e:
+            bad.append(e)
+
+    th = [threading.Thread(target=work, args=(n,)) for n in want]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not bad, bad

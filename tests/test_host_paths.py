@@ -1,0 +1,61 @@
+"""The library's host code without a GPU: libvrh with a test double of the HIP
+runtime (hip_double.cpp) loaded before it, each case in a process of its own.
+Copies, events and streams behave; kernels are counted and compute nothing."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+PRELUDE = """
+import ctypes, os, threading
+import numpy as np
+dbl = ctypes.CDLL(os.environ["HIP_DOUBLE"])
+import vring_amd
+"""
+
+
+@pytest.fixture(scope="session")
+def double(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("hip") / "hip_double.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", f"-I{ROCM}/include",
+                    os.path.join(HERE, "hip_double.cpp"), "-o", so, "-lpthread"], check=True)
+    return so
+
+
+@pytest.fixture
+def run(double):
+    def go(body):
+        env = dict(os.environ)
+        env["HIP_DOUBLE"] = double
+        env["LD_PRELOAD"] = " ".join(filter(None, [double, env.get("LD_PRELOAD", "")]))
+        env["PYTHONPATH"] = os.pathsep.join(filter(None, [os.path.dirname(HERE), env.get("PYTHONPATH", "")]))
+        r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(body)], env=env, capture_output=True,
+                           text=True, timeout=120)
+        assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
+    return go
+
+
+def test_downloads_of_one_handle_in_threads(run):
+    """Two threads that fetch different fields of one idle handle each get
+    their own: results of 9 MB go through the handle's staging memory."""
+    run("""
+    nt, nr, nz = 64, 61, 270
+    s = vring_amd.Solver(nt, nr, nz, 4.0, 12.0, 1000.0, 0.01)
+    want = {n: np.random.default_rng(q).standard_normal((nt, nr + 3, nz + 3)) for q, n in enumerate(("q1", "q2", "q3"))}
+    for n, a in want.items():
+        s.upload(n, a)
+    bad = []
+    def work(n):
+        for _ in range(4):
+            if not np.array_equal(s.download(n), want[n]):
+                bad.append(n)
+    th = [threading.Thread(target=work, args=(n,)) for n in want]
+    [t.start() for t in th]
+    [t.join() for t in th]
+    assert not bad, bad
+    """)

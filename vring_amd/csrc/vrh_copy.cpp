@@ -97,6 +97,8 @@ hipError_t host_download(HostCopy &c, hipStream_t st, void *dst, const void *src
     ~Back() { if (on) (void)hipSetDevice(dev); }
   } back{cur, staged && cur != dev};
   if (back.on) staged = hipSetDevice(dev) == hipSuccess;
+  std::unique_lock<std::mutex> turn(c.mu, std::defer_lock);
+  if (staged) turn.lock();
   if (!staged || !ready(c)) {
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
     return e != hipSuccess ? e : hipStreamSynchronize(st);
@@ -122,7 +124,9 @@ hipError_t host_download(HostCopy &c, hipStream_t st, void *dst, const void *src
 
 void host_copy_free(HostCopy &c) {
   if (c.pin) (void)hipHostFree(c.pin);
-  for (hipEvent_t &e : c.ev)
+  c.pin = nullptr;
+  for (hipEvent_t &e : c.ev) {
     if (e) (void)hipEventDestroy(e);
-  c = HostCopy{};
+    e = nullptr;
+  }
 }

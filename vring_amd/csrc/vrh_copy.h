@@ -3,11 +3,14 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <mutex>
 
 // Pinned staging of one handle (8 MB, made on the first large copy, freed
-// with the handle).  Not shared: a handle is used by one thread at a time.
+// with the handle), used by one large copy at a time: threads that fetch
+// results of the same handle take turns.
 struct HostCopy {
   static constexpr int kSlots = 8;
+  std::mutex mu;
   char *pin = nullptr;
   hipEvent_t ev[kSlots] = {};
 };
