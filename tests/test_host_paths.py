@@ -59,3 +59,28 @@ def test_downloads_of_one_handle_in_threads(run):
     [t.join() for t in th]
     assert not bad, bad
     """)
+
+
+def test_download_beside_other_work_on_the_field(run):
+    """A large result is the field at one point of the handle's stream, also
+    while another thread keeps writing the field."""
+    run("""
+    nt, nr, nz = 64, 61, 270
+    s = vring_amd.Solver(nt, nr, nz, 4.0, 12.0, 1000.0, 0.01)
+    vals = [np.full((nt, nr + 3, nz + 3), float(k)) for k in range(4)]
+    s.upload("q1", vals[0])
+    stop = threading.Event()
+    def write():
+        k = 0
+        while not stop.is_set():
+            k += 1
+            s.upload("q1", vals[k % 4])
+    t = threading.Thread(target=write)
+    t.start()
+    try:
+        mixed = sum(len(np.unique(s.download("q1"))) != 1 for _ in range(10))
+    finally:
+        stop.set()
+        t.join()
+    assert mixed == 0, mixed
+    """)

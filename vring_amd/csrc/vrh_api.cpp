@@ -782,7 +782,7 @@ int vrh_poisson_solve(vrh_t *h, const double *rhs, double *phi) {
     (void)hipStreamSynchronize(h->stream);
     return rc;
   }
-  HIPCHK(h, host_download(h->down, h->stream, phi, d, C * sizeof(double)));
+  HIPCHK(h, host_download(h->down, h->stream, phi, d, C * sizeof(double), true));
   return 0;
 }
 

@@ -5,15 +5,21 @@
 #include <cstddef>
 #include <mutex>
 
-// Pinned staging of one handle (8 MB, made on the first large copy, freed
-// with the handle), used by one large copy at a time: threads that fetch
+// Staging of one handle's large results, made on the first of them and freed
+// with the handle: pinned slots (8 MB), and on the device a buffer of the
+// largest result so far.  One copy uses it at a time: threads that fetch
 // results of the same handle take turns.
 struct HostCopy {
   static constexpr int kSlots = 8;
   std::mutex mu;
   char *pin = nullptr;
   hipEvent_t ev[kSlots] = {};
+  hipStream_t st = nullptr;     // of the copies into the slots
+  hipEvent_t taken = nullptr;   // the result is complete and out of the way of later work
+  char *dev = nullptr;
+  size_t cap = 0;
 };
-// dst[0, bytes) = src after the work on st; complete on return.
-hipError_t host_download(HostCopy &c, hipStream_t st, void *dst, const void *src, size_t bytes);
+// dst[0, bytes) = src at this point of st; complete on return.  own: no other
+// thread queues work that writes src while the call runs.
+hipError_t host_download(HostCopy &c, hipStream_t st, void *dst, const void *src, size_t bytes, bool own = false);
 void host_copy_free(HostCopy &c);
