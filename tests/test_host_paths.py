@@ -84,3 +84,20 @@ def test_download_beside_other_work_on_the_field(run):
         t.join()
     assert mixed == 0, mixed
     """)
+
+
+def test_particle_download_needs_no_device_memory(run):
+    """A batch's particles come down also where the device has no memory left
+    (by the host alone), and the next download takes the device's rows."""
+    run("""
+    s = vring_amd.Solver(8, 8, 8, 4.0, 12.0, 1000.0, 0.01)
+    s.particles_create([1000], st=[0.0], nsub=[1], scheme="trilinear_rk3")
+    dbl.dbl_fail(ctypes.c_long(-1), ctypes.c_long(0))
+    dbl.dbl_reset()
+    u, alive = s.particles_download(0, 1000)
+    assert u.shape == (1000, 6) and not u.any() and not alive.any()
+    assert dbl.dbl_runs(b"k_rows_out") == 0
+    dbl.dbl_fail(ctypes.c_long(0), ctypes.c_long(0))
+    s.particles_download(0, 1000)
+    assert dbl.dbl_runs(b"k_rows_out") == 1
+    """)

@@ -76,8 +76,11 @@ bool ready(HostCopy &c) {
   return c.pin != nullptr;
 }
 
-// device buffer of at least `bytes`
-bool room(HostCopy &c, size_t bytes) {
+}  // namespace
+
+static_assert(kThreads * kDepth == HostCopy::kSlots, "one slot for every chunk on its way");
+
+bool host_room(HostCopy &c, size_t bytes) {
   if (c.cap >= bytes) return true;
   if (c.dev) (void)hipFree(c.dev);
   c.dev = nullptr;
@@ -90,10 +93,6 @@ bool room(HostCopy &c, size_t bytes) {
   c.cap = bytes;
   return true;
 }
-
-}  // namespace
-
-static_assert(kThreads * kDepth == HostCopy::kSlots, "one slot for every chunk on its way");
 
 hipError_t host_download(HostCopy &c, hipStream_t st, void *dst, const void *src, size_t bytes, bool own) {
   // memory that the runtime knows (pinned, managed) takes the copy engine's
@@ -110,9 +109,9 @@ hipError_t host_download(HostCopy &c, hipStream_t st, void *dst, const void *src
     ~Back() { if (on) (void)hipSetDevice(dev); }
   } back{cur, staged && cur != dev};
   if (back.on) staged = hipSetDevice(dev) == hipSuccess;
-  std::unique_lock<std::mutex> turn(c.mu, std::defer_lock);
+  std::unique_lock<std::recursive_mutex> turn(c.mu, std::defer_lock);
   if (staged) turn.lock();
-  if (!staged || !ready(c) || !(own || room(c, bytes))) {
+  if (!staged || !ready(c) || !(own || host_room(c, bytes))) {
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
     return e != hipSuccess ? e : hipStreamSynchronize(st);
   }

@@ -7,11 +7,11 @@
 
 // Staging of one handle's large results, made on the first of them and freed
 // with the handle: pinned slots (8 MB), and on the device a buffer of the
-// largest result so far.  One copy uses it at a time: threads that fetch
-// results of the same handle take turns.
+// largest result so far (particle rows are formed there too).  One copy uses
+// them at a time: threads that fetch results of the same handle take turns.
 struct HostCopy {
   static constexpr int kSlots = 8;
-  std::mutex mu;
+  std::recursive_mutex mu;
   char *pin = nullptr;
   hipEvent_t ev[kSlots] = {};
   hipStream_t st = nullptr;     // of the copies into the slots
@@ -22,4 +22,6 @@ struct HostCopy {
 // dst[0, bytes) = src at this point of st; complete on return.  own: no other
 // thread queues work that writes src while the call runs.
 hipError_t host_download(HostCopy &c, hipStream_t st, void *dst, const void *src, size_t bytes, bool own = false);
+// c.dev holds at least `bytes` (false: no memory).  Its user keeps c.mu locked.
+bool host_room(HostCopy &c, size_t bytes);
 void host_copy_free(HostCopy &c);

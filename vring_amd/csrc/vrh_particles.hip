@@ -868,25 +868,48 @@ int vrh_particles_upload(vrh_t *h, int batch, long n, const double *u, const int
   return sort_batch(h, B, false);
 }
 
+// the same by the host, where the device has no memory left for the rows
+static int download_by_host(vrh_t *h, PartBatch &B, long n, int nvar, double *u, int *alive) {
+  std::vector<double> soa((size_t)nvar * B.cap);
+  std::vector<int> al(B.cap), sl(B.cap);
+  if (hipMemcpyAsync(soa.data(), B.u, soa.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream) != hipSuccess ||
+      hipMemcpyAsync(al.data(), B.alive, al.size() * sizeof(int), hipMemcpyDeviceToHost, h->stream) != hipSuccess ||
+      hipMemcpyAsync(sl.data(), B.slot, sl.size() * sizeof(int), hipMemcpyDeviceToHost, h->stream) != hipSuccess ||
+      hipStreamSynchronize(h->stream) != hipSuccess) {
+    h->err = "particle download failed";
+    return -3;
+  }
+  for (long p = 0; p < B.cap; p++) {
+    const long q = sl[p];
+    if (q < 0 || q >= B.cap) { h->err = "particle slot map corrupt"; return -3; }
+    if (q >= n) continue;
+    for (int v = 0; v < nvar; v++) u[(size_t)q * nvar + v] = soa[(size_t)v * B.cap + p];
+    if (alive) alive[q] = al[p];
+  }
+  return 0;
+}
+
 int vrh_particles_download(vrh_t *h, int batch, long n, double *u, int *alive) {
   if (!h || batch < 0 || batch >= h->nbatch || !u || n < 0) return -1;
   PartBatch &B = h->pb[batch];
   if (n > B.cap) n = B.cap;
   const int nvar = h->pscheme == VRH_PART_TRILINEAR_RK3 ? 6 : 117;
-  int rc = particle_buffers(h, B);
-  if (rc) return rc;
   // rows in the shown order, formed on the device (physical slot p holds shown
   // slot slot[p], a permutation of [0, cap)): 10^6 trilinear particles took
   // 28 ms with the arrays copied down and scattered by the host, 5 with one
-  // copy of the rows, 2.1 with the staged one
-  int *bad = B.lflag, hbad = 0;
+  // copy of the rows, 2.1 with the staged one.  The rows, the flags and the
+  // slot check stand in the copy's buffer, which no queued sort writes.
+  std::lock_guard<std::recursive_mutex> turn(h->down.mu);
+  const size_t rb = sizeof(double) * nvar * n, ab = sizeof(int) * n;
+  if (!host_room(h->down, rb + ab + sizeof(int))) return download_by_host(h, B, n, nvar, u, alive);
+  double *rows = reinterpret_cast<double *>(h->down.dev);
+  int *al = reinterpret_cast<int *>(h->down.dev + rb), *bad = al + n, hbad = 0;
   (void)hipMemsetAsync(bad, 0, sizeof(int), h->stream);
   hipLaunchKernelGGL(k_rows_out, dim3((unsigned)((B.cap + 63) / 64)), dim3(256), 0, h->stream, B.u, B.alive, B.slot,
-                     B.cap, n, nvar, B.u_tmp, B.alive_tmp, bad);
+                     B.cap, n, nvar, rows, al, bad);
   if (hipGetLastError() != hipSuccess ||
-      (n > 0 && host_download(h->down, h->stream, u, B.u_tmp, sizeof(double) * nvar * n) != hipSuccess) ||
-      (n > 0 && alive &&
-       hipMemcpyAsync(alive, B.alive_tmp, sizeof(int) * n, hipMemcpyDeviceToHost, h->stream) != hipSuccess) ||
+      (n > 0 && host_download(h->down, h->stream, u, rows, rb, true) != hipSuccess) ||
+      (n > 0 && alive && hipMemcpyAsync(alive, al, ab, hipMemcpyDeviceToHost, h->stream) != hipSuccess) ||
       hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, h->stream) != hipSuccess ||
       hipStreamSynchronize(h->stream) != hipSuccess) {
     h->err = "particle download failed";
