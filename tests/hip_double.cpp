@@ -136,10 +136,10 @@ API long dbl_lds(const char *part) {
 API long dbl_graphs() { return g_graphs; }    // graphs instantiated
 API long dbl_dead() { return g_dead; }        // launches that were given freed memory
 API long dbl_refused() { return g_refused; }  // launches refused
-API long dbl_allocated() {
+API long dbl_pinned() {                       // bytes of pinned memory
   std::lock_guard<std::mutex> l(g_mu);
   long n = 0;
-  for (auto &a : g_live) n += (long)a.second;
+  for (auto &a : g_pinned) n += (long)a.second;
   return n;
 }
 

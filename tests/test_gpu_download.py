@@ -83,3 +83,13 @@ def test_downloads_of_one_handle_in_threads():
     for t in th:
         t.join()
     assert not bad, bad
+
+
+# the same through the pinned slots, which a handle makes once it has fetched 64 MB
+@pytest.mark.parametrize("nt,nr,nz", [(64, 61, 253), (64, 61, 254), (96, 61, 509), (97, 88, 123)])
+def test_download_sizes_staged(nt, nr, nz):
+    print(f"case staged download {nt}x{nr}x{nz}", flush=True)
+    s = vring_amd.Solver(nt, nr, nz, 4.0, 12.0, 1000.0, 0.01)
+    for _ in range(8):
+        s.download("q2")
+    roundtrip(s, (nt, nr + 3, nz + 3), nt)

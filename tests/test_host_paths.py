@@ -101,3 +101,23 @@ def test_particle_download_needs_no_device_memory(run):
     s.particles_download(0, 1000)
     assert dbl.dbl_runs(b"k_rows_out") == 1
     """)
+
+
+def test_first_large_downloads_make_no_staging(run):
+    """The pinned slots take longer to make than one large download gains: a
+    handle makes them once it has fetched 64 MB, a result of 32 MB at once."""
+    run("""
+    def pinned():
+        return dbl.dbl_pinned()
+    s = vring_amd.Solver(64, 61, 270, 4.0, 12.0, 1000.0, 0.01)   # 9 MB a field
+    p0 = pinned()
+    a = np.random.default_rng(0).standard_normal((64, 64, 273))
+    s.upload("q1", a)
+    for n in range(7):
+        assert np.array_equal(s.download("q1"), a) and pinned() == p0, n
+    assert np.array_equal(s.download("q1"), a) and pinned() == p0 + (8 << 20)
+    s = vring_amd.Solver(64, 125, 653, 4.0, 12.0, 1000.0, 0.01)  # 43 MB a field
+    p0 = pinned()
+    s.download("q1")
+    assert pinned() == p0 + (8 << 20)
+    """)

@@ -16,13 +16,15 @@ namespace {
 // staging memory (11 GB/s for 48 MB, 16 for 17 MB; the link carries 55).  Four
 // threads that each copy out of pinned slots of their own, two chunks on their
 // way, took a 48 MB particle download from 5.1 to 2.1 ms and one of 17 MB from
-// 1.3 to 0.86; chunks of 512 KB 2.8 ms, of 2 MB 1.9 with twice the pinned
+// 1.17 to 0.87; chunks of 512 KB 2.8 ms, of 2 MB 1.9 with twice the pinned
 // memory, eight threads 2.2.  Below 8 MB the gain (0.33 -> 0.28 ms at 4 MB)
-// would not pay for the pinned memory, which takes 1.3 ms once.  Uploads gain
-// nothing (0.61 ms for 17 MB either way).
+// would not pay for the pinned memory.  That takes 1 to 1.2 ms once: less than a
+// result of 32 MB gains (35 MB: 3.5 -> 1.4 ms), but more than a few of 9 or 17 MB
+// do (0.1 and 0.3 ms each), so for these it is made once the handle has fetched
+// 64 MB.  Uploads gain nothing (0.61 ms for 17 MB either way).
 constexpr size_t kChunk = (size_t)1 << 20;
 constexpr int kThreads = 4, kDepth = 2;
-constexpr size_t kMin = (size_t)8 << 20;
+constexpr size_t kMin = (size_t)8 << 20, kAtOnce = (size_t)32 << 20, kPays = (size_t)64 << 20;
 
 struct Job {
   HostCopy *c;
@@ -110,7 +112,11 @@ hipError_t host_download(HostCopy &c, hipStream_t st, void *dst, const void *src
   } back{cur, staged && cur != dev};
   if (back.on) staged = hipSetDevice(dev) == hipSuccess;
   std::unique_lock<std::recursive_mutex> turn(c.mu, std::defer_lock);
-  if (staged) turn.lock();
+  if (staged) {
+    turn.lock();
+    if (c.fetched < kPays) c.fetched += bytes;
+    staged = c.pin || bytes >= kAtOnce || c.fetched >= kPays;
+  }
   if (!staged || !ready(c) || !(own || host_room(c, bytes))) {
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
     return e != hipSuccess ? e : hipStreamSynchronize(st);

@@ -5,13 +5,14 @@
 #include <cstddef>
 #include <mutex>
 
-// Staging of one handle's large results, made on the first of them and freed
-// with the handle: pinned slots (8 MB), and on the device a buffer of the
+// Staging of one handle's large results, made once it pays and freed with the
+// handle: pinned slots (8 MB), and on the device a buffer of the
 // largest result so far (particle rows are formed there too).  One copy uses
 // them at a time: threads that fetch results of the same handle take turns.
 struct HostCopy {
   static constexpr int kSlots = 8;
   std::recursive_mutex mu;
+  size_t fetched = 0;           // bytes of large results so far
   char *pin = nullptr;
   hipEvent_t ev[kSlots] = {};
   hipStream_t st = nullptr;     // of the copies into the slots
