@@ -4,7 +4,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 #include "vrh_copy.h"
@@ -142,7 +142,7 @@ hipError_t host_download(HostCopy &c, hipStream_t st, void *dst, const void *src
   std::thread th[kThreads - 1];
   try {
     for (int q = 1; q < kThreads; q++) th[q - 1] = std::thread(worker, &b, q);
-  } catch (const std::system_error &) {  // no more threads: the others take its chunks
+  } catch (const std::exception &) {  // no more threads or no memory for one: the others take its chunks
   }
   worker(&b, 0);
   for (std::thread &t : th)
