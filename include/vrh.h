@@ -169,7 +169,8 @@ int vrh_ktimer_read(vrh_t *h, int idx, char *name, size_t len, double *total_ms,
  * kernel (one z plane per block, or z marching) with HIP events on the live
  * buffers and keeps the fastest.  Call between steps.  choice[9] (optional)
  * receives M for sweeps r1 r3 r2 z1 z3 z2, theta FFT lines/block, z DCT
- * lines/block and the explicit-kernel form (0 plane, 1 marching, 2 marching
+ * lines/block (0: not timed, a length that is no power of two or an axial mesh
+ * leaves no choice) and the explicit-kernel form (0 plane, 1 marching, 2 marching
  * with one wavefront per r row within 64 KB of LDS per block, 3 the same
  * with the rows per block that keep the most waves resident within the
  * device's LDS per block and per CU). */

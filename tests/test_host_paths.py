@@ -121,3 +121,18 @@ def test_first_large_downloads_make_no_staging(run):
     s.download("q1")
     assert pinned() == p0 + (8 << 20)
     """)
+
+
+@pytest.mark.parametrize("nt,nr,nz,kernel", [(32, 24, 64, "k_dctz2"), (12, 24, 20, "k_zdense2")])
+def test_tuned_mixed_steps_share_the_low_modes_launches(run, nt, nr, nz, kernel):
+    """A chosen width of the z transforms (by the tuner or by hand) leaves a
+    small mixed grid its shared launches: six z transforms a step, no others."""
+    run(f"""
+    for tune in (lambda s: None, lambda s: s.autotune(), lambda s: s.set_tuning(dct_lines=8)):
+        s = vring_amd.Solver({nt}, {nr}, {nz}, 4.0, 12.0, 1000.0, 0.01, precision="mixed")
+        tune(s)
+        dbl.dbl_reset()
+        s.step(2)
+        assert dbl.dbl_runs(b"{kernel}") == 12 and dbl.dbl_runs(b"k_radial2") == 6
+        assert dbl.dbl_runs(b"k_dctz") + dbl.dbl_runs(b"k_zdense") == 12 and dbl.dbl_refused() == 0
+    """)

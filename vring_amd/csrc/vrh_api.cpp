@@ -924,7 +924,8 @@ extern "C" int vrh_autotune(vrh_t *h, int reps, int *choice) {
     }
     h->fft_lines = best;
   }
-  {
+  // (the dense z transforms of other lengths and of an axial mesh have one shape)
+  if ((h->nz & (h->nz - 1)) == 0 && h->zmesh[0].empty()) {
     int best = 0; double bestt = 1e30;
     for (int tl : {2, 4, 8, 16, 32}) {
       h->dct_lines = tl;

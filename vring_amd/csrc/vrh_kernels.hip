@@ -1990,7 +1990,8 @@ void lds_optin(vrh_t *h) {
         reinterpret_cast<const void *>(&k_explicit_wave<float, float, 3, 2, 2, true>),
         reinterpret_cast<const void *>(&k_explicit_wave<float, float, 4, 2, 2, true>),
         reinterpret_cast<const void *>(&k_dctz<float>),
-        reinterpret_cast<const void *>(&k_dctz<double>)};
+        reinterpret_cast<const void *>(&k_dctz<double>),
+        reinterpret_cast<const void *>(&k_dctz2)};
     for (const void *f : fns)
       ok = ok && hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lb) == hipSuccess;
   }
@@ -2194,9 +2195,11 @@ template <typename TW> void launch_poisson(vrh_t *h, int irk, const double *ext_
   // shared: 32x64x128 307 -> 267, 33x96x200 524 -> 477, 64x96x256 551 -> 521,
   // 100x128x200 1245 -> 1205, 64x128x400 1459 -> 1435, 64x192x256 even; the
   // FP32 lines then run with the FP64 kernel's registers, and 128x192x256
-  // (25 MB) took 1642 instead of 1625.  The kernel timer's entries are those of
-  // the kernels alone.
-  const bool pair = S64 && !h->kt_on && !h->zmet.m3 && radial_rows(g) == 16 && h->dct_lines <= 0 && 4 * g.ncomp <= 14L << 20;
+  // (25 MB) took 1642 instead of 1625.  A chosen width of the z
+  // transforms is that of the FP32 lines in either form (tuned steps: 290 -> 256
+  // at 32x64x128, 550 -> 518 at 64x96x256).  The kernel timer's entries are those
+  // of the kernels alone.
+  const bool pair = S64 && !h->kt_on && !h->zmet.m3 && radial_rows(g) == 16 && 4 * g.ncomp <= 14L << 20;
   const bool par = S64 && !pair && !h->kt_on && !h->serial_sweeps;
   hipStream_t s64 = par ? h->side[0] : h->stream;
   const int ie = (irk >= 1 && irk <= 3) ? irk : 0;
