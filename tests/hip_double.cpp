@@ -14,6 +14,7 @@
 #include <deque>
 #include <functional>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -132,6 +133,12 @@ API long dbl_lds(const char *part) {
   long n = 0;
   for (auto &k : g_kern) if (k.first.find(part) != std::string::npos && k.second.lds > n) n = k.second.lds;
   return n;
+}
+// what the last launch of such a kernel was given (see hipLaunchKernel)
+API const void *dbl_given(const char *part) {
+  std::lock_guard<std::mutex> l(g_mu);
+  for (auto &k : g_kern) if (k.first.find(part) != std::string::npos) return k.second.ptr;
+  return nullptr;
 }
 API long dbl_graphs() { return g_graphs; }    // graphs instantiated
 API long dbl_dead() { return g_dead; }        // launches that were given freed memory
@@ -293,9 +300,11 @@ API hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args
       return err(hipErrorInvalidValue);
     }
   }
-  // the matrix of a dense z transform: its fourth argument's first member
-  const void *ptr = name.find("k_zdense") != std::string::npos && name.find("k_zdense2") == std::string::npos
-                        ? *static_cast<const void **>(args[3]) : nullptr;
+  // the matrix of a dense z transform (first member of its fourth argument)
+  // and the axial metric of the projection (of its third)
+  const bool zd = name.find("k_zdense") != std::string::npos && name.find("k_zdense2") == std::string::npos;
+  const void *ptr = zd ? *static_cast<const void **>(args[3])
+                    : name.find("k_project") != std::string::npos ? *static_cast<const void **>(args[2]) : nullptr;
   enqueue(s, [=](Stream *q) {
     const bool dead = ptr && !inside(g_live, ptr);
     std::lock_guard<std::mutex> l(g_mu);

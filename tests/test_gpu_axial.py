@@ -140,3 +140,30 @@ def test_uniform_axial_mesh_equals_default_path_and_guards(prec):
         assert np.abs(out[0][n] - out[1][n]).max() <= tol * vs, n
     p0, p1 = out[0]["pres"], out[1]["pres"]
     assert np.abs(p0 - p1).max() <= (1e-12 if prec == "fp64" else 1e-4) * np.abs(p0).max()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_second_axial_mesh_after_steps(precision):
+    """Steps on one axial mesh, then on another (captured steps hold the first
+    one's matrices): bit for bit those of a fresh handle on the second mesh
+    that launches kernel by kernel."""
+    nt, nr, nz = 16, 24, 40
+    print(f"case second axial mesh {precision}", flush=True)
+    s = vring_amd.Solver(nt, nr, nz, R, L, 1000.0, 0.01, precision=precision)
+    s.set_axial_mesh(*tanh_axial_mesh(nz, L, 2.0))
+    for n, a in zip(("q1", "q2", "q3"), ring(nt, nr, nz)):
+        s.upload(n, a)
+    s.step(20)
+    s.set_axial_mesh(*tanh_axial_mesh(nz, L, 3.0))
+    f = vring_amd.Solver(nt, nr, nz, R, L, 1000.0, 0.01, precision=precision)
+    f.set_axial_mesh(*tanh_axial_mesh(nz, L, 3.0))
+    f.set_graph(False)
+    names = ("q1", "q2", "q3", "pres", "prg", "ru1", "ru2", "ru3", "csort", "dq3no")
+    for n in names:
+        f.upload(n, s.download(n))
+    f.set_time(s.time())
+    for _ in range(3):
+        s.step(5)
+        f.step(5)
+        for n in names:
+            assert np.array_equal(s.download(n), f.download(n)), n

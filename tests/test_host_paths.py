@@ -136,3 +136,44 @@ def test_tuned_mixed_steps_share_the_low_modes_launches(run, nt, nr, nz, kernel)
         assert dbl.dbl_runs(b"{kernel}") == 12 and dbl.dbl_runs(b"k_radial2") == 6
         assert dbl.dbl_runs(b"k_dctz") + dbl.dbl_runs(b"k_zdense") == 12 and dbl.dbl_refused() == 0
     """)
+
+
+@pytest.mark.parametrize("what", ["allocation", "copy"])
+def test_failed_axial_mesh_leaves_the_previous_one(run, what):
+    """vrh_set_axial_mesh on a handle that steps on another mesh, with each of
+    its allocations or copies failing in turn: the call reports it, the next
+    steps run on the old mesh's matrices and metric and on no freed memory."""
+    run(f"""
+    import sys
+    sys.path.insert(0, {HERE!r})
+    from oracle_lib import tanh_axial_mesh
+    nt, nr, nz = 8, 8, 16
+    dbl.dbl_given.restype = ctypes.c_void_p
+    def given(kernel, n):
+        return np.copy(np.ctypeslib.as_array(ctypes.cast(dbl.dbl_given(kernel), ctypes.POINTER(ctypes.c_double)), (n,)))
+    def used():
+        dbl.dbl_reset()
+        s.step(1)
+        return given(b"k_project", 7 * (nz + 3)), given(b"k_zdense", 64)
+    s = vring_amd.Solver(nt, nr, nz, 4.0, 12.0, 1000.0, 0.01)
+    s.set_axial_mesh(*tanh_axial_mesh(nz, 12.0, 2.0))
+    s.step(20)
+    old = used()
+    n = failed = 0
+    while True:
+        n += 1
+        dbl.dbl_fail(ctypes.c_long(n if {what!r} == "allocation" else 0), ctypes.c_long(n if {what!r} == "copy" else 0))
+        try:
+            s.set_axial_mesh(*tanh_axial_mesh(nz, 12.0, 3.0))
+            done = True
+        except RuntimeError:
+            done = False
+        dbl.dbl_fail(ctypes.c_long(0), ctypes.c_long(0))
+        now = used()
+        assert dbl.dbl_dead() == 0, n
+        if done:
+            break
+        failed += 1
+        assert all(np.array_equal(a, b) for a, b in zip(old, now)), n
+    assert failed >= 2 and not np.array_equal(old[0], now[0])
+    """)

@@ -8,6 +8,7 @@
 #include <cstring>
 #include <new>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "vrh_internal.h"
@@ -404,7 +405,7 @@ int vrh_destroy(vrh_t *h) {
                   f.q3, f.dq1, f.dq2, f.dq3, f.pres, f.dph, f.ru1, f.ru2, f.ru3, f.r1, f.r2, f.r3, f.prg1, f.prg2,
                   f.prg3, f.S, f.ib, f.S64, f.ib64, f.csort, f.dq3no, f.corr3n, f.flag};
   for (void *p : ptrs) if (p) hipFree(p);
-  void *zp[] = {h->d_rowc, h->d_zmet, h->d_zv, h->d_zvf, h->d_zeig, h->S2, h->S2_64, h->d_zcos, h->d_tdft};
+  void *zp[] = {h->d_rowc, h->S2, h->S2_64, h->d_zcos, h->d_tdft};
   for (void *p : zp) if (p) hipFree(p);
   if (h->blas) rocblas_destroy_handle((rocblas_handle)h->blas);
   for (auto &e : h->kt_pool) hipEventDestroy(e);
@@ -523,6 +524,25 @@ int vrh_set_radial_mesh(vrh_t *h, const double *rm, const double *rc, const doub
   return 0;
 }
 
+}  // extern "C"
+
+AxialMesh::~AxialMesh() {
+  void *p[] = {d_zmet, d_zv, d_zvf, d_zeig};
+  for (void *q : p) if (q) (void)hipFree(q);
+}
+void AxialMesh::swap(AxialMesh &o) {
+  for (int q = 0; q < 4; q++) zmesh[q].swap(o.zmesh[q]);
+  zlam.swap(o.zlam);
+  std::swap(zmet, o.zmet);
+  std::swap(d_zmet, o.d_zmet);
+  std::swap(d_zv, o.d_zv);
+  std::swap(d_zvf, o.d_zvf);
+  std::swap(d_zeig, o.d_zeig);
+  for (int q = 0; q < 2; q++) std::swap(zeig[q], o.zeig[q]);
+}
+
+extern "C" {
+
 // Axial mesh: metric arrays, line coefficients, and the pressure solve's z
 // transforms (generalised eigenvectors of the z operator, host-computed).
 int vrh_set_axial_mesh(vrh_t *h, const double *zm, const double *zc, const double *dmz, const double *dcz) {
@@ -540,9 +560,10 @@ int vrh_set_axial_mesh(vrh_t *h, const double *zm, const double *zc, const doubl
     return fail(h, "axial mesh: need nz >= 2, zc(1) = 0, zc(k) < zm(k) < zc(k+1), zm(0) < zm(1), zm(nz+1) > zm(nz), "
                    "dmz, dcz > 0 (k = 0..nz+1)");
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  // everything is computed and the device buffers allocated before the
+  // everything is computed and copied into new device buffers before the
   // handle's mesh state changes: a failure leaves the previous mesh in place
-  std::vector<double> zmn[4];
+  AxialMesh mz;
+  std::vector<double> *zmn = mz.zmesh;
   const double *src[4] = {zm, zc, dmz, dcz};
   for (int q = 0; q < 4; q++) {
     zmn[q].assign(src[q], src[q] + nz + 2);
@@ -562,45 +583,48 @@ int vrh_set_axial_mesh(vrh_t *h, const double *zm, const double *zc, const doubl
     fp[k] = c3[k] * m3[k];
   }
   const double h1 = 0.5 / m3[1], h2 = 1.0 / c3[2];
-  std::vector<double> vi, vf, lam;
+  std::vector<double> vi, vf;
   std::string emsg;
-  if (host_axial_transforms(m3, c3, nz, vi, vf, lam, emsg)) return fail(h, ("axial mesh: " + emsg).c_str());
+  if (host_axial_transforms(m3, c3, nz, vi, vf, mz.zlam, emsg)) return fail(h, ("axial mesh: " + emsg).c_str());
   if (h->prec == VRH_FP64 && (size_t)nz * 16 * sizeof(double) > (size_t)h->lds_block)
     return fail(h, "axial mesh: the z transform's line tile needs more LDS than the device grants", -3);
   const size_t nn = (size_t)nz * nz;
   int rc;
-  if (!h->d_zmet && (rc = dalloc(h, &h->d_zmet, mb.size()))) return rc;
+  if ((rc = dalloc(h, &mz.d_zmet, mb.size())) || (rc = h2d(h, mz.d_zmet, mb.data(), mb.size() * sizeof(double)))) return rc;
+  const double *dz = mz.d_zmet;
+  mz.zmet = ZMet{dz, dz + L, dz + 2 * L, dz + 3 * L, dz + 4 * L, dz + 5 * L, dz + 6 * L, 2.0 / (h1 * (h1 + h2)),
+                 2.0 / (h2 * (h1 + h2))};
   if (h->prec == VRH_MIXED) {
-    if (!h->d_zv && (rc = dalloc(h, &h->d_zv, 2 * nn))) return rc;
-    if (!h->d_zvf && (rc = dalloc(h, &h->d_zvf, 2 * nn))) return rc;
     if (!h->S2_64 && (rc = dalloc(h, &h->S2_64, (size_t)5 * h->nr * nz))) return rc;
     if (!h->S2 && (rc = dalloc_bytes(h, &h->S2, compact(h) * wsize(h)))) return rc;
-  }
-  if (h->prec == VRH_MIXED && !h->blas) {
-    rocblas_handle b = nullptr;
-    if (rocblas_create_handle(&b) != rocblas_status_success) return fail(h, "axial mesh: rocblas_create_handle failed", -3);
-    h->blas = b;
-    if (rocblas_set_stream(b, h->stream) != rocblas_status_success)
-      return fail(h, "axial mesh: rocblas_set_stream failed", -3);
-  }
-  if (h->prec == VRH_FP64 && (rc = dense_axial(h, vi, vf))) return rc;
-  h->hz = nullptr;  // a per-mode solve set for another mesh: switched off
-  for (int q = 0; q < 4; q++) h->zmesh[q] = zmn[q];
-  h->zlam = lam;
-  if ((rc = h2d(h, h->d_zmet, mb.data(), mb.size() * sizeof(double)))) return rc;
-  h->zmet.m3 = h->d_zmet; h->zmet.c3 = h->d_zmet + L; h->zmet.cm = h->d_zmet + 2 * L; h->zmet.cp = h->d_zmet + 3 * L;
-  h->zmet.fm = h->d_zmet + 4 * L; h->zmet.fp = h->d_zmet + 5 * L; h->zmet.zpos = h->d_zmet + 6 * L;
-  h->zmet.ws = 2.0 / (h1 * (h1 + h2));
-  h->zmet.w2 = 2.0 / (h2 * (h1 + h2));
-  if (h->prec == VRH_MIXED) {
+    if (!h->blas) {
+      rocblas_handle b = nullptr;
+      if (rocblas_create_handle(&b) != rocblas_status_success) return fail(h, "axial mesh: rocblas_create_handle failed", -3);
+      h->blas = b;
+      if (rocblas_set_stream(b, h->stream) != rocblas_status_success)
+        return fail(h, "axial mesh: rocblas_set_stream failed", -3);
+    }
     std::vector<float> zf(2 * nn);
     for (size_t i = 0; i < nn; i++) { zf[i] = (float)vi[i]; zf[nn + i] = (float)vf[i]; }
-    if ((rc = h2d(h, h->d_zv, vi.data(), nn * sizeof(double)))) return rc;
-    if ((rc = h2d(h, h->d_zv + nn, vf.data(), nn * sizeof(double)))) return rc;
-    if ((rc = h2d(h, h->d_zvf, zf.data(), zf.size() * sizeof(float)))) return rc;
+    if ((rc = dalloc(h, &mz.d_zv, 2 * nn)) || (rc = dalloc(h, &mz.d_zvf, 2 * nn)) ||
+        (rc = h2d(h, mz.d_zv, vi.data(), nn * sizeof(double))) ||
+        (rc = h2d(h, mz.d_zv + nn, vf.data(), nn * sizeof(double))) ||
+        (rc = h2d(h, mz.d_zvf, zf.data(), zf.size() * sizeof(float))))
+      return rc;
+  } else if ((rc = dense_axial(h, vi, vf, &mz.d_zeig, mz.zeig))) {
+    return rc;
   }
-  if ((rc = refresh_mesh(h))) return rc;
+  // the captured steps hold the buffers that mz takes over here and frees
   graph_invalidate(h);
+  h->swap(mz);
+  if ((rc = refresh_mesh(h))) {
+    h->swap(mz);
+    const std::string why = h->err;
+    (void)refresh_mesh(h);
+    h->err = why;
+    return rc;
+  }
+  h->hz = nullptr;  // a per-mode solve set for another mesh: switched off
   HIPCHK(h, hipStreamSynchronize(h->stream));
   return 0;
 }

@@ -485,7 +485,7 @@ template <typename F> DenseMat pack_dense(std::vector<double> &out, size_t &at, 
   return m;
 }
 
-// device copy of `pk` into *dev (the old one stays where this fails)
+// device copy of `pk` in *dev
 int upload_pack(vrh_t *h, double **dev, const std::vector<double> &pk) {
   double *nd = nullptr;
   if (hipMalloc((void **)&nd, pk.size() * sizeof(double)) != hipSuccess ||
@@ -496,7 +496,6 @@ int upload_pack(vrh_t *h, double **dev, const std::vector<double> &pk) {
     h->err = "transform matrices: device allocation or copy failed";
     return -3;
   }
-  if (*dev) (void)hipFree(*dev);
   *dev = nd;
   return 0;
 }
@@ -557,18 +556,17 @@ int dense_create(vrh_t *h) {
   return 0;
 }
 
-// V^-1 and V (row-major nz x nz) of an axial mesh, FP64 path
-int dense_axial(vrh_t *h, const std::vector<double> &vi, const std::vector<double> &vf) {
+// V^-1 and V (row-major nz x nz) of an axial mesh, FP64 path, packed into a
+// new array *dev: m[0] forward, m[1] inverse
+int dense_axial(vrh_t *h, const std::vector<double> &vi, const std::vector<double> &vf, double **dev, DenseMat m[2]) {
   std::vector<double> pk;
   size_t at[2];
   const int n = h->nz;
-  DenseMat m[2];
   m[0] = pack_dense(pk, at[0], n, n, [&](int r, int k) { return vi[(size_t)r * n + k]; });
   m[1] = pack_dense(pk, at[1], n, n, [&](int r, int k) { return vf[(size_t)r * n + k]; });
-  const int rc = upload_pack(h, &h->d_zeig, pk);
-  if (rc) return rc;
-  for (int q = 0; q < 2; q++) { h->zeig[q] = m[q]; h->zeig[q].a = h->d_zeig + at[q]; }
-  return 0;
+  const int rc = upload_pack(h, dev, pk);
+  for (int q = 0; q < 2 && !rc; q++) m[q].a = *dev + at[q];
+  return rc;
 }
 
 // In-place z transform of nl lines.  With 32 lines per block a matrix entry

@@ -163,7 +163,25 @@ struct KTimer {
   ~KTimer();
 };
 
-struct vrh_s {
+// Axial mesh set by vrh_set_axial_mesh (zm, zc, dmz, dcz over k = 0..nz+2;
+// empty: the uniform mesh) with its device arrays.  zlam: eigenvalues of the
+// pressure solve's z operator (ascending, zlam[0] = 0); d_zmet: the ZMet
+// arrays.  The z transforms V^-1 then V: FP64 path packed (d_zeig, zeig); mixed
+// path row major nz x nz, double (d_zv) and float (d_zvf), for library GEMMs.
+struct AxialMesh {
+  std::vector<double> zmesh[4], zlam;
+  ZMet zmet{};
+  double *d_zmet = nullptr, *d_zv = nullptr, *d_zeig = nullptr;
+  float *d_zvf = nullptr;
+  DenseMat zeig[2] = {};  // [0] forward, [1] inverse
+  AxialMesh() = default;
+  AxialMesh(const AxialMesh &) = delete;
+  AxialMesh &operator=(const AxialMesh &) = delete;
+  ~AxialMesh();
+  void swap(AxialMesh &o);
+};
+
+struct vrh_s : AxialMesh {
   int nt, nr, nz, nrc, nzc, prec, theta_eigen;
   int device = 0;  // HIP device current at creation (the handle's GPU)
   double rmax, zmax, Re, dt, slip, ntime;
@@ -192,22 +210,10 @@ struct vrh_s {
   // radial mesh set by vrh_set_radial_mesh (rm, rc, dmr, dcr over j = 0..nr+1);
   // empty: the uniform mesh with dmr = dcr = 1
   std::vector<double> mesh[4];
-  // axial mesh set by vrh_set_axial_mesh (zm, zc, dmz, dcz over k = 0..nz+2);
-  // empty: the uniform mesh.  zlam: eigenvalues of the pressure solve's z
-  // operator (ascending, zlam[0] = 0); d_zmet: the ZMet arrays.  The z
-  // transforms V^-1 then V: FP64 path packed (d_zeig, zeig); mixed path row
-  // major nz x nz, double (d_zv) and float (d_zvf), for library GEMMs out of
-  // place into the twins S2 and S2_64 of the spectral arrays
-  std::vector<double> zmesh[4];
-  std::vector<double> zlam;
-  ZMet zmet{};
-  double *d_zmet = nullptr, *d_zv = nullptr;
-  float *d_zvf = nullptr;
+  // twins of the spectral arrays S and S64 (mixed path on an axial mesh: library GEMMs out of place)
   void *S2 = nullptr;
   double *S2_64 = nullptr;
   void *blas = nullptr;  // rocBLAS handle of the mixed path's z transforms (on `stream`)
-  double *d_zeig = nullptr;
-  DenseMat zeig[2] = {};  // [0] forward, [1] inverse
   // lengths that are no power of two: the z cosine matrices, the forward
   // theta matrix and the inverse theta transform's (FP64) or its table (mixed)
   double *d_zcos = nullptr, *d_tdft = nullptr;
@@ -336,7 +342,7 @@ template <typename TW> void launch_sweeps(vrh_t *h, int irk, double c3s, const d
 template <typename TW> void launch_poisson(vrh_t *h, int irk, const double *ext_rhs, double *phi_out);
 // dense transforms (vrh_dense.hip)
 int dense_create(vrh_t *h);
-int dense_axial(vrh_t *h, const std::vector<double> &vi, const std::vector<double> &vf);
+int dense_axial(vrh_t *h, const std::vector<double> &vi, const std::vector<double> &vf, double **dev, DenseMat m[2]);
 size_t dense_lds_need(int nt, int nz);
 bool dense_lds_optin(int bytes);
 template <typename TW> void launch_zdense(vrh_t *h, hipStream_t st, TW *S, long nl, int dir);
