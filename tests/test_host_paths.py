@@ -177,3 +177,26 @@ def test_failed_axial_mesh_leaves_the_previous_one(run, what):
         assert all(np.array_equal(a, b) for a, b in zip(old, now)), n
     assert failed >= 2 and not np.array_equal(old[0], now[0])
     """)
+
+
+def test_first_steps_on_an_axial_mesh_are_launched_one_by_one(run):
+    """Capturing a step takes longer than the first few steps on a mesh gain."""
+    run(f"""
+    import sys
+    sys.path.insert(0, {HERE!r})
+    from oracle_lib import tanh_axial_mesh
+    s = vring_amd.Solver(8, 8, 16, 4.0, 12.0, 1000.0, 0.01)
+    for stretch in (2.0, 3.0):
+        s.set_axial_mesh(*tanh_axial_mesh(16, 12.0, stretch))
+        dbl.dbl_reset()
+        for _ in range(8):
+            s.step(1)
+        assert dbl.dbl_graphs() == 0 and dbl.dbl_runs(b"k_project") == 24
+        s.step(1)
+        s.step(3)
+        assert dbl.dbl_graphs() == 1 and dbl.dbl_runs(b"k_project") == 36
+    s.set_axial_mesh(*tanh_axial_mesh(16, 12.0, 2.0))
+    dbl.dbl_reset()
+    s.step(20)
+    assert dbl.dbl_graphs() == 1 and dbl.dbl_runs(b"k_project") == 60
+    """)

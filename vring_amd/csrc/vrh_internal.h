@@ -174,6 +174,7 @@ struct AxialMesh {
   double *d_zmet = nullptr, *d_zv = nullptr, *d_zeig = nullptr;
   float *d_zvf = nullptr;
   DenseMat zeig[2] = {};  // [0] forward, [1] inverse
+  int launched = 0;       // steps on this mesh before one was captured
   AxialMesh() = default;
   AxialMesh(const AxialMesh &) = delete;
   AxialMesh &operator=(const AxialMesh &) = delete;
