@@ -200,3 +200,19 @@ def test_first_steps_on_an_axial_mesh_are_launched_one_by_one(run):
     s.step(20)
     assert dbl.dbl_graphs() == 1 and dbl.dbl_runs(b"k_project") == 60
     """)
+
+
+@pytest.mark.parametrize("nz", [300, 320, 321])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("refused", [False, True])
+def test_dense_z_transforms_fit_the_lds_granted(run, nz, precision, refused):
+    """Tiles of 32 lines of 257 to 320 points take more than 64 KB; without the
+    device's consent to that a grid with such lines keeps tiles of 16."""
+    big = 32 * 8 * nz if nz <= 320 and not refused else 16 * 8 * nz
+    run(f"""
+    dbl.dbl_refuse_lds({int(refused)})
+    s = vring_amd.Solver(64, 128, {nz}, 4.0, 12.0, 1000.0, 0.01, precision={precision!r})
+    dbl.dbl_reset()
+    s.step(1)
+    assert dbl.dbl_refused() == 0 and dbl.dbl_lds(b"k_zdense") == {big}, (dbl.dbl_refused(), dbl.dbl_lds(b"k_zdense"))
+    """)

@@ -569,13 +569,18 @@ int dense_axial(vrh_t *h, const std::vector<double> &vi, const std::vector<doubl
   return rc;
 }
 
-// In-place z transform of nl lines.  With 32 lines per block a matrix entry
-// read from L2 feeds two products; 16 where 32 would leave CUs without a
-// block or take more LDS than lets two blocks share a CU (n > 320).
+// Tiles of 16 lines of a block: two, where a matrix entry read from L2 feeds two
+// products; one where two would leave CUs without a block, take more LDS than
+// lets two blocks share a CU (n > 320) or more than the device granted.
+static int zdense_tiles(const vrh_t *h, long nl) {
+  return nl >= 32 * 256 && h->nz <= 320 && sizeof(double) * 32 * (size_t)h->nz <= (size_t)h->lds_block ? 2 : 1;
+}
+
+// In-place z transform of nl lines.
 template <typename TW> void launch_zdense(vrh_t *h, hipStream_t st, TW *S, long nl, int dir) {
   const bool axial = h->zmet.m3 != nullptr;
   const DenseMat &m = (axial ? h->zeig : h->zdct)[dir > 0 ? 0 : 1];
-  const int n = h->nz, nt = nl >= 32 * 256 && n <= 320 ? 2 : 1;
+  const int n = h->nz, nt = zdense_tiles(h, nl);
   const double div = dir > 0 && !axial ? (double)n : 1.0;
   const dim3 grd((unsigned)((nl + 16 * nt - 1) / (16 * nt))), blk(512);
   const size_t sh = sizeof(double) * 16 * nt * (size_t)n;
@@ -586,7 +591,7 @@ template <typename TW> void launch_zdense(vrh_t *h, hipStream_t st, TW *S, long 
 // cosine transforms of the mixed path's low modes and of its FP32 lines
 void launch_zdense2(vrh_t *h, double *S64, long nl64, float *S, long nl, int dir) {
   const DenseMat &m = h->zdct[dir > 0 ? 0 : 1];
-  const int n = h->nz, nt = nl >= 32 * 256 && n <= 320 ? 2 : 1;
+  const int n = h->nz, nt = zdense_tiles(h, nl);
   const double div = dir > 0 ? (double)n : 1.0;
   const unsigned na = (unsigned)((nl64 + 15) / 16), nb = (unsigned)((nl + 16 * nt - 1) / (16 * nt));
   const size_t sh = sizeof(double) * 16 * nt * (size_t)n;
