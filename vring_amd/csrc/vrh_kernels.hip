@@ -1298,15 +1298,14 @@ template <typename T, int M>
 __device__ __forceinline__ void radial_block(unsigned blk, T (&sh_v)[16][64], T (&sh_p)[16][64], T *__restrict__ S,
                                              const T *__restrict__ ib, long nm, long nlines, int nr,
                                              const T *__restrict__ aab, const T *__restrict__ ccb) {
-  // the sums are rounded the one way in every kernel this is the body of,
-  // fused or not as written
+#pragma clang fp contract(off)
+  // Every fused operation is written out, so that all kernels and segment
+  // lengths with this body round alike: the mixed path's forms are compared bit
+  // for bit, and a last bit of an FP32 line reaches the whole field.  (The
+  // carry G joins the last row of a segment with one rounding and the others
+  // with two: the results have always had these bits.)
   auto fma_t = [](T x, T y, T z) {
     if constexpr (sizeof(T) == 4) return __builtin_fmaf(x, y, z); else return __builtin_fma(x, y, z);
-  };
-  auto add_t = [](T z, T x, T y) {
-#pragma clang fp contract(off)
-    const T p = x * y;
-    return z + p;
   };
   const int lane = threadIdx.x & 63;
   const int s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1343,7 +1342,7 @@ __device__ __forceinline__ void radial_block(unsigned blk, T (&sh_v)[16][64], T 
   sh_p[s][lane] = Pacc;
   __syncthreads();
   T G = (T)0;
-  for (int s2 = 0; s2 < s; ++s2) G = sh_v[s2][lane] + sh_p[s2][lane] * G;
+  for (int s2 = 0; s2 < s; ++s2) G = fma_t(sh_p[s2][lane], G, sh_v[s2][lane]);
   __syncthreads();
   T Pr = (T)1;
 #pragma unroll
@@ -1351,7 +1350,7 @@ __device__ __forceinline__ void radial_block(unsigned blk, T (&sh_v)[16][64], T 
     const int p = p0 + t, pc = min(p, nr - 1);
     const bool in = t < len;
     Pr = in ? Pr * (-aab[pc + 1] * w[t] * (T)(p > 0)) : Pr;
-    x[t] = !in ? x[t] : t < M - 1 ? add_t(x[t], Pr, G) : fma_t(Pr, G, x[t]);
+    x[t] = !in ? x[t] : t < M - 1 ? x[t] + Pr * G : fma_t(Pr, G, x[t]);
   }
   T xp = (T)0, Qacc = (T)1;
 #pragma unroll
@@ -1359,7 +1358,7 @@ __device__ __forceinline__ void radial_block(unsigned blk, T (&sh_v)[16][64], T 
     const int p = p0 + t, pc = min(p, nr - 1);
     const bool in = t < len;
     const T C = ccb[pc + 1] * w[t] * (T)(p < nr - 1);
-    const T v = x[t] - C * xp;
+    const T v = fma_t(-C, xp, x[t]);
     x[t] = in ? v : x[t];
     xp = in ? v : xp;
     Qacc = in ? Qacc * -C : Qacc;
@@ -1368,7 +1367,7 @@ __device__ __forceinline__ void radial_block(unsigned blk, T (&sh_v)[16][64], T 
   sh_p[s][lane] = Qacc;
   __syncthreads();
   T X = (T)0;
-  for (int s2 = P - 1; s2 > s; --s2) X = sh_v[s2][lane] + sh_p[s2][lane] * X;
+  for (int s2 = P - 1; s2 > s; --s2) X = fma_t(sh_p[s2][lane], X, sh_v[s2][lane]);
   if (!act) return;
   T Qr = (T)1;
 #pragma unroll
@@ -1376,7 +1375,7 @@ __device__ __forceinline__ void radial_block(unsigned blk, T (&sh_v)[16][64], T 
     if (t < len) {
       const int p = p0 + t;
       Qr *= -ccb[p + 1] * w[t] * (T)(p < nr - 1);
-      S[base + nm * p] = x[t] + Qr * X;
+      S[base + nm * p] = fma_t(Qr, X, x[t]);
     }
   }
 }
