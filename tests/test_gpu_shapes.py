@@ -40,6 +40,28 @@ def test_explicit_row_widths_match_oracle(nt, form):
     substeps(o, s)
 
 
+# rms error of dq2 against the oracle with the divisions by r and by the last
+# diagonal of the theta solve as such: 1.131e-16 and 8.26e-9; bare products with
+# rounded inverses 1.200e-16 and 8.93e-9
+@pytest.mark.parametrize("precision,nt,nr,nz,bound", [("fp64", 64, 96, 64, 1.15e-16), ("mixed", 16, 24, 40, 8.4e-9)])
+def test_plane_form_divides_to_the_last_bit(precision, nt, nr, nz, bound):
+    print(f"case plane form accuracy {precision}", flush=True)
+    err = []
+    for seed in range(3):
+        o, s = make_pair(nt, nr, nz, precision=precision)
+        s.set_tuning(explicit_form=0)
+        seed_random(o, s, seed=seed)
+        o.set_time(0.13)
+        s.set_time(0.13)
+        for p in ["ucoeff", "coesys", "hdnbc", "hdnl1", "hdnl2", "hdnl3", "step"]:
+            assert o.phase(p, 1) == 0
+        for p in ["hdnbc", "explicit", "adi"]:
+            s.phase(p, 1)
+        a, b = (x[:, 1 : nr + 1, 1 : nz + 1] for x in (s.download("dq2"), o.field("dq2")))
+        err.append(np.sqrt(np.mean((a - b) ** 2) / np.mean(b**2)))
+    assert np.mean(err) <= bound, err
+
+
 # r segments 16 and 24, z segments 16, 24 and 40; the last two run one by one
 @pytest.mark.parametrize("nt,nr,nz", [(5, 15, 16), (7, 16, 15), (9, 255, 30), (3, 17, 256), (8, 264, 31), (5, 271, 256),
                                       (4, 12, 520), (3, 271, 512), (3, 300, 20), (4, 9, 700)])

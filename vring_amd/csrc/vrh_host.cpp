@@ -78,14 +78,13 @@ void host_mesh_vectors(vrh_t *h) {
 void explicit_tables(vrh_t *h, std::vector<double> &tab) {
   const int nr = h->nr, nt = h->nt;
   const std::vector<double> *v = h->hv;
-  tab.assign((size_t)(nr + 1) * (kRowCoefs + 3 * kPcrRow), 0.0);
+  tab.assign((size_t)(nr + 1) * (kRowCoefs + 3 * kPcrStride), 0.0);
   const int src[18] = {2, 3, 4, 5, 6, 8, 7, 9, 10, 11, 12, 13, 14, 15, 17, 16, 18, 19};
   for (int j = 1; j <= nr; j++) {
     double *cf = &tab[(size_t)j * kRowCoefs];
     for (int q = 0; q < 18; q++) cf[q] = v[src[q]][j];
-    cf[18] = 1.0 / v[0][j + 1];
-    cf[19] = 1.0 / v[0][j];
-    cf[20] = 1.0 / v[0][j == 1 ? 1 : j - 1];
+    const double rm[3] = {v[0][j + 1], v[0][j], v[0][j == 1 ? 1 : j - 1]};
+    for (int q = 0; q < 3; q++) { cf[18 + q] = 1.0 / rm[q]; cf[21 + q] = rm[q]; }
   }
   const bool pow2 = (nt & (nt - 1)) == 0;
   int full = 0;
@@ -108,7 +107,7 @@ void explicit_tables(vrh_t *h, std::vector<double> &tab) {
       for (int j = 1; j <= nr; j++) deepest = std::max(deepest, depth(j, 1e-18, kMaxPcrLevels));
     h->theta_levels[irk] = deepest;
     for (int j = 1; j <= nr; j++) {
-      double *p = &tab[(size_t)(nr + 1) * (kRowCoefs + (size_t)(irk - 1) * kPcrRow) + (size_t)j * kPcrRow];
+      double *p = &tab[(size_t)(nr + 1) * (kRowCoefs + (size_t)(irk - 1) * kPcrStride) + (size_t)j * kPcrStride];
       const int lv = depth(j, h->prec == VRH_MIXED ? 1e-30 : 1e-18, deepest);
       p[2] = lv;
       for (int which = 0; which < 2; which++) {
@@ -120,7 +119,9 @@ void explicit_tables(vrh_t *h, std::vector<double> &tab) {
           b = std::fma(2.0 * al, a, b);
           a = al * a;
         }
-        p[which] = 1.0 / (pow2 ? std::fma(2.0, a, b) : b);
+        const double diag = pow2 ? std::fma(2.0, a, b) : b;
+        p[which] = 1.0 / diag;
+        p[kPcrRow + which] = diag;
       }
     }
   }

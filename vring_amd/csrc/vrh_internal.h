@@ -80,10 +80,12 @@ __device__ __forceinline__ long xcd_tile(long b, long nblk) {
 
 // Tables of the explicit kernels (explicit_tables), one row per r index j =
 // 0..nr: kRowCoefs metric coefficients (cf[...] in the kernels), and per
-// substep kPcrRow numbers of the theta solves: the factors 1/diagonal of the
-// q1/q3 and the q2 systems after the reduction, its depth, a pad, then the two
-// systems' reduction ratios level by level.
-constexpr int kMaxPcrLevels = 40, kRowCoefs = 24, kPcrHead = 4, kPcrRow = kPcrHead + 2 * kMaxPcrLevels;
+// substep kPcrStride numbers of the theta solves: the factors 1/diagonal of the
+// q1/q3 and the q2 systems after the reduction, its depth, a pad, the two
+// systems' reduction ratios level by level (kPcrRow numbers so far, which the
+// marching forms keep in LDS), then the two diagonals themselves.
+constexpr int kMaxPcrLevels = 40, kRowCoefs = 24, kPcrHead = 4, kPcrRow = kPcrHead + 2 * kMaxPcrLevels,
+              kPcrStride = kPcrRow + 2;
 
 // divq's right-hand side at a cell (divergence.F90:31-41) from the three
 // one-sided differences: wr = 1/rm, ct, cr, cz the difference factors.  The
@@ -245,7 +247,7 @@ struct vrh_s : AxialMesh {
   int lds_block = 65536, lds_cu = 65536;
   int theta_levels[4];  // deepest theta reduction of a row, per substep
   double *d_rowc = nullptr;  // tables of the explicit kernels: row coefficients, then substeps 1..3
-  double *pcrt(int irk) const { return d_rowc + (size_t)(nr + 1) * (kRowCoefs + (size_t)(irk - 1) * kPcrRow); }
+  double *pcrt(int irk) const { return d_rowc + (size_t)(nr + 1) * (kRowCoefs + (size_t)(irk - 1) * kPcrStride); }
   // transform tables (double): theta twiddles (nt/2 complex), z twiddles
   // (nz/2 complex), z post-twiddles (nz complex)
   double *d_twt, *d_twz, *d_ez;

@@ -112,7 +112,7 @@ __global__ __launch_bounds__(512, sizeof(TC) == 4 ? 4 : 3) void k_explicit_march
   const int jc = (j <= nr) ? j : nr;
   // this row's coefficients, and its reduction ratios, depth and last factors
   if (ti < kRowCoefs) cfs[tj * kRowCoefs + ti] = (TC)rowc[(size_t)jc * kRowCoefs + ti];
-  for (int q = ti; q < kPcrRow; q += NTP) pcr[tj * kPcrRow + q] = pcrt[(size_t)jc * kPcrRow + q];
+  for (int q = ti; q < kPcrRow; q += NTP) pcr[tj * kPcrRow + q] = pcrt[(size_t)jc * kPcrStride + q];
   // plane fetch: element e = tid + l*NTH of the (LRW x NTP) tile, three arrays
   constexpr int NL = 3;
   long goff[NL];
@@ -393,7 +393,7 @@ __global__ __launch_bounds__(64 * RJT, WPE) void k_explicit_wave(VGrid g, const 
   const int jc = (j <= nr) ? j : nr;
   // this row's coefficients, and its reduction ratios, depth and last factors
   if (lane < kRowCoefs) cfs[tj * kRowCoefs + lane] = (TC)rowc[(size_t)jc * kRowCoefs + lane];
-  for (int q = lane; q < prow; q += 64) pcr[tj * prow + q] = pcrt[(size_t)jc * kPcrRow + q];
+  for (int q = lane; q < prow; q += 64) pcr[tj * prow + q] = pcrt[(size_t)jc * kPcrStride + q];
   // plane fetch: element e = tid + l*NTH of the (LRW x NTP) tile, three arrays
   constexpr int NL = (CPL * (RJT + 2) + RJT - 1) / RJT;  // ceil((RJ + 2) NTP / (64 RJ))
   long goff[NL];
@@ -671,9 +671,11 @@ __global__ __launch_bounds__(64 * RJT, WPE) void k_explicit_wave(VGrid g, const 
 // is read through L1/L2.  Fewer registers and LDS than the marching form;
 // the autotuner picks whichever is faster for the precision and grid.
 // ROWW = 32, 64: rows of that many lanes, solved within the wavefront (no
-// block barrier); 0: rows of several wavefronts.
+// block barrier); 0: rows of several wavefronts.  The divisions by rm and by the
+// last diagonal keep a quotient's accuracy (quot below): up to 1 % of the time (rows
+// of 32 lanes, four waves a SIMD: 15.0 -> 16.0 us at 32x64x128, 64x96x256 45.9).
 template <typename TW, typename TC, bool ZS, int ROWW>
-__global__ __launch_bounds__(512) void k_explicit_cell(VGrid g, const double *__restrict__ rowc,
+__global__ __launch_bounds__(512, ROWW == 32 ? 4 : 1) void k_explicit_cell(VGrid g, const double *__restrict__ rowc,
                                                    const double *__restrict__ pcrt, VRK rk, ZMet zm,
                                                    const double *__restrict__ q1, const double *__restrict__ q2,
                                                    const double *__restrict__ q3, const double *__restrict__ prg1,
@@ -691,7 +693,17 @@ __global__ __launch_bounds__(512) void k_explicit_cell(VGrid g, const double *__
   // the row's tables; a row of whole wavefronts is uniform in each of them
   int jc = min(j, g.nr);
   if (ROWW != 32) jc = __builtin_amdgcn_readfirstlane(jc);
-  const double *cf = rowc + (size_t)jc * kRowCoefs, *pr = pcrt + (size_t)jc * kPcrRow;
+  // x / d from the rounded inverse of d, with one correction by the remainder
+  // (Markstein): the quotient's own rounding in all but a few cases, where the
+  // bare product has the inverse's on top
+  auto quot = [](TC x, TC inv, TC d) {
+    auto fma_t = [](TC a, TC b, TC c) {
+      if constexpr (sizeof(TC) == 4) return __builtin_fmaf(a, b, c); else return __builtin_fma(a, b, c);
+    };
+    const TC q = x * inv;
+    return fma_t(fma_t(-q, d, x), inv, q);
+  };
+  const double *cf = rowc + (size_t)jc * kRowCoefs, *pr = pcrt + (size_t)jc * kPcrStride;
   TC v1 = (TC)0, v2 = (TC)0, v3 = (TC)0;
   if (cell) {
   const int ip = (i == g.nt) ? 1 : i + 1, im = (i == 1) ? g.nt : i - 1;
@@ -728,8 +740,9 @@ __global__ __launch_bounds__(512) void k_explicit_cell(VGrid g, const double *__
     TC d33 = zs ? zd2c<TC>(zm, k, Q1(-sk), Q1(0), Q1(sk))
                 : (k == 1) ? (TC)(4.0 / 3.0) * (Q1(sk) - (TC)3 * Q1(0)) * dx3q
                            : (Q1(sk) - (TC)2 * Q1(0) + Q1(-sk)) * dx3q;
-    TC qn2 = (Q1(sj) * (TC)cf[18] - Q1(0) * (TC)cf[19]) * (TC)cf[9];
-    TC qs2 = (Q1(0) * (TC)cf[19] - Q1(djm) * (TC)cf[20]) * (TC)cf[10];
+    const TC w0 = quot(Q1(0), (TC)cf[19], (TC)cf[22]);
+    TC qn2 = (quot(Q1(sj), (TC)cf[18], (TC)cf[21]) - w0) * (TC)cf[9];
+    TC qs2 = (w0 - quot(Q1(djm), (TC)cf[20], (TC)cf[23])) * (TC)cf[10];
     TC d22 = (qn2 - qs2) * (TC)cf[11];
     v1 = (ga * H1 + ro * (use_ru ? ru1[o] : (TC)0) - al * prg1[pc] + aRe * (d11 + d33 + d22)) * dt;
     ru1[o] = H1;
@@ -794,7 +807,7 @@ __global__ __launch_bounds__(512) void k_explicit_cell(VGrid g, const double *__
   const int N = g.nt, mylev = (int)pr[2];
   int blev = mylev;  // the depth that the lanes which meet at the syncs share
   if (ROWW == 0) {
-    for (int r = 0; r < RJ; r++) blev = max(blev, (int)pcrt[(size_t)min(bx * RJ + r + 1, g.nr) * kPcrRow + 2]);
+    for (int r = 0; r < RJ; r++) blev = max(blev, (int)pcrt[(size_t)min(bx * RJ + r + 1, g.nr) * kPcrStride + 2]);
   } else if (ROWW == 32) {
     blev = max(mylev, __shfl_xor(mylev, 32));
   }
@@ -828,11 +841,11 @@ __global__ __launch_bounds__(512) void k_explicit_cell(VGrid g, const double *__
     sync();
   }
   if (!cell) return;
-  const TC d1 = (TC)pr[0], d2 = (TC)pr[1];
+  const TC d1 = (TC)pr[0], d2 = (TC)pr[1], b1 = (TC)pr[kPcrRow], b2 = (TC)pr[kPcrRow + 1];
   const long o = hidx(g, i, j, k);
-  r1[o] = v1 * d1;
-  if (j >= 2) r2[o] = v2 * d2;
-  if (k >= 2) r3[o] = v3 * d1;
+  r1[o] = quot(v1, d1, b1);
+  if (j >= 2) r2[o] = quot(v2, d2, b2);
+  if (k >= 2) r3[o] = quot(v3, d1, b1);
 }
 
 // ---------------------------------------------------------------------------
