@@ -585,7 +585,12 @@ KERNEL_KEYS = {  # rocprof kernel name prefix -> kernel timer name
     "k_explicit": "explicit", "k_lsq_fit": "particles", "k_lsq_step": "particles", "k_lsq_substep": "particles",
     "k_project": "project", "k_divfft": "divfft", "k_dctz": "dct", "k_radial": "radial", "k_ifft": "ifft",
     "k_hdnbc": "hdnbc", "k_part_lsq": "particles", "k_part_tri": "particles", "k_scalars": "scalars",
+    "k_divdft": "divfft", "k_idft": "ifft", "k_idft64": "ifft", "k_zdense": "dct", "k_zdense2": "dct",
+    "k_dctz2": "dct", "k_radial2": "radial", "k_sweeps": "sweeps",
 }
+# third template argument of k_line: sweeps solved in place (r of q1 and q3, z of
+# q2), z sweeps of q1 and q3, r sweep of q2
+LINE_KEYS = ("line_in_place", "line_z", "line_r")
 
 
 def _kernel_key(name):
@@ -595,8 +600,7 @@ def _kernel_key(name):
     targs = base[len(fn) + 1:].split(">")[0] if "<" in base else ""
     prec = "fp64" if targs.startswith("double") else ("mixed" if targs.startswith("float") else "")
     if fn == "k_line":
-        mode = int(targs.split(",")[2])
-        key = "line_r" if mode in (0, 1, 2) else "line_z"
+        key = LINE_KEYS[int(targs.split(",")[2])]
     else:
         key = KERNEL_KEYS.get(fn, fn)
     return key, prec
@@ -623,7 +627,7 @@ def summarize_traffic(pmc_root, out_path):
         for c in ("FETCH_SIZE", "WRITE_SIZE"):
             for r in rows(f"pmc_{prec}_{c}"):
                 key, kp = _kernel_key(r["Kernel_Name"])
-                if kp != ("fp64" if prec == "fp64" else "mixed"):
+                if kp and kp != prec:  # (a kernel without a work type is of the run's path)
                     continue
                 acc.setdefault(key, {}).setdefault(c, []).append(float(r["Counter_Value"]) * copy[c] * 1024.0)
         out[prec] = {k: round(sum(v["FETCH_SIZE"]) / len(v["FETCH_SIZE"]) + sum(v["WRITE_SIZE"]) / len(v["WRITE_SIZE"]))
