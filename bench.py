@@ -627,7 +627,7 @@ def summarize_traffic(pmc_root, out_path):
         for c in ("FETCH_SIZE", "WRITE_SIZE"):
             for r in rows(f"pmc_{prec}_{c}"):
                 key, kp = _kernel_key(r["Kernel_Name"])
-                if kp and kp != prec:  # (a kernel without a work type is of the run's path)
+                if key.startswith("__") or kp and kp != prec:  # (a kernel without a work type is of the run's path)
                     continue
                 acc.setdefault(key, {}).setdefault(c, []).append(float(r["Counter_Value"]) * copy[c] * 1024.0)
         out[prec] = {k: round(sum(v["FETCH_SIZE"]) / len(v["FETCH_SIZE"]) + sum(v["WRITE_SIZE"]) / len(v["WRITE_SIZE"]))
