@@ -1,7 +1,7 @@
 """The dense FP64 matrix-core transforms (vrh_dense.hip) against the oracle at
 the edges of their tiles: lengths around multiples of 16 and 32, odd and even,
 the shortest and longest, line counts that fill no block, and the two tile
-widths (32 lines per block from 16384 lines on, up to 320 z points)."""
+widths (32 lines per block from 8192 lines on, up to 320 z points)."""
 from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np

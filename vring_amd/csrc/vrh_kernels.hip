@@ -915,9 +915,6 @@ template <typename T> constexpr int fft_qt() { return 1; }
 
 // One radix-2^LR pass of the Stockham autosort FFT (ls bits already done):
 // every butterfly reads its R inputs at stride n/R, applies the twiddles,
-// and after the barrier writes the in-register DFT at stride 2^ls.
-// One radix-2^LR pass of the Stockham autosort FFT (ls bits already done):
-// every butterfly reads its R inputs at stride n/R, applies the twiddles,
 // and after the barrier writes the in-register DFT at stride 2^ls.  The
 // length and pass (logn, ls) come either from template arguments (CL > 0:
 // logn = CL, ls = CS; the LDS offsets r << lg then fold into immediates) or
@@ -1010,13 +1007,6 @@ __device__ __forceinline__ void lds_fft(T *re, T *im, int nfft, int logn, int ss
     ls += lr;
   }
 }
-
-// XCD-aware tile index: the dispatcher deals consecutive workgroups round
-// robin to the 8 XCDs, each with its own L2.  Renumbering so that tiles t
-// and t + 1 run on the same XCD, one dispatch round apart, lets tiles that
-// share 128-byte lines (narrow tiles of a strided layout) meet in one L2
-// instead of each fetching the whole line from HBM.  A bijection on
-// [0, nblk) for any nblk.
 
 // byte offset rounded up to 16
 __host__ __device__ constexpr size_t al16(size_t b) { return (b + 15) & ~(size_t)15; }
@@ -1848,16 +1838,23 @@ template <typename TW> void launch_explicit(vrh_t *h, int irk) {
   const int ntp = (g.nt + 63) / 64 * 64;  // lanes of a theta row
   const int nlev = h->theta_levels[irk];
   const double *rowc = h->d_rowc, *pcrt = h->pcrt(irk);
-  // The default form (the tuner times all four).  us, the best chunk length of each:
-  //   FP64   64x128x256: plane 72, marching 98, wave 84; 128x256x512: 628, 459, 387;
-  //          256x128x256: 326, 268, 850 (its registers spill)
-  //   mixed  64x128x256: marching 53, wave 41; 128x256x512: 349, 295;
-  //          129x128x128: 68, 58 (four rows of 192 lanes); 256x128x256: 179, 193
+  // The default form (the tuner times all four).  us at the chunk lengths below,
+  // plane, marching, wave (2), wave (3):
+  //   FP64   32x64x128: 16, 34, 29, 32; 64x96x256: 53, 70, 62, 127; 64x400x64: 57, 83, 74, 134
+  //          96x64x256: 58, 59, 64, 50; 100x96x200: 74, 73, 74, 63; 128x256x512: 642, 453, 436, 387
+  //          129x128x128: 91, 106, 106, 107; 144x96x160: 92, 92, 92, 108; 192x40x600: 186, 146, 145, 184
+  //          200x96x160: 140, 132, 132, 435; 256x64x128: 71, 71, 71, 221; 256x128x256: 328, 264, 264, 857
+  //   mixed  32x64x128: 14.7, 21, 17, 17; 64x128x256: 53, 52, 43, 43; 64x400x64: 41, 47, 39, 39
+  //          100x96x200: 60, 60, 72, 46; 128x256x512: 514, 341, 391, 321
+  //          129x128x128: 71, 89, 58, 58; 192x40x600: 149, 138, 103, 103
+  //          200x96x160: 109, 97, 100, 101; 256x128x256: 270, 182, 219, 219
   // so rows of up to 64 lanes take the plane form in FP64 and the wave form in
   // mixed, up to 128 the wave form, beyond the marching form, or in mixed up to
-  // 192 the wave form.  The mixed default leaves the plane form out: its
-  // contraction of q3's terms rounds differently from the others', which agree
-  // bit for bit.
+  // 192 the wave form (four rows of 192 lanes).  Two sizes miss their best: FP64
+  // rows just beyond 128 (129x128x128), where the line cannot be drawn by the
+  // row's width alone, and narrow mixed rows, whose default leaves the plane form
+  // out: its contraction of q3's terms and its quotients round differently from
+  // the others', which agree bit for bit.
   const bool f64 = sizeof(TW) == 8;
   const int var = h->explicit_variant >= 0 ? h->explicit_variant
                   : g.nt <= 64             ? (f64 ? 0 : 2)

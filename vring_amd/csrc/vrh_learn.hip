@@ -62,7 +62,9 @@ __device__ __forceinline__ double sdiag(const Geo &g, int b, int k, int j) {
   return __builtin_fma(g.rv[j], g.izm[k] + g.izm[k + 1],
                        __builtin_fma(mm, g.dz[k] * g.drm[j], g.dz[k] * (g.rf[j] + g.rf[j + 1])));
 }
-// the same diagonal as the initial residual's kernel rounds it
+// The same diagonal, rounded otherwise: the initial residual's kernel has always
+// fused the other two of the first three products, and a solve's iterates (and
+// iteration counts) keep their bits only with it.
 __device__ __forceinline__ double sdiag0(const Geo &g, int b, int k, int j) {
 #pragma clang fp contract(off)
   const double mm = (double)g.m[b] * (double)g.m[b];
