@@ -1148,7 +1148,7 @@ int vrh_ensemble_step(vrh_ens_t *e, int nsteps) {
     vrh_t *h = e->m[q];
     if (h->kt_on) return efail(e, "member " + std::to_string(q) + " has the kernel timer enabled");
     if (!h->zmesh[0].empty())
-      return efail(e, "member " + std::to_string(q) + " has an axial mesh (stepped eagerly, not in a graph)");
+      return efail(e, "member " + std::to_string(q) + " has an axial mesh (ensembles step uniform ones)");
     ECHK(e, hipStreamSynchronize(h->stream));
     if (h->epoch != e->epochs[q]) stale = true;
   }
