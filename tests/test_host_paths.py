@@ -216,3 +216,22 @@ def test_dense_z_transforms_fit_the_lds_granted(run, nz, precision, refused):
     s.step(1)
     assert dbl.dbl_refused() == 0 and dbl.dbl_lds(b"k_zdense") == {big}, (dbl.dbl_refused(), dbl.dbl_lds(b"k_zdense"))
     """)
+
+
+@pytest.mark.parametrize("nt,nr,nz", [(16, 16, 16), (64, 64, 300)])
+def test_pressure_solves_of_one_handle_in_threads(run, nt, nr, nz):
+    """Each thread's solve has the handle's array to itself until its result is
+    out (no kernel computes here: the result is the right-hand side)."""
+    run(f"""
+    s = vring_amd.Solver({nt}, {nr}, {nz}, 4.0, 12.0, 1000.0, 0.01)
+    bad = []
+    def work(q):
+        rhs = np.asfortranarray(np.random.default_rng(q).standard_normal(({nt}, {nr}, {nz})))
+        for _ in range(8):
+            if not np.array_equal(s.poisson(rhs), rhs):
+                bad.append(q)
+    th = [threading.Thread(target=work, args=(q,)) for q in range(3)]
+    [t.start() for t in th]
+    [t.join() for t in th]
+    assert not bad, bad
+    """)

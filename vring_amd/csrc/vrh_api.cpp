@@ -415,7 +415,6 @@ int vrh_destroy(vrh_t *h) {
   if (h->copy_stream) hipStreamSynchronize(h->copy_stream);
   if (h->d_snap) hipFree(h->d_snap);
   if (h->d_anl) hipFree(h->d_anl);
-  if (h->d_poi) hipFree(h->d_poi);
   host_copy_free(h->down);
   if (h->h_snap) hipHostFree(h->h_snap);
   if (h->snap_ev) hipEventDestroy(h->snap_ev);
@@ -798,11 +797,12 @@ int vrh_poisson_solve(vrh_t *h, const double *rhs, double *phi) {
   if (!h || !rhs || !phi) return -1;
   const size_t C = compact(h);
   // One array for both directions: the forward theta transform reads all of
-  // the right-hand side before the inverse one writes phi.  It stays with the
-  // handle: allocating and freeing two arrays took 120 of a call's 1980 us
-  // at 64x128x256 (with the staged copy of the result it is 1630).
-  if (!h->d_poi) HIPCHK(h, hipMalloc(&h->d_poi, C * sizeof(double)));
-  double *d = h->d_poi;
+  // the right-hand side before the inverse one writes phi.  It is the buffer of
+  // the handle's large copies, this call's alone until phi is out; allocating
+  // and freeing two arrays took 120 of a call's 1980 us at 64x128x256.
+  std::lock_guard<std::recursive_mutex> turn(h->down.mu);
+  if (!host_room(h->down, C * sizeof(double))) return fail(h, "vrh_poisson_solve: device allocation failed", -3);
+  double *d = reinterpret_cast<double *>(h->down.dev);
   HIPCHK(h, hipMemcpyAsync(d, rhs, C * sizeof(double), hipMemcpyHostToDevice, h->stream));
   if (h->prec == VRH_MIXED) launch_poisson<float>(h, 1, d, d);
   else launch_poisson<double>(h, 1, d, d);

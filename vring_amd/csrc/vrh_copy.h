@@ -6,9 +6,10 @@
 #include <mutex>
 
 // Staging of one handle's large results, made once it pays and freed with the
-// handle: pinned slots (8 MB), and on the device a buffer of the
-// largest result so far (particle rows are formed there too).  One copy uses
-// them at a time: threads that fetch results of the same handle take turns.
+// handle: pinned slots (8 MB), and on the device a buffer of the largest result
+// so far, in which particle rows and the pressure solve's array stand as well.
+// One call uses them at a time: threads that fetch results of the same handle
+// take turns.
 struct HostCopy {
   static constexpr int kSlots = 8;
   std::recursive_mutex mu;

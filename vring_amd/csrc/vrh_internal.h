@@ -282,7 +282,6 @@ struct vrh_s : AxialMesh {
   double *d_snap = nullptr, *h_snap = nullptr;
   double *d_anl = nullptr;  // vrh_analysis block partials and result (first use)
   HostCopy down;            // staging of large downloads
-  double *d_poi = nullptr;  // vrh_poisson_solve's right-hand side and solution (first use)
   hipStream_t copy_stream = nullptr;
   hipEvent_t snap_ev = nullptr;
   bool snap_pending = false;
