@@ -164,7 +164,11 @@ API hipError_t hipFuncSetAttribute(const void *f, hipFuncAttribute, int v) {
   return hipSuccess;
 }
 API hipError_t hipGetLastError() { const hipError_t e = t_err; t_err = hipSuccess; return e; }
-API const char *hipGetErrorString(hipError_t) { return "test double"; }
+API const char *hipGetErrorString(hipError_t e) {
+  thread_local std::string s;
+  s = "error " + std::to_string((int)e);
+  return s.c_str();
+}
 API hipError_t hipGetSymbolAddress(void **p, const void *) { static char scratch[1 << 20]; *p = scratch; return hipSuccess; }
 
 // ---- memory ----
@@ -197,7 +201,7 @@ API hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p) 
   return hipSuccess;
 }
 API hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind kind, hipStream_t s) {
-  if (fails(g_fail_copy)) return err(hipErrorUnknown);
+  if (fails(g_fail_copy)) return err(hipErrorInvalidValue);
   if (kind == hipMemcpyHostToDevice && !inside(g_pinned, src)) {  // pageable: taken before the call returns
     auto tmp = std::make_shared<std::vector<char>>(static_cast<const char *>(src), static_cast<const char *>(src) + n);
     enqueue(s, [=](Stream *) { std::memcpy(dst, tmp->data(), n); });

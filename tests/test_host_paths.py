@@ -235,3 +235,22 @@ def test_pressure_solves_of_one_handle_in_threads(run, nt, nr, nz):
     [t.join() for t in th]
     assert not bad, bad
     """)
+
+
+def test_failed_chunk_is_reported_as_itself(run):
+    """Any of a staged download's copies failing: the call returns -3 with the
+    failure's own error, and the next download is whole."""
+    run("""
+    dbl.hipGetErrorString.restype = ctypes.c_char_p
+    s = vring_amd.Solver(64, 125, 653, 4.0, 12.0, 1000.0, 0.01)
+    a = np.random.default_rng(0).standard_normal((64, 128, 656))
+    s.upload("q1", a)
+    for n in (1, 2, 5, 17, 42):
+        dbl.dbl_fail(ctypes.c_long(0), ctypes.c_long(n))
+        try:
+            s.download("q1")
+            raise SystemExit(f"copy {n} not reported")
+        except RuntimeError as e:
+            assert "(-3)" in str(e) and "error 1" in str(e), e
+        assert np.array_equal(s.download("q1"), a), n
+    """)

@@ -33,13 +33,18 @@ struct Job {
   const char *src;
   size_t bytes;
   std::atomic<size_t> next{0};
-  std::atomic<int> err{0};
+  std::atomic<hipError_t> err{hipSuccess};  // the first failure
+  bool ok(hipError_t e) {
+    hipError_t none = hipSuccess;
+    if (e != hipSuccess) err.compare_exchange_strong(none, e);
+    return e == hipSuccess;
+  }
 };
 
 // Takes chunks from the job's counter until none is left, keeping kDepth of
 // them on their way into its own slots while it copies the oldest out.
 void worker(Job *b, int q) {
-  if (hipSetDevice(b->dev) != hipSuccess) { b->err = 1; return; }
+  if (!b->ok(hipSetDevice(b->dev))) return;
   const size_t nc = (b->bytes + kChunk - 1) / kChunk;
   size_t id[kDepth];
   auto len = [&](size_t c) { return std::min(kChunk, b->bytes - c * kChunk); };
@@ -47,17 +52,15 @@ void worker(Job *b, int q) {
     id[s] = b->next.fetch_add(1);
     if (id[s] >= nc) return;
     const int g = q * kDepth + s;
-    if (hipMemcpyAsync(b->c->pin + g * kChunk, b->src + id[s] * kChunk, len(id[s]), hipMemcpyDeviceToHost,
-                       b->c->st) != hipSuccess ||
-        hipEventRecord(b->c->ev[g], b->c->st) != hipSuccess) {
-      b->err = 1;
+    if (!b->ok(hipMemcpyAsync(b->c->pin + g * kChunk, b->src + id[s] * kChunk, len(id[s]), hipMemcpyDeviceToHost,
+                              b->c->st)) ||
+        !b->ok(hipEventRecord(b->c->ev[g], b->c->st)))
       id[s] = nc;
-    }
   };
   for (int s = 0; s < kDepth; s++) issue(s);
   for (int s = 0; id[s] < nc; s = (s + 1) % kDepth) {
     const int g = q * kDepth + s;
-    if (hipEventSynchronize(b->c->ev[g]) != hipSuccess) { b->err = 1; return; }
+    if (!b->ok(hipEventSynchronize(b->c->ev[g]))) return;
     memcpy(b->dst + id[s] * kChunk, b->c->pin + g * kChunk, len(id[s]));
     issue(s);
   }
@@ -147,8 +150,8 @@ hipError_t host_download(HostCopy &c, hipStream_t st, void *dst, const void *src
   worker(&b, 0);
   for (std::thread &t : th)
     if (t.joinable()) t.join();
-  e = hipStreamSynchronize(c.st);
-  return b.err ? hipErrorUnknown : e;
+  (void)b.ok(hipStreamSynchronize(c.st));
+  return b.err;
 }
 
 void host_copy_free(HostCopy &c) {
